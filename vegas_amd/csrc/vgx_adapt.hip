@@ -101,6 +101,151 @@ __global__ void adapt_exact_kernel(AdaptArgs a) {
     }
 }
 
+// The exact adapt with one workgroup per axis and the axis in LDS: the same
+// operations on the same values as adapt_axis_exact, so the same bits.
+// What is independent per increment (averages, smoothing, the compression's
+// log and pow, the new nodes' divisions) is spread over the threads; the
+// reference's sequential sums and its CDF walk stay sequential, in one wave
+// that reads the values from LDS 8 ahead (sums) or keeps 64 of them in its
+// lanes (walk).  The chain of dependent FP64 additions bounds it.  5 axes of
+// 400 increments: 732 us with one lane doing everything from global memory,
+// about 110 us so.
+constexpr int kExactThreads = 256;
+constexpr int kExactLds = 60 * 1024;  // bytes: av[old], tmp/acc[max(old, nn)], jj[nn]
+inline size_t exact_lds_bytes(int old, int nn) {
+    return (size_t)old * 8 + (size_t)(old > nn ? old : nn) * 8 + (size_t)nn * 4;
+}
+
+// s + v[0] + v[1] + ... in order (every lane of the calling wave alike).
+__device__ inline double seq_sum(double s, const double* v, int n) {
+    int i = 0;
+    for (; i + 8 <= n; i += 8) {
+        double t[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) t[k] = v[i + k];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s += t[k];
+    }
+    for (; i < n; ++i) s += v[i];
+    return s;
+}
+
+__device__ inline double read_lane(double v, int l) {
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, l);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+__global__ __launch_bounds__(kExactThreads) void adapt_exact_lds_kernel(AdaptArgs a) {
+    extern __shared__ double el[];
+    __shared__ double s_sum;
+    __shared__ int s_last;  // nodes 1..s_last-1 were placed by the walk
+    if (a.status && *a.status) return;
+    const int d = blockIdx.x, T = kExactThreads;
+    const int old = a.ninc[d], nn = a.new_ninc[d];
+    double* av = el;
+    double* tmp = el + old;  // smoothed values, then the walk's accumulator per node
+    int* jj = reinterpret_cast<int*>(tmp + (old > nn ? old : nn));
+    double* ng = a.new_grid + (int64_t)d * a.new_ld;
+    const double* g = source_row(a, d, T);
+    const bool wave0 = threadIdx.x < 64;
+    for (int i = threadIdx.x; i < old; i += T) {
+        double v = 1.0;
+        if (a.alpha != 0 && old > 1 && a.has_training) {
+            const double nf = a.n_f[(int64_t)d * a.nb + i];
+            v = nf > 0 ? a.sum_f[(int64_t)d * a.nb + i] / nf : 0.;
+        }
+        av[i] = v;
+    }
+    __syncthreads();
+    if (a.alpha > 0 && old > 1) {
+        for (int i = threadIdx.x; i < old; i += T) {
+            double t;
+            if (i == 0) t = fabs(7. * av[0] + av[1]) / 8.;
+            else if (i == old - 1) t = fabs(7. * av[old - 1] + av[old - 2]) / 8.;
+            else t = fabs(6. * av[i] + av[i - 1] + av[i + 1]) / 8.;
+            tmp[i] = t;
+        }
+        __syncthreads();
+        if (wave0) {
+            const double s = seq_sum(tmp[0] + tmp[old - 1], tmp + 1, old - 2);
+            if (threadIdx.x == 0) s_sum = s;
+        }
+        __syncthreads();
+        const double s = s_sum;
+        for (int i = threadIdx.x; i < old; i += T) {
+            double v = s > 0 ? tmp[i] / s + kTiny : kTiny;
+            if (v > 0 && v <= 0.99999999) v = pow(-(1 - v) / log(v), a.alpha);
+            av[i] = v;
+        }
+        __syncthreads();
+    }
+    if (wave0) {
+        const int lane = threadIdx.x;
+        const double f = seq_sum(0., av, old) / (double)nn;
+        // the walk: lane l holds increment base + l
+        int base = 0, j = -1, i = 1;
+        double cur = lane < old ? av[lane] : 0.0;
+        double acc = 0.;
+        while (i < nn) {
+            bool stopped = false;
+            while (__builtin_amdgcn_readfirstlane(acc < f)) {
+                j += 1;
+                if (j >= old) {
+                    stopped = true;
+                    break;
+                }
+                if (j - base == 64) {
+                    base = j;
+                    cur = base + lane < old ? av[base + lane] : 0.0;
+                }
+                acc += read_lane(cur, j - base);
+            }
+            if (stopped) break;
+            acc -= f;
+            if (lane == 0) {
+                tmp[i] = acc;
+                jj[i] = j;
+            }
+            ++i;
+        }
+        if (lane == 0) s_last = i;
+    }
+    __syncthreads();
+    // node i from the increment the walk stopped in; nodes after an early
+    // stop (round-off only) at the upper limit, as adapt_axis_exact
+    const int last = s_last;
+    const double glo = g[0], ghi = g[old];
+    for (int i = 1 + threadIdx.x; i < nn; i += T) {
+        double xv = ghi;
+        if (i < last) {
+            const int j = jj[i];  // -1 only when the weights sum to 0 or NaN
+            xv = j >= 0 ? g[j + 1] - (tmp[i] / av[j]) * (g[j + 1] - g[j]) : glo - 0.0 * tmp[i];
+        }
+        ng[i] = xv;
+    }
+    if (threadIdx.x == 0) ng[0] = glo;
+    for (int i = nn + (int)threadIdx.x; i < a.new_ld; i += T) ng[i] = ghi;
+    clear_row(a, d, T);
+}
+
+// The exact adapt of every axis on stream st: by adapt_exact_lds_kernel
+// where each axis fits its LDS (up to 3072 increments to as many: the bins
+// and nodes of one axis in 60 KiB), else, or when the axes are chained
+// (pyx:534), by one lane per axis.
+static void launch_adapt_exact(const AdaptArgs& a, hipStream_t st) {
+    size_t need = 0;
+    for (int d = 0; d < a.dim; ++d) {
+        const size_t b = exact_lds_bytes(a.ninc[d], a.new_ninc[d]);
+        need = b > need ? b : need;
+    }
+    if (!a.chain && need <= (size_t)kExactLds)
+        hipLaunchKernelGGL(adapt_exact_lds_kernel, dim3(a.dim), dim3(kExactThreads), need, st, a);
+    else
+        hipLaunchKernelGGL(adapt_exact_kernel, dim3(a.chain ? 1 : a.dim), dim3(64), 0, st, a);
+}
+
 __global__ __launch_bounds__(1024) void adapt_parallel_kernel(AdaptArgs a) {
     __shared__ double av[kAdaptLdsMax];
     __shared__ double P[kAdaptLdsMax];
@@ -159,7 +304,7 @@ int adapt_in_place(vgx_ctx* ctx, int dim, const int32_t* ninc, double* grid, int
     if (parallel)
         hipLaunchKernelGGL(adapt_parallel_kernel, dim3(dim), dim3(1024), 0, st, a);
     else
-        hipLaunchKernelGGL(adapt_exact_kernel, dim3(a.chain ? 1 : dim), dim3(64), 0, st, a);
+        launch_adapt_exact(a, st);
     return check_launch();
 }
 
@@ -213,7 +358,7 @@ extern "C" int vgx_adapt(vgx_ctx* ctx, int dim, const int32_t* ninc, const doubl
         int rc = ctx->adapt_tmp.ensure(need);
         if (rc) return rc;
         a.buf = (double*)ctx->adapt_tmp.ptr;
-        hipLaunchKernelGGL(adapt_exact_kernel, dim3(a.chain ? 1 : dim), dim3(64), 0, st, a);
+        launch_adapt_exact(a, st);
     } else {
         hipLaunchKernelGGL(adapt_parallel_kernel, dim3(dim), dim3(1024), 0, st, a);
     }
