@@ -28,3 +28,23 @@ def test_adapt_exact_sizes(va, orc, old, new, alpha):
         q.add_training_data(y, f)
         q.adapt(alpha=alpha, ninc=np.array([new, new]))
     np.testing.assert_allclose(m.grid[:, :new + 1], o.grid[:, :new + 1], rtol=1e-13, atol=1e-13)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 1024, 1025, 17 * 1024 + 1])
+@pytest.mark.parametrize("ninc", [[1, 2], [63, 64, 65], [1000] * 12, [1025, 2049]])
+def test_train_hist_ordered_sizes(va, orc, n, ninc):
+    """Wave, tile and scan-run remainders; bins beyond one scan block; more
+    axes than one workgroup's counts; points crowded into few bins."""
+    rng = np.random.default_rng(n)
+    dim = len(ninc)
+    m, o = va.AdaptiveMap([[0, 1]] * dim, ninc=ninc), orc.OracleMap([[0, 1]] * dim, ninc=ninc)
+    y = rng.uniform(0, 1, (n, dim))
+    y[:, -1] = y[:, -1] ** 8
+    y[::7, 0] = 0.0
+    f = rng.normal(size=n) * np.exp(rng.uniform(-20, 20, n))
+    for _ in range(2):
+        m.add_training_data(y, f)
+        o.add_training_data(y, f)
+    for d, k in enumerate(ninc):
+        assert np.array_equal(m.sum_f[d, :k], o.sum_f[d, :k])
+        assert np.array_equal(m.n_f[d, :k], o.n_f[d, :k])

@@ -9,9 +9,10 @@
 // counting sort groups |f| by (axis, bin) keeping point order, then one lane
 // per bin adds the group in point order onto the existing sum:
 //   1 hist_count    per-tile, per-bin counts (LDS)
-//   2 hist_scan     exclusive scan over tiles per bin, then over bins
+//   2 hist_scan     exclusive scan over tiles per bin; hist_start over bins
 //   3 hist_scatter  one wave per (tile, axis); stable ranks from ballots
 //   4 hist_sum      sequential per-bin sums in point order
+#include <algorithm>
 #include <mutex>
 
 #include "vgx_internal.h"
@@ -104,109 +105,210 @@ __global__ __launch_bounds__(256) void hist_fast_kernel(HistArgs a) {
 }
 
 // ---- ordered mode ---------------------------------------------------------
-__global__ __launch_bounds__(256) void hist_count_kernel(HistArgs a) {
+constexpr size_t kCountLds = 32 * 1024;  // bytes of LDS counts of one hist_count workgroup
+
+// One workgroup per tile and group of axes (as many as have LDS counts in
+// kCountLds): the workgroups of a tile read its rows of y once per group.
+__global__ __launch_bounds__(256) void hist_count_kernel(HistArgs a, int daxes) {
     extern __shared__ uint32_t cl[];
-    const int tile = blockIdx.x, d = blockIdx.y;
-    const int ni = a.ninc[d];
-    for (int k = threadIdx.x; k < a.nb; k += blockDim.x) cl[k] = 0u;
+    const int tile = blockIdx.x, d0 = blockIdx.y * daxes;
+    const int nd = min(daxes, a.dim - d0);
+    for (int k = threadIdx.x; k < nd * a.nb; k += blockDim.x) cl[k] = 0u;
     __syncthreads();
     const int64_t p0 = (int64_t)tile * kHistTile, n = npoints(a);
     for (int j = threadIdx.x; j < kHistTile; j += blockDim.x) {
-        int64_t i = p0 + j;
+        const int64_t i = p0 + j;
         if (i >= n) break;
-        int k = point_bin(a, i, d, ni);
-        if (k >= 0) atomicAdd(&cl[k], 1u);
+        for (int e = 0; e < nd; ++e) {
+            const int k = point_bin(a, i, d0 + e, a.ninc[d0 + e]);
+            if (k >= 0) atomicAdd(&cl[e * a.nb + k], 1u);
+        }
     }
     __syncthreads();
-    uint32_t* out = a.cnt + ((int64_t)d * a.ntiles + tile) * a.nb;
-    for (int k = threadIdx.x; k < a.nb; k += blockDim.x) out[k] = cl[k];
+    for (int e = 0; e < nd; ++e) {
+        uint32_t* out = a.cnt + ((int64_t)(d0 + e) * a.ntiles + tile) * a.nb;
+        for (int k = threadIdx.x; k < a.nb; k += blockDim.x) out[k] = cl[e * a.nb + k];
+    }
 }
 
-// One workgroup per axis: per-bin exclusive scan over tiles (in place), then
-// an exclusive scan over bins of the bin totals.
-__global__ __launch_bounds__(1024) void hist_scan_kernel(HistArgs a) {
-    __shared__ uint32_t part[1024];
-    const int d = blockIdx.x;
-    for (int k = threadIdx.x; k < a.nb; k += blockDim.x) {
-        uint32_t run = 0;
-        for (int t = 0; t < a.ntiles; ++t) {
-            uint32_t* p = a.cnt + ((int64_t)d * a.ntiles + t) * a.nb + k;
-            uint32_t v = *p;
-            *p = run;
-            run += v;
-        }
-        a.total[d * a.nb + k] = run;
+// Per-bin exclusive scan over the tiles (in place) and the bin totals.  One
+// workgroup per axis and 64 bins: wave s takes the s-th of 16 runs of tiles
+// (its sum first, then the scan from the runs before it), so 16 runs are read
+// at once and a wave's loads are 256 contiguous bytes.  One workgroup per
+// axis walking all tiles in turn took 49 us at 196 tiles of 5 x 400 bins.
+constexpr int kScanBins = 64, kScanRuns = 16;
+
+__global__ __launch_bounds__(kScanBins * kScanRuns) void hist_scan_kernel(HistArgs a) {
+    __shared__ uint32_t part[kScanRuns][kScanBins];
+    const int lane = threadIdx.x % kScanBins, run = threadIdx.x / kScanBins;
+    const int d = blockIdx.y, k = blockIdx.x * kScanBins + lane;
+    const int per = (a.ntiles + kScanRuns - 1) / kScanRuns;
+    const int t0 = min(run * per, a.ntiles), t1 = min(t0 + per, a.ntiles);
+    const bool live = k < a.nb;
+    uint32_t* col = a.cnt + (int64_t)d * a.ntiles * a.nb + k;
+    uint32_t s = 0;
+    if (live) {
+#pragma unroll 4
+        for (int t = t0; t < t1; ++t) s += col[(int64_t)t * a.nb];
     }
+    part[run][lane] = s;
     __syncthreads();
-    // exclusive scan of total[d][0..nb) -> start[d][..]; chunked over 1024 bins
+    uint32_t pre = 0;
+    for (int r = 0; r < run; ++r) pre += part[r][lane];
+    if (!live) return;
+#pragma unroll 4
+    for (int t = t0; t < t1; ++t) {
+        const uint32_t v = col[(int64_t)t * a.nb];
+        col[(int64_t)t * a.nb] = pre;
+        pre += v;
+    }
+    if (run == kScanRuns - 1) a.total[d * a.nb + k] = pre;
+}
+
+// Exclusive scan of an axis's bin totals -> bin starts; one workgroup per axis.
+__global__ __launch_bounds__(1024) void hist_start_kernel(HistArgs a) {
+    __shared__ uint32_t wsum[16];
+    const int d = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     uint32_t carry = 0;
-    for (int base = 0; base < a.nb; base += blockDim.x) {
-        int k = base + threadIdx.x;
-        uint32_t v = k < a.nb ? a.total[d * a.nb + k] : 0u;
-        part[threadIdx.x] = v;
-        __syncthreads();
-        for (int o = 1; o < (int)blockDim.x; o <<= 1) {
-            uint32_t add = threadIdx.x >= (unsigned)o ? part[threadIdx.x - o] : 0u;
-            __syncthreads();
-            part[threadIdx.x] += add;
-            __syncthreads();
+    for (int base = 0; base < a.nb; base += 1024) {
+        const int k = base + threadIdx.x;
+        const uint32_t v = k < a.nb ? a.total[d * a.nb + k] : 0u;
+        uint32_t incl = v;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t t = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += t;
         }
-        if (k < a.nb) a.start[d * a.nb + k] = carry + part[threadIdx.x] - v;
-        uint32_t chunk_total = part[blockDim.x - 1];
+        if (lane == 63) wsum[w] = incl;
         __syncthreads();
-        carry += chunk_total;
+        uint32_t pre = carry, tot = carry;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            if (q < w) pre += wsum[q];
+            tot += wsum[q];
+        }
+        if (k < a.nb) a.start[d * a.nb + k] = pre + incl - v;
+        carry = tot;
+        __syncthreads();
     }
 }
 
 // One wave per (tile, axis).  Points of the tile are taken 64 at a time in
-// order; equal keys within a group get consecutive ranks in lane order.
-__global__ __launch_bounds__(64) void hist_scatter_kernel(HistArgs a) {
+// order; equal keys within a group get consecutive ranks in lane order.  The
+// lanes that share a lane's key are found from one ballot per key bit (a
+// fixed number of instructions however many distinct keys the group has: a
+// loop over the distinct keys took 251 us for 2e5 points and 5 axes of 400
+// bins, this 20 us).  run[k]: the next position of bin k.
+__global__ __launch_bounds__(64) void hist_scatter_kernel(HistArgs a, int keybits) {
     extern __shared__ uint32_t run[];
     const int tile = blockIdx.x, d = blockIdx.y;
     const int ni = a.ninc[d];
     const int lane = threadIdx.x;
-    for (int k = lane; k < a.nb; k += 64) run[k] = 0u;
-    __syncthreads();
     const uint32_t* tbase = a.cnt + ((int64_t)d * a.ntiles + tile) * a.nb;
     const uint32_t* bstart = a.start + d * a.nb;
-    double* out = a.sorted + (int64_t)d * a.n;
     const int64_t p0 = (int64_t)tile * kHistTile, n = npoints(a);
-    for (int g = 0; g < kHistTile; g += 64) {
-        const int64_t i = p0 + g + lane;
-        int key = -1;
-        double fa = 0.0;
-        if (i < n) {
-            key = point_bin(a, i, d, ni);
-            fa = fabs(a.f[i]);
+    // the whole tile's loads in flight at once, with those of run[]
+    constexpr int kGroups = kHistTile / 64;
+    int key[kGroups];
+    double fa[kGroups];
+#pragma unroll
+    for (int q = 0; q < kGroups; ++q) {
+        const int64_t i = p0 + 64 * q + lane;
+        key[q] = i < n ? point_bin(a, i, d, ni) : -1;
+        fa[q] = i < n ? fabs(a.f[i]) : 0.0;
+    }
+#pragma unroll 4
+    for (int k = lane; k < a.nb; k += 64) run[k] = bstart[k] + tbase[k];
+    __syncthreads();
+    double* out = a.sorted + (int64_t)d * a.n;
+    const uint64_t below = (1ull << lane) - 1ull;
+#pragma unroll
+    for (int q = 0; q < kGroups; ++q) {
+        const bool on = key[q] >= 0;
+        uint64_t m = __ballot(on);
+        for (int b = 0; b < keybits; ++b) {
+            const bool bit = (key[q] >> b) & 1;
+            const uint64_t set = __ballot(bit);
+            m &= bit ? set : ~set;
         }
-        uint64_t active = __ballot(key >= 0);
-        while (active) {
-            const int leader = __ffsll((unsigned long long)active) - 1;
-            const int lk = __shfl(key, leader, 64);
-            const uint64_t m = __ballot(key == lk) & active;
-            const uint32_t base = run[lk];
-            if ((m >> lane) & 1ull) {
-                const uint32_t rank = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-                out[bstart[lk] + tbase[lk] + base + rank] = fa;
-            }
-            __builtin_amdgcn_wave_barrier();
-            if (lane == leader) run[lk] = base + (uint32_t)__popcll(m);
-            __builtin_amdgcn_wave_barrier();
-            active &= ~m;
+        uint32_t base = 0;
+        if (on) base = run[key[q]];
+        __builtin_amdgcn_wave_barrier();
+        if (on) {
+            out[base + (uint32_t)__popcll(m & below)] = fa[q];
+            if ((m & below) == 0) run[key[q]] = base + (uint32_t)__popcll(m);
         }
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
+// acc + lane 0's v + lane 1's v + ... + lane 15's v of each 16-lane row, in
+// that order (every lane of the row alike): v_mov row_newbcast moves.
+template <int L>
+__device__ __forceinline__ void row_add(double& acc, double v) {
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = (uint32_t)dpp0_i<0x150 + L>((int)(uint32_t)u);
+    const uint32_t hi = (uint32_t)dpp0_i<0x150 + L>((int)(uint32_t)(u >> 32));
+    acc += __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+    if constexpr (L < 15) row_add<L + 1>(acc, v);
+}
+
+// The sums of a bin's values in point order: a 16-lane row per bin reads 16
+// consecutive values at once (4 such loads in flight) and adds them one
+// after the other from the row's lanes.  Past a bin's last value it adds
+// +0.0 to a sum of absolute values, which leaves it as it is.  One thread
+// per bin, each loading its own values, took 166 us for 2e5 points and 5 x
+// 400 bins (the loads' latency per value), this 9 us.
 __global__ __launch_bounds__(256) void hist_sum_kernel(HistArgs a) {
-    const int d = blockIdx.y;
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= a.ninc[d]) return;
-    const uint32_t s = a.start[d * a.nb + k], t = a.total[d * a.nb + k];
-    const double* in = a.sorted + (int64_t)d * a.n;
-    double acc = a.sum_f[d * a.nb + k];
-    for (uint32_t j = 0; j < t; ++j) acc += in[s + j];
-    a.sum_f[d * a.nb + k] = acc;
-    a.n_f[d * a.nb + k] = a.n_f[d * a.nb + k] + (double)t;
+    const int d = blockIdx.y, row = threadIdx.x >> 4, l = threadIdx.x & 15;
+    const int k = blockIdx.x * 16 + row;
+    const bool live = k < a.ninc[d];
+    const uint32_t s = live ? a.start[d * a.nb + k] : 0u, t = live ? a.total[d * a.nb + k] : 0u;
+    const double* in = a.sorted + (int64_t)d * a.n + s;
+    double acc = live ? a.sum_f[d * a.nb + k] : 0.0;
+    constexpr int kAhead = 4;
+    double cur[kAhead], nxt[kAhead];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) cur[q] = (uint32_t)(16 * q + l) < t ? in[16 * q + l] : 0.0;
+    for (uint64_t j = 0; __any(j < t); j += 16 * kAhead) {
+#pragma unroll
+        for (int q = 0; q < kAhead; ++q) {
+            const uint64_t i = j + 16 * (kAhead + q) + l;
+            nxt[q] = i < t ? in[i] : 0.0;
+        }
+        if (j < t) {
+#pragma unroll
+            for (int q = 0; q < kAhead; ++q) row_add<0>(acc, cur[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < kAhead; ++q) cur[q] = nxt[q];
+    }
+    if (live && l == 0) {
+        a.sum_f[d * a.nb + k] = acc;
+        a.n_f[d * a.nb + k] = a.n_f[d * a.nb + k] + (double)t;
+    }
+}
+
+// The four passes on stream st; a's tables and counts are set.
+static int launch_ordered(const HistArgs& a, hipStream_t st) {
+    int maxn = 0, keybits = 1;
+    for (int d = 0; d < a.dim; ++d) maxn = a.ninc[d] > maxn ? a.ninc[d] : maxn;
+    while ((1 << keybits) < maxn) ++keybits;
+    const size_t row = (size_t)a.nb * sizeof(uint32_t);
+    // axes per hist_count workgroup: all that its LDS holds where the tiles
+    // alone fill the chip (a tile's rows of y are then read once); fewer where
+    // they do not (196 tiles of 5 axes: 5.0 us by axis, 9.7 us together)
+    const int groups = std::min(a.dim, (1024 + a.ntiles - 1) / a.ntiles);
+    const int fit = row >= kCountLds ? 1 : (int)(kCountLds / row);
+    const int daxes = std::min(fit, (a.dim + groups - 1) / groups);
+    hipLaunchKernelGGL(hist_count_kernel, dim3(a.ntiles, (a.dim + daxes - 1) / daxes), dim3(256), row * daxes, st, a,
+                       daxes);
+    hipLaunchKernelGGL(hist_scan_kernel, dim3((a.nb + kScanBins - 1) / kScanBins, a.dim), dim3(kScanBins * kScanRuns),
+                       0, st, a);
+    hipLaunchKernelGGL(hist_start_kernel, dim3(a.dim), dim3(1024), 0, st, a);
+    hipLaunchKernelGGL(hist_scatter_kernel, dim3(a.ntiles, a.dim), dim3(64), row, st, a, keybits);
+    hipLaunchKernelGGL(hist_sum_kernel, dim3((maxn + 15) / 16, a.dim), dim3(256), 0, st, a);
+    return check_launch();
 }
 
 }  // namespace vgx
@@ -255,14 +357,7 @@ extern "C" int vgx_train_hist(vgx_ctx* ctx, int dim, const int32_t* ninc, int ld
     a.start = (uint32_t*)ctx->hist_start.ptr;
     a.total = a.start + (size_t)dim * a.nb;
     a.sorted = (double*)ctx->hist_sorted.ptr;
-    size_t lds = (size_t)a.nb * sizeof(uint32_t);
-    hipLaunchKernelGGL(hist_count_kernel, dim3(a.ntiles, dim), dim3(256), lds, st, a);
-    hipLaunchKernelGGL(hist_scan_kernel, dim3(dim), dim3(1024), 0, st, a);
-    hipLaunchKernelGGL(hist_scatter_kernel, dim3(a.ntiles, dim), dim3(64), lds, st, a);
-    int maxn = 0;
-    for (int d = 0; d < dim; ++d) maxn = ninc[d] > maxn ? ninc[d] : maxn;
-    hipLaunchKernelGGL(hist_sum_kernel, dim3((maxn + 255) / 256, dim), dim3(256), 0, st, a);
-    return check_launch();
+    return launch_ordered(a, st);
 }
 
 namespace vgx {
@@ -287,11 +382,7 @@ int train_hist_records(vgx_ctx* ctx, int dim, const int32_t* ninc, int nb, const
     a.rbins = rbins;
     a.rstride = rstride;
     a.nrange = nrange;
-    int maxn = 0;
-    for (int d = 0; d < dim; ++d) {
-        a.ninc[d] = ninc[d];
-        maxn = ninc[d] > maxn ? ninc[d] : maxn;
-    }
+    for (int d = 0; d < dim; ++d) a.ninc[d] = ninc[d];
     a.ntiles = (int)((cap + kHistTile - 1) / kHistTile);
     int rc = ctx->hist_cnt.ensure((size_t)dim * a.ntiles * a.nb * sizeof(uint32_t));
     if (rc) return rc;
@@ -301,12 +392,7 @@ int train_hist_records(vgx_ctx* ctx, int dim, const int32_t* ninc, int nb, const
     a.start = (uint32_t*)ctx->hist_start.ptr;
     a.total = a.start + (size_t)dim * a.nb;
     a.sorted = (double*)ctx->hist_sorted.ptr;
-    const size_t lds = (size_t)a.nb * sizeof(uint32_t);
-    hipLaunchKernelGGL(hist_count_kernel, dim3(a.ntiles, dim), dim3(256), lds, st, a);
-    hipLaunchKernelGGL(hist_scan_kernel, dim3(dim), dim3(1024), 0, st, a);
-    hipLaunchKernelGGL(hist_scatter_kernel, dim3(a.ntiles, dim), dim3(64), lds, st, a);
-    hipLaunchKernelGGL(hist_sum_kernel, dim3((maxn + 255) / 256, dim), dim3(256), 0, st, a);
-    return check_launch();
+    return launch_ordered(a, st);
 }
 
 }  // namespace vgx
@@ -366,11 +452,9 @@ extern "C" int vgx_train_hist_noalloc(int dim, const int32_t* ninc, int ld, cons
     a.n = n;
     a.sum_f = sum_f;
     a.n_f = n_f;
-    int maxn = 0;
     for (int d = 0; d < dim; ++d) {
         if (ninc[d] < 1 || ninc[d] > a.nb) return VGX_EINVAL;
         a.ninc[d] = ninc[d];
-        maxn = ninc[d] > maxn ? ninc[d] : maxn;
     }
     if ((size_t)a.nb * sizeof(uint32_t) > 64 * 1024) return VGX_ERANGE;
     size_t o_start = 0, o_sorted = 0;
@@ -383,11 +467,5 @@ extern "C" int vgx_train_hist_noalloc(int dim, const int32_t* ninc, int ld, cons
     a.start = (uint32_t*)(base + o_start);
     a.total = a.start + (size_t)dim * a.nb;
     a.sorted = (double*)(base + o_sorted);
-    hipStream_t st = (hipStream_t)stream;
-    const size_t lds = (size_t)a.nb * sizeof(uint32_t);
-    hipLaunchKernelGGL(hist_count_kernel, dim3(a.ntiles, dim), dim3(256), lds, st, a);
-    hipLaunchKernelGGL(hist_scan_kernel, dim3(dim), dim3(1024), 0, st, a);
-    hipLaunchKernelGGL(hist_scatter_kernel, dim3(a.ntiles, dim), dim3(64), lds, st, a);
-    hipLaunchKernelGGL(hist_sum_kernel, dim3((maxn + 255) / 256, dim), dim3(256), 0, st, a);
-    return check_launch();
+    return launch_ordered(a, (hipStream_t)stream);
 }
