@@ -107,9 +107,10 @@ __global__ void adapt_exact_kernel(AdaptArgs a) {
 // log and pow, the new nodes' divisions) is spread over the threads; the
 // reference's sequential sums and its CDF walk stay sequential, in one wave
 // that reads the values from LDS 8 ahead (sums) or keeps 64 of them in its
-// lanes (walk).  The chain of dependent FP64 additions bounds it.  5 axes of
-// 400 increments: 732 us with one lane doing everything from global memory,
-// about 110 us so.
+// lanes (walk, one branch-free step per addition).  The chain of dependent
+// operations bounds it.  5 axes of 400 increments: 732 us with one lane doing
+// everything from global memory, 108 us so with a branching walk, 48 us with
+// the walk branch-free (14 instructions a step).
 constexpr int kExactThreads = 256;
 constexpr int kExactLds = 60 * 1024;  // bytes: av[old], tmp/acc[max(old, nn)], jj[nn]
 inline size_t exact_lds_bytes(int old, int nn) {
@@ -183,32 +184,52 @@ __global__ __launch_bounds__(kExactThreads) void adapt_exact_lds_kernel(AdaptArg
     }
     if (wave0) {
         const int lane = threadIdx.x;
-        const double f = seq_sum(0., av, old) / (double)nn;
-        // the walk: lane l holds increment base + l
-        int base = 0, j = -1, i = 1;
-        double cur = lane < old ? av[lane] : 0.0;
+        const double f = read_lane(seq_sum(0., av, old) / (double)nn, 0);
+        // The walk, one addition a step: the next increment's weight while
+        // acc < f, else -f for a node placed (i and j are scalars, and
+        // acc + (-f) is acc - f).  In a window of kWalk steps lane l holds
+        // increment j0 + 1 + l, and collects the accumulator and increment of
+        // node i0 + l: every step writes the node it may have placed, a step
+        // that placed none is overwritten by the one that does.
+        constexpr int kWalk = 32;
+        int j = -1, i = 1;
         double acc = 0.;
-        while (i < nn) {
-            bool stopped = false;
-            while (__builtin_amdgcn_readfirstlane(acc < f)) {
-                j += 1;
-                if (j >= old) {
-                    stopped = true;
-                    break;
+        bool walking = true;
+        while (walking) {
+            const int j0 = j, i0 = i;
+            const double cur = j0 + 1 + lane < old ? av[j0 + 1 + lane] : 0.0;
+            double rec = 0.0;
+            int recj = 0, taken = 0;
+            // step s of the window: after it i - i0 = s + 1 - taken
+            auto step = [&](int s) {
+                const double next = read_lane(cur, taken);
+                const bool take = acc < f;
+                acc += take ? next : -f;
+                const bool mine = lane == s - taken;  // the node being placed
+                rec = mine ? acc : rec;
+                recj = mine ? s : recj;  // its increment is j0 + s - (i - i0)
+                taken += (int)(__ballot(take) & 1);
+            };
+            int steps = 0;
+            if (i0 + kWalk <= nn && j0 + kWalk < old) {
+#pragma unroll
+                for (int s = 0; s < kWalk; ++s) step(s);
+                steps = kWalk;
+            } else {
+                for (; steps < kWalk; ++steps) {
+                    if (i0 + steps - taken >= nn || (j0 + taken + 1 >= old && (__ballot(acc < f) & 1))) {
+                        walking = false;
+                        break;
+                    }
+                    step(steps);
                 }
-                if (j - base == 64) {
-                    base = j;
-                    cur = base + lane < old ? av[base + lane] : 0.0;
-                }
-                acc += read_lane(cur, j - base);
             }
-            if (stopped) break;
-            acc -= f;
-            if (lane == 0) {
-                tmp[i] = acc;
-                jj[i] = j;
+            j = j0 + taken;
+            i = i0 + steps - taken;
+            if (lane < i - i0) {
+                tmp[i0 + lane] = rec;
+                jj[i0 + lane] = j0 + recj - lane;
             }
-            ++i;
         }
         if (lane == 0) s_last = i;
     }
