@@ -48,3 +48,29 @@ def test_train_hist_ordered_sizes(va, orc, n, ninc):
     for d, k in enumerate(ninc):
         assert np.array_equal(m.sum_f[d, :k], o.sum_f[d, :k])
         assert np.array_equal(m.n_f[d, :k], o.n_f[d, :k])
+
+
+@pytest.mark.parametrize("dim,ninc", [(1, 1), (1, 1000), (3, 7), (8, 1000), (17, 1000), (18, 1000), (64, 5)])
+@pytest.mark.parametrize("n", [1, 63, 1025, 70001])
+def test_map_invmap_sizes(va, orc, dim, ninc, n):
+    """Tile remainders; grids staged in LDS (up to 17 axes of 1000) or not;
+    invmap's search table (from 65536 points) on a grid with wide and narrow
+    increments; x on the nodes, beside them and outside."""
+    rng = np.random.default_rng(dim * n)
+    grid = np.cumsum(np.exp(rng.normal(0, 2, (dim, ninc + 1))), axis=1)
+    m, o = va.AdaptiveMap(grid.tolist()), orc.OracleMap(grid.tolist())
+    y = rng.uniform(0, 1, (n, dim))
+    y[::5] = rng.integers(0, ninc + 1, y[::5].shape) / ninc
+    x, jac = m.map(y)
+    xo, jo = o.map(y)
+    assert np.array_equal(x.cpu().numpy(), xo)
+    assert np.array_equal(jac.cpu().numpy(), jo)
+    assert np.array_equal(m.jac1d(y[:1025]), o.jac1d(y[:1025]))
+    lo, hi = grid[:, 0], grid[:, -1]
+    xo[1::7] = lo - 1
+    xo[2::7] = hi + rng.uniform(0, 1, xo[2::7].shape)
+    xo[3::7] = np.nextafter(xo[3::7], -np.inf)
+    yi, ji = m.invmap(xo)
+    yr, jr = o.invmap(xo)
+    assert np.array_equal(yi.cpu().numpy(), yr)
+    assert np.array_equal(ji.cpu().numpy(), jr)
