@@ -303,6 +303,40 @@ constexpr size_t kBLdsCnts = (size_t)(kBHist / 2) * sizeof(uint32_t);
 constexpr size_t kBLdsOffs = (size_t)16 * kNoff * sizeof(uint32_t);
 constexpr size_t kBLds = kBLdsGrid + kBLdsSums + kBLdsCnts + kBLdsOffs;
 
+// The tiles of one work item: the waves take them from an LDS counter (faster
+// waves take more); each tile's sums go to tile_part and are summed in tile
+// order at the item's close.
+template <int DIM, bool PER>
+__device__ __forceinline__ void b_item_tiles(const BArgs& a, const TileGeom& tg, const TileIO& tio,
+                                             const GaussMix32& fcn, const AxisC* ax, const double* G, double* Ls,
+                                             uint32_t* Lc, uint32_t* offs, uint32_t t0, uint32_t ntl, uint32_t hend,
+                                             uint32_t off_end, uint32_t hbase, uint32_t pshift, uint32_t* s_tile,
+                                             int lane, TileAcc& acc) {
+#pragma unroll 1
+    for (;;) {
+        uint32_t n = 0u;
+        if (lane == 0) n = atomicAdd(s_tile, 1u);
+        n = __builtin_amdgcn_readfirstlane(n);
+        if (n >= ntl) break;
+        const uint32_t t = t0 + n;
+        const uint32_t plo = t * kT;
+        const TilePos tp{t, plo, min(plo + (uint32_t)kT, off_end), (uint32_t)a.tile_h[t], hend, off_end, hbase, pshift};
+        uint32_t ov[kOffRegs];
+        load_offsets(a.off, tp.hf, hend, off_end, lane, ov);
+        store_offsets(offs, lane, ov);
+        tile_body<DIM, PER>(tg, tio, fcn, ax, G, Ls, Lc, offs, tp, lane, acc);
+        const double m = wave_total(acc.am.hi + acc.am.lo), v = wave_total(acc.av.hi + acc.av.lo),
+                     qs = wave_total(acc.as.hi + acc.as.lo);
+        if (lane == 63) {
+            double* o = a.tile_part + 3 * (size_t)t;
+            o[0] = m; o[1] = v; o[2] = qs;
+        }
+        acc.am = DD{0.0, 0.0};
+        acc.av = DD{0.0, 0.0};
+        acc.as = DD{0.0, 0.0};
+    }
+}
+
 template <bool PER>
 __global__ __launch_bounds__(kFusedThreads) void b_fused_kernel(BArgs a, int it, int train) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -359,33 +393,29 @@ __global__ __launch_bounds__(kFusedThreads) void b_fused_kernel(BArgs a, int it,
         const TileIO tio{a.off, a.sigf, a.slots, nullptr, nullptr, nullptr, 0u, 0u};  // LDS histogram
         TileAcc acc{{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, 0.0, 0};
         const uint32_t hend = q.hbase + (uint32_t)q.nhcube, off_end = pl.P + pl.T;
-        // the waves take the item's tiles from an LDS counter (faster waves
-        // take more); each tile's sums go to tile_part and are summed in tile
-        // order at the item's close
         const uint32_t ntl = itm.t1 - itm.t0;
-#pragma unroll 1
-        for (;;) {
-            uint32_t n = 0u;
-            if (lane == 0) n = atomicAdd(&s_tile, 1u);
-            n = __builtin_amdgcn_readfirstlane(n);
-            if (n >= ntl) break;
-            const uint32_t t = itm.t0 + n;
-            const uint32_t plo = t * kT;
-            const TilePos tp{t, plo, min(plo + (uint32_t)kT, off_end), (uint32_t)a.tile_h[t], hend, off_end,
-                             q.hbase, pl.P};
-            uint32_t ov[kOffRegs];
-            load_offsets(a.off, tp.hf, hend, off_end, lane, ov);
-            store_offsets(offs, lane, ov);
-            tile_body<-kBD, PER>(tg, tio, fcn, ax, G, Ls, Lc, offs, tp, lane, acc);
-            const double m = wave_total(acc.am.hi + acc.am.lo), v = wave_total(acc.av.hi + acc.av.lo),
-                         qs = wave_total(acc.as.hi + acc.as.lo);
-            if (lane == 63) {
-                double* o = a.tile_part + 3 * (size_t)t;
-                o[0] = m; o[1] = v; o[2] = qs;
+        if constexpr (PER) {
+            // the tile loop of the item's own dimension: the axes unrolled with
+            // no end-of-axes tests and their increments held in registers
+            // (1024 integrals of 2-10 axes: the runtime-dimension loop took
+            // 4.5 ms an iteration, with register spills; these 3.5, without)
+            switch (dim) {
+#define B_ITEM(D) b_item_tiles<D, PER>(a, tg, tio, fcn, ax, G, Ls, Lc, offs, itm.t0, ntl, hend, off_end, q.hbase, pl.P, \
+                                           &s_tile, lane, acc)
+                case 1: B_ITEM(1); break;
+                case 2: B_ITEM(2); break;
+                case 3: B_ITEM(3); break;
+                case 4: B_ITEM(4); break;
+                case 5: B_ITEM(5); break;
+                case 6: B_ITEM(6); break;
+                case 7: B_ITEM(7); break;
+                case 8: B_ITEM(8); break;
+                case 9: B_ITEM(9); break;
+                default: B_ITEM(10); break;
             }
-            acc.am = DD{0.0, 0.0};
-            acc.av = DD{0.0, 0.0};
-            acc.as = DD{0.0, 0.0};
+        } else {
+            B_ITEM(-kBD);
+#undef B_ITEM
         }
         __syncthreads();
         if (train) {
