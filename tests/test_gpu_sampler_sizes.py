@@ -1,0 +1,42 @@
+"""The fused sampler where a dimension, a tile or a launch shape ends: FP64
+parity mode against the oracle (the bars of test_gpu_integrator.py)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def va():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import vegas_amd
+    return vegas_amd
+
+
+@pytest.mark.parametrize("dim,neval", [(14, 20000), (15, 20000), (16, 20000), (18, 2000), (24, 2000), (25, 2000),
+                                       (40, 1000)])
+def test_dims(va, orc, dim, neval):
+    """Dimensions of their own up to 16, shared up to 24, and above."""
+    c = [0.5 + 0.02 * ((d % 3) - 1) for d in range(dim)]
+    f, fo = va.GaussianMixture([1.0], [8.0], [c]), orc.GaussMix([1.0], [8.0], [c])
+    integ = va.Integrator([[0, 1]] * dim, neval=neval, seed=23, precision='f64', exact=True)
+    r = integ(f, nitn=1)
+    o = orc.OracleIntegrator([(0, 1)] * dim, neval=neval, seed=23)
+    mean, var, nev = o.run(fo, 1)
+    m = r.itn_results[0]
+    assert integ.last_neval == nev[0]
+    assert abs(m.mean - mean[0]) <= 1e-12 * abs(mean[0])
+    assert abs(m.var - var[0]) <= 1e-10 * var[0]
+    np.testing.assert_allclose(integ.sigf, o.sigf, rtol=1e-11)
+    np.testing.assert_allclose(integ.map.grid, o.map.grid, rtol=1e-11, atol=1e-13)
+
+    @va.lbatchintegrand
+    def fl(x):
+        return np.exp(-8.0 * ((x - np.array(c)) ** 2).sum(1))
+
+    ra = va.Integrator([[0, 1]] * dim, neval=neval, seed=29, precision='f32')(f, nitn=1).itn_results[0]
+    rb = va.Integrator([[0, 1]] * dim, neval=neval, seed=29, precision='f32')(fl, nitn=1).itn_results[0]
+    assert abs(ra.mean - rb.mean) <= 2e-5 * abs(rb.mean)
+    assert abs(ra.sdev - rb.sdev) <= 1e-3 * rb.sdev

@@ -1,5 +1,5 @@
-// Instantiates the fused sampler for the GaussMix32 integrand: dimensions 1-12
-// specialised (unrolled, register-resident x) plus a generic runtime-dim path.
+// Instantiates the fused sampler for the GaussMix32 integrand: dimensions 1-16
+// specialised (unrolled, register-resident x), a runtime dimension of 17-24 and one of up to 64.
 #include "vgx_fused.h"
 
 namespace vgx {
@@ -20,7 +20,13 @@ int launch_fused<GaussMix32>(const IterGeom& g, const FusedPtrs& io, const Gauss
         case 10: return launch_fused_dim<10>(g, io, fcn, blocks, lds, st, ev0, ev1);
         case 11: return launch_fused_dim<11>(g, io, fcn, blocks, lds, st, ev0, ev1);
         case 12: return launch_fused_dim<12>(g, io, fcn, blocks, lds, st, ev0, ev1);
-        default: return launch_fused_dim<0>(g, io, fcn, blocks, lds, st, ev0, ev1);
+        case 13: return launch_fused_dim<13>(g, io, fcn, blocks, lds, st, ev0, ev1);
+        case 14: return launch_fused_dim<14>(g, io, fcn, blocks, lds, st, ev0, ev1);
+        case 15: return launch_fused_dim<15>(g, io, fcn, blocks, lds, st, ev0, ev1);
+        case 16: return launch_fused_dim<16>(g, io, fcn, blocks, lds, st, ev0, ev1);
+        default:
+            return g.dim <= 24 ? launch_fused_dim<-24>(g, io, fcn, blocks, lds, st, ev0, ev1)
+                               : launch_fused_dim<0>(g, io, fcn, blocks, lds, st, ev0, ev1);
     }
 }
 
