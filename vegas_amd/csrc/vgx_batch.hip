@@ -391,7 +391,7 @@ __global__ __launch_bounds__(kFusedThreads) void b_fused_kernel(BArgs a, int it,
         __syncthreads();
         const GaussMix32 fcn{1, a.fA + i, a.fB + i, a.fc + (size_t)i * kBD};
         const TileIO tio{a.off, a.sigf, a.slots, nullptr, nullptr, nullptr, 0u, 0u};  // LDS histogram
-        TileAcc acc{{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, 0.0, 0};
+        TileAcc acc{{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, 0};
         const uint32_t hend = q.hbase + (uint32_t)q.nhcube, off_end = pl.P + pl.T;
         const uint32_t ntl = itm.t1 - itm.t0;
         if constexpr (PER) {

@@ -155,12 +155,6 @@ __device__ inline DD wave_sum_dd(DD v) {
     return v;
 }
 
-__device__ inline double wave_max(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, kWave));
-    return v;
-}
-
 // ---- DPP lane movement (gfx9 encodings): another lane's value through the
 // VALU's data-parallel-primitive path instead of an LDS permute.
 constexpr int kDppRowShl = 0x100;     // + n: row_shl:n (within 16-lane rows)

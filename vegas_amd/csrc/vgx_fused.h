@@ -368,7 +368,6 @@ __device__ __forceinline__ void store_record(const TileIO& io, int dim, uint32_t
 // Per-wave accumulators across tiles.
 struct TileAcc {
     DD am, av, as;           // sum of S + D, of var_h, of sigf_h
-    double wmax;
     int nan_seen;
 };
 
@@ -489,7 +488,6 @@ __device__ __forceinline__ void tile_body(const TileGeom& g, const TileIO& io, c
             if (f != f) acc.nan_seen = 1;
             vj = w * f;
             const double tn = vj * (double)ncur;
-            acc.wmax = fmax(acc.wmax, fabs(tn));
             if (g.train_points) {
                 const double c2 = tn * tn;
                 if (io.rec_c2) {
@@ -889,50 +887,14 @@ __device__ __forceinline__ bool added_before(HistSeq& hs, int dim, uint32_t upto
     return __ballot(!ok) == 0;
 }
 
-// Workgroup reduction of the wave accumulators into out[0..5] (DD mean,
-// var, sigf sums, fixed order) and the run-wide max |w f n| / NaN flag.
-__device__ inline void block_close(TileAcc& acc, double* Lred, double* out, Scalars* sc) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nwave = blockDim.x >> 6;
-    acc.am = wave_sum_dd(acc.am);
-    acc.av = wave_sum_dd(acc.av);
-    acc.as = wave_sum_dd(acc.as);
-    const double wmax = wave_max(acc.wmax);
-    const int anynan = __any(acc.nan_seen);
-    if (lane == 0) {
-        Lred[wave * 6 + 0] = acc.am.hi; Lred[wave * 6 + 1] = acc.am.lo;
-        Lred[wave * 6 + 2] = acc.av.hi; Lred[wave * 6 + 3] = acc.av.lo;
-        Lred[wave * 6 + 4] = acc.as.hi; Lred[wave * 6 + 5] = acc.as.lo;
-        if (wmax > 0.0) atomicMax((unsigned long long*)&sc->wfn_max_bits,
-                                  (unsigned long long)__double_as_longlong(wmax));
-        if (anynan) atomicOr(&sc->status, (int32_t)VGX_ENAN);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        DD m{0, 0}, v{0, 0}, s{0, 0};
-        for (int k = 0; k < nwave; ++k) {
-            m = dd_sum(m, DD{Lred[k * 6 + 0], Lred[k * 6 + 1]});
-            v = dd_sum(v, DD{Lred[k * 6 + 2], Lred[k * 6 + 3]});
-            s = dd_sum(s, DD{Lred[k * 6 + 4], Lred[k * 6 + 5]});
-        }
-        out[0] = m.hi; out[1] = m.lo; out[2] = v.hi; out[3] = v.lo; out[4] = s.hi; out[5] = s.lo;
-    }
-}
-
 // Workgroup close of the fused sampler: the sums of its tiles
 // tile_part[tb..te) in tile order, in DD, into out[0..5] (mean, var, sigf
 // sums; lane l takes tiles tb + l, tb + l + 64, ..., then a fixed-order
-// butterfly), and
-// the run-wide max |w f n| / NaN flag from the lanes' accumulators.
+// butterfly), and the NaN flag from the lanes' accumulators.
 __device__ inline void block_close_tiles(const TileAcc& acc, const double* tpart, uint32_t tb, uint32_t te,
                                          double* out, Scalars* sc) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const double wmax = wave_max(acc.wmax);
-    const int anynan = __any(acc.nan_seen);
-    if (lane == 0) {
-        if (wmax > 0.0) atomicMax((unsigned long long*)&sc->wfn_max_bits,
-                                  (unsigned long long)__double_as_longlong(wmax));
-        if (anynan) atomicOr(&sc->status, (int32_t)VGX_ENAN);
-    }
+    if (__any(acc.nan_seen) && lane == 0) atomicOr(&sc->status, (int32_t)VGX_ENAN);
     __syncthreads();  // every tile's sums are stored
     if (wave == 0) {
         DD m{0, 0}, v{0, 0}, q{0, 0};
@@ -1033,7 +995,7 @@ __global__ __launch_bounds__(kFusedThreads) void fused_kernel(IterGeom g, FusedP
     }
     __syncthreads();
 
-    TileAcc acc{{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, 0.0, 0};
+    TileAcc acc{{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, 0};
 #pragma unroll 1
     for (;;) {
         uint32_t n = 0u;

@@ -36,7 +36,6 @@ __global__ void iter_init_kernel(IterGeom g, double* sum_f, double* n_f, Scalars
             sc->status = 0;  // the NaN flag is sticky within one run only
             sc->reset_sigf = 0;
         }
-        sc->wfn_max_bits = 0;
         for (int k = 0; k < 6; ++k) sc->acc[k] = 0.0;
         sc->overflow = 0;
     }
@@ -467,7 +466,6 @@ __device__ void finalize_body(const IterGeom& g, Scalars* sc, const vgx_state& s
     st.ravg[2] = chi2;
     st.ravg[3] = (double)(n - 1);
     // next iteration of this run
-    sc->wfn_max_bits = 0;
     for (int k = 0; k < 6; ++k) sc->acc[k] = 0.0;
 }
 

@@ -64,7 +64,6 @@ struct Scalars {
     int32_t nh_min, nh_max;
     // current batch (whole iteration for device integrands)
     uint32_t b_p0, b_p1, b_h0, b_h1, b_ntiles, pad0;
-    uint64_t wfn_max_bits;  // max |w f n| seen (non-negative double bits)
     double acc[6];          // iteration sums (DD): mean, var, sum_sigf
     int32_t status;         // 0 or VGX_ENAN
     int32_t reset_sigf;
