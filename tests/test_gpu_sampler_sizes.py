@@ -40,3 +40,26 @@ def test_dims(va, orc, dim, neval):
     rb = va.Integrator([[0, 1]] * dim, neval=neval, seed=29, precision='f32')(fl, nitn=1).itn_results[0]
     assert abs(ra.mean - rb.mean) <= 2e-5 * abs(rb.mean)
     assert abs(ra.sdev - rb.sdev) <= 1e-3 * rb.sdev
+
+
+@pytest.mark.parametrize("dim", [1, 4, 9])
+@pytest.mark.parametrize("neval", [100, 2000, 4 * 256 * 256 - 1000, 4 * 256 * 256 + 50000, 8 * 256 * 256 + 50000])
+@pytest.mark.parametrize("mode", ["parity", "f32", "unordered"])
+def test_few_tiles(va, orc, dim, neval, mode):
+    """From less than one tile, over one and two rounds of tiles per
+    workgroup, to the launch shape of many: two iterations in parity mode;
+    otherwise the oracle with the same 24-bit uniforms (FP32 bars)."""
+    c = [0.5 + 0.02 * ((d % 3) - 1) for d in range(dim)]
+    f, fo = va.GaussianMixture([1.0], [8.0], [c]), orc.GaussMix([1.0], [8.0], [c])
+    kw = dict(precision='f64', exact=True) if mode == "parity" else dict(precision='f32',
+                                                                         deterministic=mode == "f32")
+    integ = va.Integrator([[0, 1]] * dim, neval=neval, seed=31, **kw)
+    r = integ(f, nitn=2 if mode == "parity" else 1)
+    o = orc.OracleIntegrator([(0, 1)] * dim, neval=neval, seed=31, rng_f32=mode != "parity")
+    mean, var, nev = o.run(fo, len(r.itn_results))
+    assert integ.last_neval == nev[-1]
+    rm, rv, rg = (1e-12, 1e-10, 1e-11) if mode == "parity" else (2e-5, 2e-3, 1e-3)
+    for m, mo, vo in zip(r.itn_results, mean, var):
+        assert abs(m.mean - mo) <= rm * abs(mo)
+        assert abs(m.var - vo) <= rv * vo
+    np.testing.assert_allclose(integ.map.grid, o.map.grid, rtol=rg, atol=1e-13)

@@ -216,16 +216,23 @@ __device__ __forceinline__ void eval_point(const TileGeom& g, const AxisC* __res
             const double inc = g1 - g0;
             x[d] = __builtin_fma(inc, dl, g0);
             J *= inc;
-        } else if (k < ni) {
-            const double g0 = gd[k], g1 = gd[k + 1];
-            const double inc = g1 - g0;
-            x[d] = g0 + inc * dl;
-            J *= inc * (double)ni;
         } else {
-            x[d] = gd[ni];
-            J *= (gd[ni] - gd[ni - 1]) * (double)ni;
+            // (k = ninc: x is the last node, with the last increment); selects,
+            // no branch, so that the axes' grid reads overlap
+            const bool in = k < ni;
+            const double g0 = gd[in ? k : ni - 1], g1 = gd[in ? k + 1 : ni];
+            const double inc = g1 - g0;
+            x[d] = in ? g0 + inc * dl : g1;
+            J *= inc * (double)ni;
         }
         kbin[d] = kv;
+        if (!PER) {
+            // formed here: left to the compiler, bin and Jacobian are computed
+            // where they are used, after the integrand, and every axis' y,
+            // increment and indices stay in registers (and spill) until then
+            asm volatile("" : "+v"(kbin[d]));
+            asm volatile("" : "+v"(J));
+        }
     }
     if (PER) J *= g.jn;
 }
@@ -396,161 +403,91 @@ __device__ __forceinline__ void store_offsets(uint32_t* offs, int lane, const ui
         if (lane + kWave * q < kNoff) offs[lane + kWave * q] = v[q];
 }
 
-// One wave tile (kT points, kK per lane): sample, map, integrand, training
-// histogram, and the reference's two passes per hcube as segmented scans.
+// One point: hcube h (integral-local) of ncur points, weight factor wdiv =
+// dv_y / ncur, point index pj.  Samples, maps, evaluates, and stores or adds
+// the training data.  Returns w f.
 template <int DIM, bool PER, class Fcn>
-__device__ __forceinline__ void tile_body(const TileGeom& g, const TileIO& io, const Fcn& fcn,
-                                          const AxisC* __restrict__ ax, const double* __restrict__ G,
-                                          double* Ls, uint32_t* Lc, uint32_t* offs, const TilePos& tp,
-                                          int lane, TileAcc& acc) {
+__device__ __forceinline__ double tile_point(const TileGeom& g, const TileIO& io, const Fcn& fcn,
+                                             const AxisC* __restrict__ ax, const double* __restrict__ G,
+                                             double* Ls, uint32_t* Lc, const TilePos& tp, uint32_t h,
+                                             uint32_t ncur, double wdiv, const PackedCoords<DIM>& pc, uint32_t pj,
+                                             const uint32_t* perv, TileAcc& acc) {
     constexpr bool R32 = Fcn::kRng32;
     constexpr int ND = nd_max(DIM);
     const int dim = DIM > 0 ? DIM : g.dim;
-    const double eps = kEpsilon;
-    const uint32_t t = tp.t, plo = tp.plo, phi = tp.phi, hf = tp.hf;
-    // offs[] (the offsets of hcubes hf, hf+1, ...) is staged by the caller
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // hcube (local index) of this lane's first point
-    const uint32_t pl0 = plo + lane * kK;
-    int li = 0;
-    {
-        int lo = 0, hi = kNoff - 2;  // largest i with offs[i] <= pl0
-        while (lo < hi) {
-            int mid = (lo + hi + 1) >> 1;
-            if (offs[mid] <= pl0) lo = mid; else hi = mid - 1;
-        }
-        li = lo;
-    }
-    // Points are evaluated one at a time (no unrolling: one point's
-    // registers live at once); results rotate through a register window so
-    // element j ends in key[j], wf[j], nn[j].
-    int key[kK];
-    double wf[kK];
-    uint32_t nn[kK];
-#pragma unroll
-    for (int j = 0; j < kK; ++j) {
-        key[j] = kKeySentinel;
-        wf[j] = 0.0;
-        nn[j] = 1;
-    }
-    // hcube cur_i (local index) of the lane's current point: its end offset
-    // nxt, its point count, dv_y / n_h (pyx:1749) and, PER, its coordinates
-    int cur_i = li;
-    uint32_t nxt = 0xFFFFFFFFu;
-    double wdiv = 0.0;
-    uint32_t ncur = 1;
-    PackedCoords<DIM> pc;
-    if (pl0 < phi) {
-        nxt = offs[li + 1];
-        ncur = nxt - offs[li];
-        wdiv = g.dv_y / (double)ncur;
-        if (PER) pc.set(ax, dim, hf + li - tp.hbase);
-    }
-    // PER with the dimension known (up to 8 axes; above, the registers would
-    // spill): each axis's increments per stratum in a vector register for
-    // the tile (the empty asm leaves it there)
-    constexpr bool kPinPer = PER && DIM > 0 && DIM <= 8;
-    uint32_t perv[ND];
-    if constexpr (kPinPer) {
-#pragma unroll
-        for (int d = 0; d < ND; ++d) {
-            uint32_t v = ldc(ax, d).per;
-            asm volatile("" : "+v"(v));
-            perv[d] = v & 0xFFFFFu;
-        }
-    }
-#pragma unroll 1
-    for (int j = 0; j < kK; ++j) {
-        const uint32_t pj = pl0 + j;
-        int kj = kKeySentinel;
-        double vj = 0.0;
-        uint32_t nj = 1;
-        if (pj < phi) {
-            while (pj >= nxt && cur_i < kNoff - 2) {  // next hcube (one step: hcubes have >= 2 points)
-                ++cur_i;
-                const uint32_t o0 = nxt;
-                nxt = offs[cur_i + 1];
-                ncur = nxt - o0;
-                wdiv = g.dv_y / (double)ncur;
-                if (PER) pc.step(ax, dim);
-            }
-            kj = cur_i;
-            nj = ncur;
-            double x[ND];
-            int kb[ND];
-            double J;
-            uint32_t zmin = 0xFFFFFFFFu;
-            eval_point<DIM, R32, PER>(g, ax, G, pc, hf + cur_i - tp.hbase, pj - tp.pshift, x, J, kb, zmin,
-                                      kPinPer ? perv : nullptr);
-            const double w = J * wdiv;
-            const double f = fcn.template eval<DIM>(x, dim, pj);
-            if (f != f) acc.nan_seen = 1;
-            vj = w * f;
-            const double tn = vj * (double)ncur;
-            if (g.train_points) {
-                const double c2 = tn * tn;
-                if (io.rec_c2) {
-                    // a record per point; the histogram sums are built from
-                    // them in a fixed order (here, in tile order, or after the
-                    // launch); the counts, integers, need no order and go
-                    // into the LDS at once when Lc is given
-                    const uint64_t zm = (PER && zmin == 0) ? per_zero_axes<DIM>(g, pc, pj - tp.pshift) : 0ull;
-                    store_record<DIM>(io, dim, pj - io.rec_p0, kb, zm, c2);
-                    if (Lc) {
-                        if (PER && zm == 0) {
-                            // every axis inside (0,1): no per-axis test
-#pragma unroll
-                            for (int d = 0; d < ND; ++d) {
-                                if (DIM <= 0 && d >= dim) break;
-                                const int idx = d * g.nb + kb[d];
-                                atomicAdd(&Lc[idx >> 1], pair_inc(idx));
-                            }
-                        } else {
-#pragma unroll
-                            for (int d = 0; d < ND; ++d) {
-                                if (DIM <= 0 && d >= dim) break;
-                                const int k = kb[d];
-                                if (k < 0 || ((zm >> d) & 1)) continue;
-                                const int idx = d * g.nb + k;
-                                atomicAdd(&Lc[idx >> 1], pair_inc(idx));
-                            }
-                        }
-                    }
-                } else if (PER && zmin != 0) {
-                    // LDS histogram, every axis inside (0,1): no per-axis test
+    double x[ND];
+    int kb[ND];
+    double J;
+    uint32_t zmin = 0xFFFFFFFFu;
+    eval_point<DIM, R32, PER>(g, ax, G, pc, h, pj - tp.pshift, x, J, kb, zmin, perv);
+    const double w = J * wdiv;
+    const double f = fcn.template eval<DIM>(x, dim, pj);
+    if (f != f) acc.nan_seen = 1;
+    const double vj = w * f;
+    const double tn = vj * (double)ncur;
+    if (g.train_points) {
+        const double c2 = tn * tn;
+        if (io.rec_c2) {
+            // a record per point; the histogram sums are built from
+            // them in a fixed order (here, in tile order, or after the
+            // launch); the counts, integers, need no order and go
+            // into the LDS at once when Lc is given
+            const uint64_t zm = (PER && zmin == 0) ? per_zero_axes<DIM>(g, pc, pj - tp.pshift) : 0ull;
+            store_record<DIM>(io, dim, pj - io.rec_p0, kb, zm, c2);
+            if (Lc) {
+                if (PER && zm == 0) {
+                    // every axis inside (0,1): no per-axis test
 #pragma unroll
                     for (int d = 0; d < ND; ++d) {
                         if (DIM <= 0 && d >= dim) break;
                         const int idx = d * g.nb + kb[d];
-                        unsafeAtomicAdd(&Ls[idx], c2);
                         atomicAdd(&Lc[idx >> 1], pair_inc(idx));
                     }
                 } else {
-                    const uint64_t zm = (PER && zmin == 0) ? per_zero_axes<DIM>(g, pc, pj - tp.pshift) : 0ull;
 #pragma unroll
                     for (int d = 0; d < ND; ++d) {
                         if (DIM <= 0 && d >= dim) break;
                         const int k = kb[d];
                         if (k < 0 || ((zm >> d) & 1)) continue;
                         const int idx = d * g.nb + k;
-                        unsafeAtomicAdd(&Ls[idx], c2);
                         atomicAdd(&Lc[idx >> 1], pair_inc(idx));
                     }
                 }
             }
-        }
-        // rotate: element j enters at the back of the window
+        } else if (PER && zmin != 0) {
+            // LDS histogram, every axis inside (0,1): no per-axis test
 #pragma unroll
-        for (int q = 0; q < kK - 1; ++q) {
-            key[q] = key[q + 1];
-            wf[q] = wf[q + 1];
-            nn[q] = nn[q + 1];
+            for (int d = 0; d < ND; ++d) {
+                if (DIM <= 0 && d >= dim) break;
+                const int idx = d * g.nb + kb[d];
+                unsafeAtomicAdd(&Ls[idx], c2);
+                atomicAdd(&Lc[idx >> 1], pair_inc(idx));
+            }
+        } else {
+            const uint64_t zm = (PER && zmin == 0) ? per_zero_axes<DIM>(g, pc, pj - tp.pshift) : 0ull;
+#pragma unroll
+            for (int d = 0; d < ND; ++d) {
+                if (DIM <= 0 && d >= dim) break;
+                const int k = kb[d];
+                if (k < 0 || ((zm >> d) & 1)) continue;
+                const int idx = d * g.nb + k;
+                unsafeAtomicAdd(&Ls[idx], c2);
+                atomicAdd(&Lc[idx >> 1], pair_inc(idx));
+            }
         }
-        key[kK - 1] = kj;
-        wf[kK - 1] = vj;
-        nn[kK - 1] = nj;
     }
+    return vj;
+}
+
+// The reference's two passes per hcube over the tile's w f (element j of a
+// lane: point plo + lane * kK + j, of local hcube key[j] with nn[j] points)
+// as segmented scans: the sums of the tile's hcubes into acc, sigf, and the
+// slots of hcubes cut by its edges.  Runs on one wave.
+__device__ __forceinline__ void tile_scan(const TileGeom& g, const TileIO& io, const uint32_t* offs,
+                                          const TilePos& tp, int lane, int (&key)[kK], double (&wf)[kK],
+                                          uint32_t (&nn)[kK], TileAcc& acc) {
+    const double eps = kEpsilon;
+    const uint32_t t = tp.t, plo = tp.plo, phi = tp.phi, hf = tp.hf, pl0 = plo + lane * kK;
     // ---- pass 1: S per segment (pyx:2147-2152)
     double P[kK];
     seg_prefix(key, wf, P, lane);
@@ -692,6 +629,101 @@ __device__ __forceinline__ void tile_body(const TileGeom& g, const TileIO& io, c
     __builtin_amdgcn_wave_barrier();
 }
 
+// One wave tile (kT points, kK per lane): sample, map, integrand, training
+// histogram, and the reference's two passes per hcube as segmented scans.
+template <int DIM, bool PER, class Fcn>
+__device__ __forceinline__ void tile_body(const TileGeom& g, const TileIO& io, const Fcn& fcn,
+                                          const AxisC* __restrict__ ax, const double* __restrict__ G,
+                                          double* Ls, uint32_t* Lc, uint32_t* offs, const TilePos& tp,
+                                          int lane, TileAcc& acc) {
+    constexpr int ND = nd_max(DIM);
+    const int dim = DIM > 0 ? DIM : g.dim;
+    const uint32_t plo = tp.plo, phi = tp.phi, hf = tp.hf;
+    // offs[] (the offsets of hcubes hf, hf+1, ...) is staged by the caller
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    // hcube (local index) of this lane's first point
+    const uint32_t pl0 = plo + lane * kK;
+    int li = 0;
+    {
+        int lo = 0, hi = kNoff - 2;  // largest i with offs[i] <= pl0
+        while (lo < hi) {
+            int mid = (lo + hi + 1) >> 1;
+            if (offs[mid] <= pl0) lo = mid; else hi = mid - 1;
+        }
+        li = lo;
+    }
+    // Points are evaluated one at a time (no unrolling: one point's
+    // registers live at once); results rotate through a register window so
+    // element j ends in key[j], wf[j], nn[j].
+    int key[kK];
+    double wf[kK];
+    uint32_t nn[kK];
+#pragma unroll
+    for (int j = 0; j < kK; ++j) {
+        key[j] = kKeySentinel;
+        wf[j] = 0.0;
+        nn[j] = 1;
+    }
+    // hcube cur_i (local index) of the lane's current point: its end offset
+    // nxt, its point count, dv_y / n_h (pyx:1749) and, PER, its coordinates
+    int cur_i = li;
+    uint32_t nxt = 0xFFFFFFFFu;
+    double wdiv = 0.0;
+    uint32_t ncur = 1;
+    PackedCoords<DIM> pc;
+    if (pl0 < phi) {
+        nxt = offs[li + 1];
+        ncur = nxt - offs[li];
+        wdiv = g.dv_y / (double)ncur;
+        if (PER) pc.set(ax, dim, hf + li - tp.hbase);
+    }
+    // PER with the dimension known (up to 8 axes; above, the registers would
+    // spill): each axis's increments per stratum in a vector register for
+    // the tile (the empty asm leaves it there)
+    constexpr bool kPinPer = PER && DIM > 0 && DIM <= 8;
+    uint32_t perv[ND];
+    if constexpr (kPinPer) {
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+            uint32_t v = ldc(ax, d).per;
+            asm volatile("" : "+v"(v));
+            perv[d] = v & 0xFFFFFu;
+        }
+    }
+#pragma unroll 1
+    for (int j = 0; j < kK; ++j) {
+        const uint32_t pj = pl0 + j;
+        int kj = kKeySentinel;
+        double vj = 0.0;
+        uint32_t nj = 1;
+        if (pj < phi) {
+            while (pj >= nxt && cur_i < kNoff - 2) {  // next hcube (one step: hcubes have >= 2 points)
+                ++cur_i;
+                const uint32_t o0 = nxt;
+                nxt = offs[cur_i + 1];
+                ncur = nxt - o0;
+                wdiv = g.dv_y / (double)ncur;
+                if (PER) pc.step(ax, dim);
+            }
+            kj = cur_i;
+            nj = ncur;
+            vj = tile_point<DIM, PER>(g, io, fcn, ax, G, Ls, Lc, tp, hf + cur_i - tp.hbase, ncur, wdiv, pc, pj,
+                                      kPinPer ? perv : nullptr, acc);
+        }
+        // rotate: element j enters at the back of the window
+#pragma unroll
+        for (int q = 0; q < kK - 1; ++q) {
+            key[q] = key[q + 1];
+            wf[q] = wf[q + 1];
+            nn[q] = nn[q + 1];
+        }
+        key[kK - 1] = kj;
+        wf[kK - 1] = vj;
+        nn[kK - 1] = nj;
+    }
+    tile_scan(g, io, offs, tp, lane, key, wf, nn, acc);
+}
 
 // The u16 pair-packed LDS counts into a workgroup's own row of u32 counts
 // (written, or added to when add), one lane per pair.
@@ -913,8 +945,22 @@ __device__ inline void block_close_tiles(const TileAcc& acc, const double* tpart
     }
 }
 
+// Threads of a sampler workgroup (one per CU): 16 waves as long as the kernel
+// fits their 128 registers, else 12 (168) or 8 (256).  No sampler may spill
+// vector registers: besides the time, this compiler places some of the spill
+// stores before the exec mask is restored at the end of a branch, and the
+// lanes that skipped the branch then lose the value (the 9-axis FP64 sampler's
+// sums came out wrong so).  us per launch of 1e6 points, 1024 threads with
+// spills / without: 9 axes f64 49 / 41, 13 axes 91 / 61.
+constexpr int sampler_threads(int dim, bool per) {
+    if (dim > 16) dim = 0;
+    if (dim <= 0) return per ? 768 : kFusedThreads;  // (runtime dimension: its arrays are in scratch)
+    if (dim <= (per ? 9 : 6)) return kFusedThreads;
+    return dim <= (per ? 14 : 10) ? 768 : 512;
+}
+
 template <int DIM, bool PER, class Fcn>
-__global__ __launch_bounds__(kFusedThreads) void fused_kernel(IterGeom g, FusedPtrs io, Fcn fcn) {
+__global__ __launch_bounds__(sampler_threads(DIM, PER)) void fused_kernel(IterGeom g, FusedPtrs io, Fcn fcn) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int s_skip;
     __shared__ uint32_t s_broken;
@@ -1108,31 +1154,167 @@ __global__ __launch_bounds__(kFusedThreads) void fused_kernel(IterGeom g, FusedP
     block_close_tiles(acc, io.tile_part, tb, te, io.blk_part + 6 * (size_t)blockIdx.x, sc);
 }
 
+// The sampler of a launch with few tiles.  fused_kernel's waves each take a
+// whole tile, so with a few tiles per CU most of its waves have none and the
+// launch lasts as long as one wave needs for four points per lane in turn.
+// Here four waves share a tile: each evaluates 64 of its points, one per lane
+// (w f goes through LDS), then one of the four does the tile's scans, the
+// same operations on the same values as fused_kernel (same bits); 16 waves
+// take four tiles a round.  The ordered LDS histogram needs no locks here:
+// after the last round, wave k adds the records of axis pair k in tile order.
+// Latency bound: a round's points, then its scans.
+constexpr int kSplitGroups = kFusedThreads / 64 / 4;  // tiles per round, at most
+// LDS after the offsets slices: w f of kSplitGroups tiles
+constexpr size_t kSplitLds = (size_t)kSplitGroups * kT * sizeof(double);
+
+template <int DIM, bool PER, class Fcn>
+__global__ __launch_bounds__(sampler_threads(DIM, PER)) void split_kernel(IterGeom g, FusedPtrs io, Fcn fcn) {
+    constexpr int kThreads = sampler_threads(DIM, PER), kGroups = kThreads / 64 / 4;
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ int s_skip;
+    Scalars* sc = io.sc;
+    if (threadIdx.x == 0) s_skip = sc->status;
+    const TileGeom tg = tile_geom(g);
+    const int dim = DIM > 0 ? DIM : g.dim;
+    const uint32_t ntiles = sc->b_ntiles, p0 = sc->b_p0, p1 = sc->b_p1, hend = sc->b_h1;
+    const uint32_t off_end = io.off[hend];
+    const int tot = dim * g.nb;
+    const bool lds_hist = PER && g.hist_lds && g.train_points;
+    // ---- LDS: grid | histogram sums, u16 pair counts | offsets slices | w f
+    double* const G = reinterpret_cast<double*>(smem);
+    size_t cur = (size_t)dim * g.ld * sizeof(double);
+    double* const Ls = reinterpret_cast<double*>(smem + cur);
+    uint32_t* const Lc = reinterpret_cast<uint32_t*>(smem + cur + (size_t)tot * sizeof(double));
+    if (lds_hist) cur += (size_t)tot * sizeof(double) + (size_t)((tot + 1) / 2) * sizeof(uint32_t);
+    cur = (cur + 15) & ~(size_t)15;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, grp = wave >> 2, sub = wave & 3;
+    uint32_t* const offs = reinterpret_cast<uint32_t*>(smem + cur) + wave * kNoff;
+    double* const xch = reinterpret_cast<double*>(smem + cur + (size_t)16 * kNoff * sizeof(uint32_t)) + grp * kT;
+    for (int i = threadIdx.x; i < dim * g.ld; i += kThreads) G[i] = io.grid[i];
+    if (lds_hist) {
+        for (int i = threadIdx.x; i < tot; i += kThreads) Ls[i] = 0.0;
+        for (int i = threadIdx.x; i < (tot + 1) / 2; i += kThreads) Lc[i] = 0u;
+    }
+    const bool unordered = lds_hist && g.hist_unordered;
+    const TileIO tio{io.off, io.sigf, io.slots, io.errv, unordered ? nullptr : io.rec_bins,
+                     unordered ? nullptr : io.rec_c2, p0, io.rec_stride};
+    const AxisC* ax = io.axes;
+    const uint32_t chunk = (ntiles + gridDim.x - 1) / gridDim.x;
+    const uint32_t tb = blockIdx.x * chunk, te = min(tb + chunk, ntiles);
+    TileAcc acc{{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, 0};
+    __syncthreads();
+    if (s_skip) return;
+#pragma unroll 1
+    for (uint32_t t0 = tb; t0 < te; t0 += kGroups) {
+        const uint32_t t = t0 + (uint32_t)grp;
+        TilePos tp{};
+        if (t < te) {
+            const uint32_t plo = p0 + t * kT;
+            tp = TilePos{t, plo, min(plo + (uint32_t)kT, p1), (uint32_t)io.tile_h[t], hend, off_end, 0u, 0u};
+            uint32_t ov[kOffRegs];
+            load_offsets(io.off, tp.hf, hend, off_end, lane, ov);
+            store_offsets(offs, lane, ov);
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const uint32_t pj = plo + (uint32_t)(sub * kWave + lane);
+            double v = 0.0;
+            if (pj < tp.phi) {
+                int lo = 0, hi = kNoff - 2;  // largest i with offs[i] <= pj
+                while (lo < hi) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    if (offs[mid] <= pj) lo = mid; else hi = mid - 1;
+                }
+                const uint32_t n = offs[lo + 1] - offs[lo], h = tp.hf + (uint32_t)lo;
+                PackedCoords<DIM> pc;
+                if (PER) pc.set(ax, dim, h);
+                v = tile_point<DIM, PER>(tg, tio, fcn, ax, G, unordered ? Ls : nullptr, lds_hist ? Lc : nullptr, tp, h,
+                                         n, tg.dv_y / (double)n, pc, pj, nullptr, acc);
+            }
+            xch[sub * kWave + lane] = v;
+        }
+        __syncthreads();
+        if (t < te && sub == 0) {
+            const uint32_t pl0 = tp.plo + (uint32_t)lane * kK;
+            int key[kK];
+            double wf[kK];
+            uint32_t nn[kK];
+            int li = 0, hi = kNoff - 2;
+            while (li < hi) {
+                const int mid = (li + hi + 1) >> 1;
+                if (offs[mid] <= pl0) li = mid; else hi = mid - 1;
+            }
+#pragma unroll
+            for (int j = 0; j < kK; ++j) {
+                const uint32_t pj = pl0 + j;
+                const bool live = pj < tp.phi;
+                // (hcubes have two points or more: one step at most)
+                if (live && pj >= offs[li + 1] && li < kNoff - 2) ++li;
+                key[j] = live ? li : kKeySentinel;
+                wf[j] = live ? xch[lane * kK + j] : 0.0;
+                nn[j] = live ? offs[li + 1] - offs[li] : 1u;
+            }
+            tile_scan(tg, tio, offs, tp, lane, key, wf, nn, acc);
+            const double m = wave_total(acc.am.hi + acc.am.lo), v = wave_total(acc.av.hi + acc.av.lo),
+                         q = wave_total(acc.as.hi + acc.as.lo);
+            if (lane == 63) {
+                double* o = io.tile_part + 3 * (size_t)t;
+                o[0] = m; o[1] = v; o[2] = q;
+            }
+            acc.am = DD{0.0, 0.0};
+            acc.av = DD{0.0, 0.0};
+            acc.as = DD{0.0, 0.0};
+        }
+        __syncthreads();
+    }
+    if (lds_hist) {
+        if (!unordered) {
+            // the records of this workgroup's tiles (stored before the barrier)
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+            for (int k = wave; k < (dim + kGroupAxes - 1) / kGroupAxes; k += kThreads / 64) {
+                PairRec R, N;
+                if (tb < te) pair_load(tio, k, tb * (uint32_t)kT, lane, R);
+                for (uint32_t t = tb; t < te; ++t) {
+                    if (t + 1 < te) pair_load(tio, k, (t + 1) * (uint32_t)kT, lane, N);
+                    pair_add(tg, dim, k, R, min((uint32_t)kT, p1 - p0 - t * kT), Ls, lane);
+                    R = N;
+                }
+            }
+            __syncthreads();
+        }
+        double* srow = io.hpart_s + (size_t)blockIdx.x * tot;
+        for (int i = threadIdx.x; i < tot; i += kThreads) srow[i] = Ls[i];
+        counts_to_row(Lc, tot, io.hpart_c + (size_t)blockIdx.x * tot, false, false);
+    }
+    block_close_tiles(acc, io.tile_part, tb, te, io.blk_part + 6 * (size_t)blockIdx.x, sc);
+}
+
 template <int DIM, class Fcn>
 int launch_fused_dim(const IterGeom& g, const FusedPtrs& io, const Fcn& fcn, int blocks, size_t lds,
                      hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
-    auto kern = fused_kernel<DIM, false, Fcn>;
+    auto kern = g.split ? split_kernel<DIM, false, Fcn> : fused_kernel<DIM, false, Fcn>;
     if constexpr (Fcn::kRng32) {
-        if (g.per_all) kern = fused_kernel<DIM, true, Fcn>;
+        if (g.per_all) kern = g.split ? split_kernel<DIM, true, Fcn> : fused_kernel<DIM, true, Fcn>;
     }
     // the LDS limit of this instantiation is raised once, to the largest
     // request seen (a host-side attribute, not a per-launch cost)
     static size_t lds_set = 64 * 1024;
     if (lds > lds_set) {
-        if (hipFuncSetAttribute((const void*)fused_kernel<DIM, false, Fcn>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+        auto raise = [&](const void* k) {
+            return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+        };
+        if (!raise((const void*)fused_kernel<DIM, false, Fcn>) || !raise((const void*)split_kernel<DIM, false, Fcn>))
             return VGX_EHIP;
         if constexpr (Fcn::kRng32) {
-            if (hipFuncSetAttribute((const void*)fused_kernel<DIM, true, Fcn>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+            if (!raise((const void*)fused_kernel<DIM, true, Fcn>) || !raise((const void*)split_kernel<DIM, true, Fcn>))
                 return VGX_EHIP;
         }
         lds_set = lds;
     }
+    const int threads = sampler_threads(DIM, g.per_all && Fcn::kRng32);
     if (ev0)
-        hipExtLaunchKernelGGL(kern, dim3(blocks), dim3(kFusedThreads), (uint32_t)lds, st, ev0, ev1, 0, g, io, fcn);
+        hipExtLaunchKernelGGL(kern, dim3(blocks), dim3(threads), (uint32_t)lds, st, ev0, ev1, 0, g, io, fcn);
     else
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kFusedThreads), lds, st, g, io, fcn);
+        hipLaunchKernelGGL(kern, dim3(blocks), dim3(threads), lds, st, g, io, fcn);
     return check_launch();
 }
 

@@ -843,7 +843,19 @@ static size_t fused_lds(const IterGeom& g) {
         b += tot * sizeof(double) + ((tot + 1) / 2) * sizeof(uint32_t);
     b = (b + 15) & ~(size_t)15;
     b += (size_t)16 * kNoff * sizeof(uint32_t);
+    if (g.split) b += kSplitLds;
     return b;
+}
+
+// Few tiles per workgroup: split_kernel, where its LDS plan fits too.  It pays
+// as long as it needs one round of tiles (four waves each), and a second on
+// the 8-wave samplers.  us per launch, fused / split: 1.2e5 points 4 axes f64
+// 18 / 14, 8 axes f32 31 / 26; 2.5e5 (four tiles) 8 axes f32 32 / 30, 14 axes
+// f64 39 / 35; 3.2e5 (two rounds of four waves) 8 axes f32 34 / 38.
+static void plan_split(const DeviceInfo& info, uint32_t tiles, uint32_t blocks, IterGeom* g) {
+    const int waves = (g->rng32 && g->per_all ? sampler_threads(g->dim, true) : sampler_threads(g->dim, false)) / 64;
+    g->split = tiles <= (waves == 8 ? 4u : (uint32_t)waves / 4u) * blocks;
+    if (fused_lds(*g) + 1024 > info.max_lds) g->split = 0;
 }
 
 static uint64_t max_points(const vgx_config* c, const IterGeom& g) {
@@ -875,7 +887,9 @@ struct Run {
     uint32_t* rows_c;
 };
 
-static int prepare(vgx_ctx* ctx, const vgx_config* c, vgx_state* st, Run* R) {
+// npts: points of the batch to be sampled or accumulated (0: as many as the
+// allocation may give a whole iteration).
+static int prepare(vgx_ctx* ctx, const vgx_config* c, vgx_state* st, Run* R, uint64_t npts = 0) {
     int rc = build_geom(c, ctx->info, &R->g);
     if (rc) return rc;
     const IterGeom& g = R->g;
@@ -883,7 +897,11 @@ static int prepare(vgx_ctx* ctx, const vgx_config* c, vgx_state* st, Run* R) {
     if (R->cap >= 0xFFFFFFF0ull) return VGX_ERANGE;
     R->maxtiles = (uint32_t)((R->cap + kT - 1) / kT) + 1;
     R->nblk_alloc = (int)((c->nhcube + kAllocPerBlock - 1) / kAllocPerBlock);
-    R->fused_blocks = ctx->info.cus;
+    // (workgroups past the last tile would only write empty rows and sums)
+    const uint64_t pts = npts ? npts : R->cap;
+    const uint32_t tiles = (uint32_t)((pts + kT - 1) / kT);
+    R->fused_blocks = (int)(tiles < (uint32_t)ctx->info.cus ? tiles : (uint32_t)ctx->info.cus);
+    plan_split(ctx->info, tiles, (uint32_t)R->fused_blocks, &R->g);
     R->strad_blocks = (int)((2ull * R->maxtiles + kStradThreads - 1) / kStradThreads);
     R->lds = fused_lds(g);
     if (R->lds > ctx->info.max_lds) return VGX_ERANGE;
@@ -1217,7 +1235,7 @@ extern "C" int vgx_iter_accumulate(vgx_ctx* ctx, const vgx_config* c, vgx_state*
     if (h0 < 0 || h1 > c->nhcube || h0 >= h1 || p0 < 0 || p1 <= p0) return VGX_EINVAL;
     hipStream_t s = (hipStream_t)stream;
     Run R;
-    int rc = prepare(ctx, c, st, &R);
+    int rc = prepare(ctx, c, st, &R, (uint64_t)(p1 - p0));
     if (rc) return rc;
     if ((rc = init_axes(&R, s))) return rc;
     set_iter(&R, c, it);

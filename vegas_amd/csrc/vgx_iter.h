@@ -30,6 +30,7 @@ struct IterGeom {
     int rng32;             // 24-bit uniforms (FP32 integrand) else 53-bit
     int exact_div;         // y = (c+u)/s by IEEE division
     int hist_lds, grid_lds;
+    int split;             // few tiles: split_kernel instead of fused_kernel
     int hist_unordered;    // hist_lds: LDS atomics in timing order (VGX_FLAG_UNORDERED_HIST)
     int weighted;
     int adapt;
