@@ -63,3 +63,38 @@ def test_few_tiles(va, orc, dim, neval, mode):
         assert abs(m.mean - mo) <= rm * abs(mo)
         assert abs(m.var - vo) <= rv * vo
     np.testing.assert_allclose(integ.map.grid, o.map.grid, rtol=rg, atol=1e-13)
+
+
+@pytest.mark.parametrize("nc,dim,neval,kind", [(256, 5, 4200000, "zeros"), (257, 12, 4200000, "plain"),
+                                               (258, 8, 4200000, "negative"), (259, 7, 4200000, "wide"),
+                                               (259, 6, 4200000, "huge"), (255, 8, 4200000, "plain"),
+                                               (259, 4, 4200000, "plain"), (259, 13, 4200000, "plain")])
+def test_long_mixture(va, nc, dim, neval, kind):
+    """The long mixtures' loop and its neighbours, with every remainder of its
+    steps, against FP64 terms at the same points (FP32 bars)."""
+    import torch
+    rng = np.random.default_rng(nc)
+    sigma = 0.4 if kind == "wide" else 0.03 * np.sqrt(dim)
+    f32 = lambda a: np.asarray(a, np.float32).astype(np.float64)
+    A = f32(rng.uniform(0.5, 1.5, nc) * (1e30 if kind == "huge" else 1.0))
+    if kind == "zeros":
+        A[::3] = 0.0
+        A[-1] = 0.0
+    if kind == "negative":
+        A[::5] *= -0.25
+    B = f32(0.5 / (sigma * rng.uniform(0.7, 1.3, nc)) ** 2)
+    c = f32(np.linspace(0.25, 0.75, nc)[:, None] + rng.uniform(-0.02, 0.02, (nc, dim)))
+    f = va.GaussianMixture(A, B, c)
+    dA, dB, dc = (torch.as_tensor(a, device="cuda") for a in (A, B, c))
+
+    @va.gpu_lbatchintegrand
+    def g(x):
+        y = torch.zeros(x.shape[0], dtype=torch.float64, device=x.device)
+        for k in range(nc):
+            y += dA[k] * torch.exp(-dB[k] * ((x - dc[k]) ** 2).sum(1))
+        return y
+
+    ra = va.Integrator([[0, 1]] * dim, neval=neval, seed=29, precision='f32')(f, nitn=1).itn_results[0]
+    rb = va.Integrator([[0, 1]] * dim, neval=neval, seed=29, precision='f32')(g, nitn=1).itn_results[0]
+    assert abs(ra.mean - rb.mean) <= 2e-5 * abs(rb.mean)
+    assert abs(ra.sdev - rb.sdev) <= 1e-3 * rb.sdev

@@ -736,6 +736,24 @@ __global__ void to_float_kernel(const double* a, float* b, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) b[i] = (float)a[i];
 }
 
+// out[0]: the least integer e (as a float) with every A[i] < 2^e; infinity
+// when one is negative or not finite.
+__global__ __launch_bounds__(1024) void max_exponent_kernel(const double* A, int n, float* out) {
+    __shared__ float red[16];
+    float m = -INFINITY;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        const double a = (double)(float)A[i];
+        m = fmaxf(m, a == 0.0 ? -INFINITY : a > 0.0 && a < INFINITY ? (float)__builtin_amdgcn_frexp_exp(a) : INFINITY);
+    }
+    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, kWave));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; ++w) m = fmaxf(m, red[w]);
+        out[0] = m;
+    }
+}
+
 // Staged path: x, y, weight and hcube of points [p0, p1) (pyx:1731-1759).
 template <bool R32>
 __global__ __launch_bounds__(256) void sample_kernel(IterGeom g, const AxisC* axes, const double* grid,
@@ -878,6 +896,7 @@ struct Run {
     uint64_t* stat;
     int32_t* nh;
     float* fparams;
+    float* fmax;  // GaussMany32's exponent bound
     AxisC* axes;
     double* errv;
     double* sigf_part;
@@ -919,12 +938,13 @@ static int prepare(vgx_ctx* ctx, const vgx_config* c, vgx_state* st, Run* R, uin
         R->errv = (double*)ctx->errv.ptr;
     }
     // misc: Scalars | axes | sigf partials | float integrand parameters
-    const size_t misc = 1024 + VGX_MAXDIM * sizeof(AxisC) + 2 * 256 * sizeof(double) + 1024 * 1024;
+    const size_t misc = 1024 + VGX_MAXDIM * sizeof(AxisC) + 2 * 256 * sizeof(double) + 1024 * 1024 + 64;
     if ((rc = ctx->misc.ensure(misc))) return rc;
     R->sc = (Scalars*)ctx->misc.ptr;
     R->axes = (AxisC*)((char*)ctx->misc.ptr + 1024);
     R->sigf_part = (double*)((char*)R->axes + VGX_MAXDIM * sizeof(AxisC));
     R->fparams = (float*)((char*)R->sigf_part + 2 * 256 * sizeof(double));
+    R->fmax = R->fparams + 256 * 1024;
     R->stat = (uint64_t*)ctx->blocksum.ptr;
     R->nh = (int32_t*)ctx->nh.ptr;
     FusedPtrs& io = R->io;
@@ -1141,6 +1161,11 @@ static int make_fcn_and_run(vgx_ctx* ctx, Run* R, const vgx_config* c, const vgx
                 hipLaunchKernelGGL(to_float_kernel, dim3(64), dim3(256), 0, s, f->A, A, nc);
                 hipLaunchKernelGGL(to_float_kernel, dim3(64), dim3(256), 0, s, f->B, B, nc);
                 hipLaunchKernelGGL(to_float_kernel, dim3(64), dim3(256), 0, s, f->c, C, ncc);
+            }
+            if (f->kind == VGX_FCN_GAUSSMIX && many_pays(nc, c->dim, c->neval)) {
+                if (convert) hipLaunchKernelGGL(max_exponent_kernel, dim3(1), dim3(1024), 0, s, f->A, nc, R->fmax);
+                GaussMany32 fn{nc, A, B, C, R->fmax};
+                return accumulate_kernels(ctx, R, fn, s, timed, reduce);
             }
             if (f->kind == VGX_FCN_GAUSSMIX) {
                 GaussMix32 fn{nc, A, B, C};
