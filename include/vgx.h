@@ -315,7 +315,8 @@ int vgx_flow_get_params(const vgx_flow* fl, float* host, float* grad_host, void*
  * sums[0] = sum f J, sums[1] = sum (f J)^2 (host; the call then waits for
  * the stream).  sums may be NULL when xout and fout are given: nothing is
  * read back and the call returns without waiting.  fcn: GAUSSMIX or
- * DIAGRIDGE with device FP64 parameters (evaluated in FP32).  xout, fout
+ * DIAGRIDGE with device FP64 parameters (evaluated in FP32; read by the
+ * kernel, so kept until the stream has passed it).  xout, fout
  * (device, optional): the points and f J.  status: device int32, set to
  * VGX_ENAN when f is NaN.                                                 */
 int vgx_flow_sample(vgx_flow* fl, const vgx_integrand* fcn, int64_t n, uint64_t base, uint64_t seed,

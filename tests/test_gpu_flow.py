@@ -258,3 +258,47 @@ def test_config3_ridge_8d_flow_and_grid(torch):
           "%.6f +- %.2g from %d samples" % (r.itn_results[-1].mean, fm.flow_var_per_sample, vegas_var,
                                             est.mean, est.sdev, n))
     assert est.sdev < 1e-3 * abs(est.mean) and abs(est.mean - 1.0) < 5 * est.sdev, (est.mean, est.sdev, n)
+
+
+def test_sample_shapes_agree(torch):
+    """The first n of many samples are the same bits at every launch shape
+    (4, 8, 12 waves, 2 or 6 tiles, several passes), and so are the sums and
+    the inverse."""
+    import vegas_amd as va
+    from vegas_amd.flow import CouplingFlow
+    f = va.DiagonalRidge([1.0] * 17, [20.0] * 17, np.linspace(0.3, 0.7, 17), 5)
+    flow = CouplingFlow(5, 4, seed=3)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    N = 2 * 72 * 16 * cus + 3
+    _, _, x, fj = flow.sample(f, N, seed=7, iteration=2, keep_points=True)
+    lq, u0 = flow.logq(x)
+    for n in (1, 127, 8 * 16 * cus, 8 * 16 * cus + 1, 16 * 16 * cus + 1, 24 * 16 * cus, 24 * 16 * cus + 1,
+              72 * 16 * cus + 5):
+        s1, s2, xn, fn = flow.sample(f, n, seed=7, iteration=2, keep_points=True)
+        # as bits: a coordinate z that rounds to 1 makes its f J a NaN
+        assert torch.equal(xn, x[:n]) and torch.equal(fn.view(torch.int32), fj[:n].view(torch.int32))
+        # sums are of f J before the rounding to FP32 (2^-24 a term)
+        np.testing.assert_allclose(s1, fj[:n].double().sum().item(), rtol=6e-8)
+        np.testing.assert_allclose(s2, (fj[:n].double() ** 2).sum().item(), rtol=1.2e-7)
+        lqn, un = flow.logq(xn)
+        assert torch.equal(lqn, lq[:n]) and torch.equal(un, u0[:n])
+
+
+@pytest.mark.parametrize("nc", [1, 3, 4, 15, 16, 17, 33, 2000, 4000])
+def test_ridge_component_counts(torch, nc):
+    """The ridge's unrolled loop with every remainder and, at 4000 terms,
+    with fewer waves: f J against FP64 terms at the points, J from a run with
+    one wide term.  B r^2 <= 60 here with a relative error of about 4 2^-24
+    each: 3e-5 for the two runs' quotient, held to 1e-4."""
+    import vegas_amd as va
+    from vegas_amd.flow import CouplingFlow
+    flow = CouplingFlow(3, 3, seed=5)
+    t = np.linspace(0.3, 0.7, nc)
+    f, one = va.DiagonalRidge(1.0 + t, [20.0] * nc, t, 3), va.DiagonalRidge([1.0], [1e-3], [0.5], 3)
+    _, _, x, fj = flow.sample(f, 5000, seed=9, keep_points=True)
+    _, _, x1, f1 = flow.sample(one, 5000, seed=9, keep_points=True)
+    assert torch.equal(x, x1)
+    xs = x[:, :3].double().cpu().numpy()
+    want = f1.double().cpu().numpy() / one(xs) * f(xs)
+    np.testing.assert_allclose(fj.double().cpu().numpy(), want, rtol=1e-4, atol=0)
+    np.testing.assert_allclose(flow.eval_fcn(f, x).double().cpu().numpy(), f(xs), rtol=1e-4, atol=0)

@@ -47,14 +47,28 @@ constexpr float kSMax = 4.0f;
 // FP32 master parameters of one layer: W1 | W2 | b2 | W3 | b3
 constexpr int kPW1 = 0, kPW2 = kPW1 + kFH * kFI, kPB2 = kPW2 + kFH * kFH, kPW3 = kPB2 + kFH,
               kPB3 = kPW3 + kFO * kFH, kPLayer = kPB3 + kFO;
-// bf16 weights of one layer: W1 | W2 | W3, and the transposes W1t | W2t | W3t,
-// with padded row strides so that the 16 rows of an MFMA A fragment fall in
-// distinct LDS banks (a 256-byte stride puts them all in one bank)
-constexpr int kS1 = 20, kS2 = 132, kS3 = 132;          // W1 [128][16], W2 [128][128], W3 [32][128]
-constexpr int kT1 = 132, kT2 = 132, kT3 = 36;          // W1t [16][128], W2t [128][128], W3t [128][32]
-constexpr int kHW1 = 0, kHW2 = kHW1 + kFH * kS1, kHW3 = kHW2 + kFH * kS2, kHLayer = kHW3 + kFO * kS3;
-constexpr int kTW1 = 0, kTW2 = kTW1 + kFI * kT1, kTW3 = kTW2 + kFH * kT2;
-static_assert(kTW3 + kFH * kT3 <= kHLayer, "transposed layout fits the layer block");
+// bf16 weights of one layer, W1 | W2 | W3, and the transposes W1t [16][128] |
+// W2t [128][128] | W3t [128][32], in MFMA fragment order: blocks of 64 lanes
+// by 8 values, so that an A operand is one 16-byte LDS read per lane whose
+// lanes are consecutive (a row-major layout, whatever its padding, took two
+// 8-byte reads with every second bank shared).  Value j of lane l of block
+//   W2, W3, W1t, W2t (mt, kp): row 16 mt + l%16, column 32 kp + 16 (j/4) +
+//                              4 (l/16) + j%4 (k-steps 2 kp and 2 kp + 1)
+//   W3t: the same with its one kp; W1 (p): row 16 (2 p + j/4) + l%16, column
+//                              4 (l/16) + j%4 (output tiles 2 p and 2 p + 1)
+constexpr int kFrag = 64 * 8;
+constexpr int kHW1 = 0, kHW2 = kHW1 + kFH * kFI, kHW3 = kHW2 + kFH * kFH, kHLayer = kHW3 + kFO * kFH;
+constexpr int kTW1 = 0, kTW2 = kTW1 + kFI * kFH, kTW3 = kTW2 + kFH * kFH;
+
+// Where element (row, col) of a matrix of nkp column blocks of 32 lies.
+__host__ __device__ constexpr int frag_pos(int row, int col, int nkp) {
+    return ((row >> 4) * nkp + (col >> 5)) * kFrag + (16 * ((col >> 2) & 3) + (row & 15)) * 8 + 4 * ((col >> 4) & 1) +
+           (col & 3);
+}
+// The same of W1 [128][16].
+__host__ __device__ constexpr int frag_pos1(int row, int col) {
+    return (row >> 5) * kFrag + (16 * (col >> 2) + (row & 15)) * 8 + 4 * ((row >> 4) & 1) + (col & 3);
+}
 
 // FP32 -> bf16, round to nearest even (v_cvt_pk_bf16_f32 on gfx950).
 __device__ inline uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
@@ -88,26 +102,42 @@ __device__ inline f32x4_t mfma32(bf16x8_t a, bf16x8_t b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// A operand fragment of W (bf16 row-major, row stride `ld`): rows 16 mt ..,
-// columns 16 kt + (l/16)*4 .. +3.
-__device__ inline bf16x4_t frag_a(const uint16_t* W, int ld, int mt, int kt, int lane) {
-    return *reinterpret_cast<const bf16x4_t*>(W + (16 * mt + (lane & 15)) * ld + 16 * kt + (lane >> 4) * 4);
+// Block b of weights in fragment order: this lane's 8 values.
+__device__ inline bf16x8_t frag_w(const uint16_t* W, int b, int lane) {
+    return *reinterpret_cast<const bf16x8_t*>(W + b * kFrag + lane * 8);
 }
-// The A operand of k-steps kt and kt+1 together (mfma32).
-__device__ inline bf16x8_t frag_a2(const uint16_t* W, int ld, int mt, int kt, int lane) {
-    const uint16_t* p = W + (16 * mt + (lane & 15)) * ld + 16 * kt + (lane >> 4) * 4;
-    return cat8(*reinterpret_cast<const bf16x4_t*>(p), *reinterpret_cast<const bf16x4_t*>(p + 16));
+__device__ inline bf16x4_t half8(bf16x8_t v, int hi) {
+    typedef short s16x8_t __attribute__((ext_vector_type(8)));
+    const s16x8_t w = __builtin_bit_cast(s16x8_t, v);
+    return hi ? __builtin_shufflevector(w, w, 4, 5, 6, 7) : __builtin_shufflevector(w, w, 0, 1, 2, 3);
 }
+
+// max(v, 0), 0 for a NaN: the median with 0 and infinity (relu_top) in one
+// instruction (fmaxf takes a second to quiet its operand, 64 more a tile and
+// layer; so does the median with a known infinity, which becomes fmaxf).
+__device__ inline float relu_top() {
+    float top = INFINITY;
+    asm("" : "+s"(top));
+    return top;
+}
+__device__ inline float relu(float v, float top) { return __builtin_amdgcn_fmed3f(v, 0.0f, top); }
 
 __device__ inline float logsigp(float u) {
     const float au = fabsf(u);
     return -au - 2.0f * __logf(1.0f + __expf(-au));
 }
 
-__device__ inline float tanh_f(float x) {
-    const float e = __expf(-2.0f * fabsf(x));
-    const float t = (1.0f - e) / (1.0f + e);
-    return copysignf(t, x);
+// tanh(x / kSMax) = (1 - e)/(1 + e), e = exp(-2 |x| / kSMax) in [0, 1]: the
+// quotient by the reciprocal, refined, and one correction of the quotient
+// (the steps of a division without its scaling, which 1 <= 1 + e <= 2 does
+// not need).
+__device__ inline float tanh_s(float x) {
+    const float e = __expf(fabsf(x) * (-2.0f / kSMax));
+    const float n = 1.0f - e, d = 1.0f + e;
+    float r = __builtin_amdgcn_rcpf(d);
+    r = __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+    const float q = n * r;
+    return copysignf(__builtin_fmaf(__builtin_fmaf(-d, q, n), r, q), x);
 }
 
 __device__ inline float group_sum(float v) {
@@ -126,18 +156,18 @@ struct FlowArgs {
 
 // One layer's weights and biases in LDS.
 struct LayerLds {
-    uint16_t W[kHLayer];
-    float b2[kFH], b3[kFO];
+    alignas(16) uint16_t W[kHLayer];
+    alignas(16) float b2[kFH], b3[kFO];
 };
 
 __device__ inline void load_layer(const FlowArgs& f, int k, LayerLds* s, bool transposed, uint16_t* Wt) {
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(f.H + (size_t)k * kHLayer);
-    uint32_t* dst = reinterpret_cast<uint32_t*>(s->W);
-    for (int i = threadIdx.x; i < kHLayer / 2; i += blockDim.x) dst[i] = src[i];
+    const uint4* src = reinterpret_cast<const uint4*>(f.H + (size_t)k * kHLayer);
+    uint4* dst = reinterpret_cast<uint4*>(s->W);
+    for (int i = threadIdx.x; i < kHLayer / 8; i += blockDim.x) dst[i] = src[i];
     if (transposed) {
-        const uint32_t* st = reinterpret_cast<const uint32_t*>(f.HT + (size_t)k * kHLayer);
-        uint32_t* dt = reinterpret_cast<uint32_t*>(Wt);
-        for (int i = threadIdx.x; i < kHLayer / 2; i += blockDim.x) dt[i] = st[i];
+        const uint4* st = reinterpret_cast<const uint4*>(f.HT + (size_t)k * kHLayer);
+        uint4* dt = reinterpret_cast<uint4*>(Wt);
+        for (int i = threadIdx.x; i < kHLayer / 8; i += blockDim.x) dt[i] = st[i];
     }
     const float* p = f.P + (size_t)k * kPLayer;
     for (int i = threadIdx.x; i < kFH; i += blockDim.x) s->b2[i] = p[kPB2 + i];
@@ -155,142 +185,208 @@ __device__ inline bf16x4_t cond_input(const f32x4_t u, uint32_t amask, int D, in
     return pack_bf(a);
 }
 
-// Layer 1 of the conditioner MLP: h1 = relu(W1 a) (bf16 fragments, output
-// tile mt = k-step mt of layer 2) and its ReLU mask (bit 4 mt + i:
-// pre-activation > 0).
-__device__ inline uint32_t layer1(const LayerLds* s, bf16x4_t a, int lane, bf16x4_t* h1) {
+// Layer 1 of the conditioner MLP for NT sample tiles: h1 = relu(W1 a) (bf16
+// fragments, output tile mt = k-step mt of layer 2); m1: tile 0's ReLU mask
+// (bit 4 mt + i: pre-activation > 0).
+template <int NT>
+__device__ inline uint32_t layer1(const LayerLds* s, const bf16x4_t (&a)[NT], int lane, bf16x4_t (&h1)[NT][8]) {
     const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    const float top = relu_top();
     uint32_t m1 = 0;
 #pragma unroll
     for (int mt = 0; mt < 8; ++mt) {
-        f32x4_t c = mfma16(frag_a(s->W + kHW1, kS1, mt, 0, lane), a, zero);
+        const bf16x4_t w = half8(frag_w(s->W + kHW1, mt / 2, lane), mt & 1);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            m1 |= (c[i] > 0.f ? 1u : 0u) << (4 * mt + i);
-            c[i] = fmaxf(c[i], 0.f);
+        for (int t = 0; t < NT; ++t) {
+            f32x4_t c = mfma16(w, a[t], zero);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (t == 0) m1 |= (c[i] > 0.f ? 1u : 0u) << (4 * mt + i);
+                c[i] = relu(c[i], top);
+            }
+            h1[t][mt] = pack_bf(c);
         }
-        h1[mt] = pack_bf(c);
     }
     return m1;
 }
 
-// The conditioner MLP of one tile: o[0] = raw s, o[1] = t rows (l/16)*4+i.
-// Optionally keeps h2 (bf16 fragments) and the ReLU masks of h1 and h2.
+// The conditioner MLP of NT tiles: o[t][0] = raw s, o[t][1] = t rows
+// (l/16)*4+i.  Each weight fragment read serves every tile.  Optionally keeps
+// (tile 0) h2 as bf16 fragments and the ReLU masks of h1 and h2.
 struct MlpKeep {
     bf16x4_t h2[8];
     uint32_t m1, m2;   // bit 4 mt + i: pre-activation > 0
 };
 
-template <bool KEEP>
-__device__ inline void mlp(const LayerLds* s, bf16x4_t a, int lane, f32x4_t* o, MlpKeep* keep) {
-    bf16x4_t h1[8];
+template <int NT, bool KEEP>
+__device__ inline void mlp(const LayerLds* s, const bf16x4_t (&a)[NT], int lane, f32x4_t (&o)[NT][2],
+                           MlpKeep* keep) {
+    // layer 2's output tiles accumulate MB at a time side by side
+    // (independent MFMA chains), k-step by k-step
+    constexpr int MB = NT == 1 ? 8 : 4;
+    bf16x4_t h1[NT][8], h2[NT][8];
+    const float top = relu_top();
     uint32_t m2 = 0;
-    const uint32_t m1 = layer1(s, a, lane, h1);
-    // h2: the eight output tiles accumulate side by side (independent MFMA
-    // chains), k-step by k-step
-    f32x4_t acc[8];
+    const uint32_t m1 = layer1<NT>(s, a, lane, h1);
 #pragma unroll
-    for (int mt = 0; mt < 8; ++mt)
+    for (int mb = 0; mb < 8; mb += MB) {
+        f32x4_t acc[NT][MB];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[mt][i] = s->b2[16 * mt + (lane >> 4) * 4 + i];
+        for (int m = 0; m < MB; ++m) {
+            const f32x4_t b = *reinterpret_cast<const f32x4_t*>(s->b2 + 16 * (mb + m) + (lane >> 4) * 4);
 #pragma unroll
-    for (int kt = 0; kt < 8; kt += 2) {
-        const bf16x8_t b = cat8(h1[kt], h1[kt + 1]);
-#pragma unroll
-        for (int mt = 0; mt < 8; ++mt) acc[mt] = mfma32(frag_a2(s->W + kHW2, kS2, mt, kt, lane), b, acc[mt]);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    bf16x4_t h2[8];
-#pragma unroll
-    for (int mt = 0; mt < 8; ++mt) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            m2 |= (acc[mt][i] > 0.f ? 1u : 0u) << (4 * mt + i);
-            acc[mt][i] = fmaxf(acc[mt][i], 0.f);
+            for (int t = 0; t < NT; ++t) acc[t][m] = b;
         }
-        h2[mt] = pack_bf(acc[mt]);
-    }
-    f32x4_t o0, o1;
+        // a wave in its products goes first: the SIMD's waves, together after
+        // the barrier, drift apart and their vector work fills the matrix
+        // cores' gaps
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        o0[i] = s->b3[(lane >> 4) * 4 + i];
-        o1[i] = s->b3[16 + (lane >> 4) * 4 + i];
+        for (int kp = 0; kp < 4; ++kp) {
+#pragma unroll
+            for (int m = 0; m < MB; ++m) {
+                const bf16x8_t w = frag_w(s->W + kHW2, (mb + m) * 4 + kp, lane);
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                    acc[t][m] = mfma32(w, cat8(h1[t][2 * kp], h1[t][2 * kp + 1]), acc[t][m]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (t == 0) m2 |= (acc[t][m][i] > 0.f ? 1u : 0u) << (4 * (mb + m) + i);
+                    acc[t][m][i] = relu(acc[t][m][i], top);
+                }
+                h2[t][mb + m] = pack_bf(acc[t][m]);
+            }
     }
 #pragma unroll
-    for (int kt = 0; kt < 8; kt += 2) {
-        const bf16x8_t b = cat8(h2[kt], h2[kt + 1]);
-        o0 = mfma32(frag_a2(s->W + kHW3, kS3, 0, kt, lane), b, o0);
-        o1 = mfma32(frag_a2(s->W + kHW3, kS3, 1, kt, lane), b, o1);
+    for (int q = 0; q < 2; ++q) {
+        const f32x4_t b = *reinterpret_cast<const f32x4_t*>(s->b3 + 16 * q + (lane >> 4) * 4);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) o[t][q] = b;
     }
-    o[0] = o0;
-    o[1] = o1;
+#pragma unroll
+    for (int kp = 0; kp < 4; ++kp)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const bf16x8_t w = frag_w(s->W + kHW3, q * 4 + kp, lane);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) o[t][q] = mfma32(w, cat8(h2[t][2 * kp], h2[t][2 * kp + 1]), o[t][q]);
+        }
     if (KEEP) {
 #pragma unroll
-        for (int q = 0; q < 8; ++q) keep->h2[q] = h2[q];
+        for (int q = 0; q < 8; ++q) keep->h2[q] = h2[0][q];
         keep->m1 = m1;
         keep->m2 = m2;
     }
 }
 
 // ------------------------------------------------------------- sampling ----
-constexpr int kFlowThreads = 1024;
-constexpr int kFlowTiles = 4;        // sample tiles (16 samples) per wave per pass
+constexpr int kFlowThreads = 768;
+constexpr int kFlowTiles = 6;        // sample tiles (16 samples) per wave per pass
+constexpr int kFlowNT = 2;           // of which the MLP takes this many at once
 constexpr int kFlowWaves = kFlowThreads / 64;
-constexpr int kFlowPass = kFlowWaves * kFlowTiles * 16;  // samples per workgroup pass
+
 
 struct FlowFcn {
     int kind;            // VGX_FCN_GAUSSMIX or VGX_FCN_DIAGRIDGE
     int ncomp;
-    const float* A;
-    const float* B;
-    const float* c;      // GAUSSMIX: [ncomp][D]; DIAGRIDGE: [ncomp]
+    const double* A;
+    const double* B;
+    const double* c;     // GAUSSMIX: [ncomp][D]; DIAGRIDGE: [ncomp]
 };
+
+// The parameters A | B | c as FP32 in LDS.
+__device__ inline void load_fcn(const FlowFcn& F, int D, float* Lc) {
+    const int ncp = F.kind == VGX_FCN_DIAGRIDGE ? 3 * F.ncomp : F.ncomp * (2 + D);
+    for (int i = threadIdx.x; i < ncp; i += blockDim.x)
+        Lc[i] = (float)(i < F.ncomp ? F.A[i] : i < 2 * F.ncomp ? F.B[i - F.ncomp] : F.c[i - 2 * F.ncomp]);
+}
 
 struct SampleArgs {
     uint64_t n;          // samples
     uint64_t base;       // first sample index (Philox counter)
     uint32_t seed_lo, seed_hi, iteration;
+    int tiles;           // sample tiles per wave and pass (even, up to kFlowTiles)
     double* part;        // [gridDim.x][4]: DD sum f J, DD sum (f J)^2
     float* xout;         // optional [n][16] x, and fout [n] = f J
     float* fout;
     int32_t* status;
 };
 
-// f at x for the sample of this lane (dims (l/16)*4 + i), all four lanes of
-// the sample cooperating; every lane of the sample returns f.
-__device__ inline float flow_fcn(const FlowFcn& F, const float* Lc, f32x4_t x, int D, int lane) {
+// f at x of NT samples of this lane (dims (l/16)*4 + i), all four lanes of a
+// sample cooperating; every lane of the sample returns f.  One LDS read of
+// the parameters serves the NT samples.
+template <int NT>
+__device__ inline void flow_fcn(const FlowFcn& F, const float* Lc, const f32x4_t (&x)[NT], int D, int lane,
+                                float (&fv)[NT]) {
     const int g = lane >> 4;
-    float acc = 0.f;
+    float acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = 0.f;
     if (F.kind == VGX_FCN_DIAGRIDGE) {
-        float s1 = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (4 * g + i < D) s1 += x[i];
-        const float xbar = group_sum(s1) / (float)D;
-        float p = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (4 * g + i < D) p += (x[i] - xbar) * (x[i] - xbar);
-        const float P = group_sum(p);
         const float fd = (float)D;
-        for (int k = g; k < F.ncomp; k += 4) {
-            const float t = xbar - Lc[2 * F.ncomp + k];
-            acc = __builtin_fmaf(Lc[k], __expf(-Lc[F.ncomp + k] * __builtin_fmaf(fd * t, t, P)), acc);
+        float xbar[NT], P[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            float s1 = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (4 * g + i < D) s1 += x[t][i];
+            xbar[t] = group_sum(s1) / fd;
+            float p = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (4 * g + i < D) p += (x[t][i] - xbar[t]) * (x[t][i] - xbar[t]);
+            P[t] = group_sum(p);
         }
-        return group_sum(acc);
+        const float* A = Lc + g;
+        const float* B = A + F.ncomp;
+        const float* C = B + F.ncomp;
+        auto term = [&](int k) {
+            const float Ak = A[k], Bk = B[k], Ck = C[k];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const float dt = xbar[t] - Ck;
+                acc[t] = __builtin_fmaf(Ak, __expf(-Bk * __builtin_fmaf(fd * dt, dt, P[t])), acc[t]);
+            }
+        };
+        // four terms a step: their reads share the addresses and one wait
+        // (a term a step spent more on addresses and waits than on the term)
+        int k = 0;
+        for (; k + 16 <= F.ncomp; k += 16) {
+            term(k);
+            term(k + 4);
+            term(k + 8);
+            term(k + 12);
+        }
+        for (; k + g < F.ncomp; k += 4) term(k);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) fv[t] = group_sum(acc[t]);
+        return;
     }
     for (int k = 0; k < F.ncomp; ++k) {
-        float r = 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (4 * g + i < D) {
-                const float t = x[i] - Lc[2 * F.ncomp + k * D + 4 * g + i];
-                r = __builtin_fmaf(t, t, r);
-            }
-        r = group_sum(r);
-        acc = __builtin_fmaf(Lc[k], __expf(-Lc[F.ncomp + k] * r), acc);
+        for (int t = 0; t < NT; ++t) {
+            float r = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (4 * g + i < D) {
+                    const float dt = x[t][i] - Lc[2 * F.ncomp + k * D + 4 * g + i];
+                    r = __builtin_fmaf(dt, dt, r);
+                }
+            r = group_sum(r);
+            acc[t] = __builtin_fmaf(Lc[k], __expf(-Lc[F.ncomp + k] * r), acc[t]);
+        }
     }
-    return acc;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) fv[t] = acc[t];
 }
 
 // Per-wave tile state in LDS (kFlowTiles tiles: u as float4 per lane, and
@@ -299,24 +395,65 @@ struct TileState {
     f32x4_t u[kFlowTiles][64];
     float l[kFlowTiles][64];
 };
+constexpr size_t kLdsLayer = (sizeof(LayerLds) + 15) & ~(size_t)15;
 constexpr size_t kStateLds = kFlowWaves * sizeof(TileState);
+// What they leave of a CU's LDS for an integrand's parameters (1 KiB: the sums).
+constexpr size_t kFlowFcnLds = 160 * 1024 - 1024 - kLdsLayer - kStateLds;
+static_assert(160 * 1024 - 1024 - kLdsLayer - 8 * sizeof(TileState) >= 48 * 1024, "8 waves fit any mixture");
 
+// A workgroup's waves and tiles of 16 samples per wave and pass: the smallest
+// of these shapes whose workgroups, one per CU, cover the n samples in one
+// pass; the last is full.  (At the full shape alone 20,000 samples would keep
+// 18 of the CUs busy: a sample call of 2000 to 20,000 took 258-276 us, now
+// 110-130, the copies above included.)
+struct FlowShape {
+    int waves, tiles, blocks;
+};
+static FlowShape flow_shape(int64_t n, int cus, int full_blocks, size_t fcn_lds) {
+    static const int shapes[4][2] = {{4, 2}, {8, 2}, {12, 2}, {kFlowWaves, kFlowTiles}};
+    const int64_t nt = (n + 15) / 16;
+    for (const auto& s : shapes) {
+        const int64_t blocks = (nt + s[0] * s[1] - 1) / (s[0] * s[1]);
+        if (blocks <= cus && (s[0] <= 8 || fcn_lds <= kFlowFcnLds)) return {s[0], s[1], (int)blocks};
+    }
+    // (a long mixture leaves no LDS for the state of all the waves' tiles)
+    const int waves = fcn_lds <= kFlowFcnLds ? kFlowWaves : 8;
+    const int64_t blocks = (nt + waves * kFlowTiles - 1) / (waves * kFlowTiles);
+    return {waves, kFlowTiles, (int)std::min<int64_t>(full_blocks, blocks)};
+}
+
+
+// A call, or its constants would take registers from the layers' loop.
+__device__ __noinline__ double exp_jac(double x) { return exp(x); }
+
+// Bound by vector instructions (relu, conversions, the couplings' tanh and
+// exp, the integrand) with the matrix cores 40-50 % busy.  4e6 samples, 9
+// axes, 6 layers, 500 components: 2450 us with row-major weights and a tile
+// at a time, 2480 -> 2175 with one-instruction relu and four ridge terms a
+// step, 1940 with the products' priority and the couplings' short quotient,
+// 1570 a call with the parameters read in place (before: three copies to the
+// host and one back, each waited for).  12 waves hold all of a layer in
+// registers; with 16 the kernels spill 35 and are no faster, with 8 and four
+// tiles at once 2012 where 12 took 1945.
 __global__ __launch_bounds__(kFlowThreads) void flow_sample_kernel(FlowArgs f, FlowFcn F, SampleArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     LayerLds* L = reinterpret_cast<LayerLds*>(smem);
-    TileState* TS = reinterpret_cast<TileState*>(smem + ((sizeof(LayerLds) + 15) & ~(size_t)15)) +
+    TileState* TS = reinterpret_cast<TileState*>(smem + kLdsLayer) +
                     (threadIdx.x >> 6);
-    float* Lc = reinterpret_cast<float*>(smem + ((sizeof(LayerLds) + 15) & ~(size_t)15) + kStateLds);
+    float* Lc = reinterpret_cast<float*>(smem + kLdsLayer +
+                                         (blockDim.x >> 6) * sizeof(TileState));
     __shared__ double red[kFlowWaves * 4];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4;
-    const int ncp = F.kind == VGX_FCN_DIAGRIDGE ? 3 * F.ncomp : F.ncomp * (2 + f.D);
-    for (int i = threadIdx.x; i < ncp; i += blockDim.x)
-        Lc[i] = i < F.ncomp ? F.A[i] : i < 2 * F.ncomp ? F.B[i - F.ncomp] : F.c[i - 2 * F.ncomp];
+    const int wave = threadIdx.x >> 6;
+    int lane = threadIdx.x & 63;
+    load_fcn(F, f.D, Lc);
     DD s1{0, 0}, s2{0, 0};
-    for (uint64_t pb = (uint64_t)blockIdx.x * kFlowPass; pb < a.n; pb += (uint64_t)gridDim.x * kFlowPass) {
+    const uint64_t pass = (blockDim.x >> 6) * a.tiles * 16;  // samples per pass of the workgroup
+    for (uint64_t pb = blockIdx.x * pass; pb < a.n; pb += gridDim.x * pass) {
+        asm volatile("" : "+v"(lane));  // addresses are formed when used, not held over the passes
+        const int g = lane >> 4;
 #pragma unroll 1
-        for (int q = 0; q < kFlowTiles; ++q) {
-            const uint64_t sidx = a.base + pb + (uint64_t)(wave * kFlowTiles + q) * 16 + (lane & 15);
+        for (int q = 0; q < a.tiles; ++q) {
+            const uint64_t sidx = a.base + pb + (uint64_t)(wave * a.tiles + q) * 16 + (lane & 15);
             const U4 w = philox4x32_10_dev(U4{(uint32_t)sidx, (uint32_t)(sidx >> 32), a.iteration, (uint32_t)g},
                                        a.seed_lo, a.seed_hi);
             const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
@@ -325,61 +462,84 @@ __global__ __launch_bounds__(kFlowThreads) void flow_sample_kernel(FlowArgs f, F
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float z = (float)(ws[i] >> 8) * (1.0f / 16777216.0f) + (1.0f / 33554432.0f);
-                const float uu = __logf(z) - __logf(1.0f - z);
-                uq[i] = uu;
-                if (4 * g + i < f.D) l -= logsigp(uu);
+                const float l0 = __logf(z), l1 = __logf(1.0f - z);
+                uq[i] = l0 - l1;
+                if (4 * g + i < f.D) l -= l0 + l1;  // dz/du = z (1 - z)
             }
             TS->u[q][lane] = uq;
             TS->l[q][lane] = l;
         }
         for (int k = 0; k < f.L; ++k) {
+            asm volatile("" : "+v"(lane));
+            const int g = lane >> 4;
             __syncthreads();
             load_layer(f, k, L, false, nullptr);
             __syncthreads();
             const uint32_t am = f.amask[k];
 #pragma unroll 1
-            for (int q = 0; q < kFlowTiles; ++q) {
-                f32x4_t uq = TS->u[q][lane];
-                float l = TS->l[q][lane];
-                f32x4_t o[2];
-                mlp<false>(L, cond_input(uq, am, f.D, lane), lane, o, nullptr);
+            for (int q = 0; q < a.tiles; q += kFlowNT) {
+                bf16x4_t a[kFlowNT];
+                f32x4_t o[kFlowNT][2];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int d = 4 * g + i;
-                    if (d < f.D && !((am >> d) & 1u)) {
-                        const float sv = kSMax * tanh_f(o[0][i] / kSMax);
-                        uq[i] = uq[i] * __expf(sv) + o[1][i];
-                        l += sv;
+                for (int t = 0; t < kFlowNT; ++t) a[t] = cond_input(TS->u[q + t][lane], am, f.D, lane);
+                mlp<kFlowNT, false>(L, a, lane, o, nullptr);
+#pragma unroll
+                for (int t = 0; t < kFlowNT; ++t) {
+                    f32x4_t uq = TS->u[q + t][lane];
+                    float l = TS->l[q + t][lane];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int d = 4 * g + i;
+                        if (d < f.D && !((am >> d) & 1u)) {
+                            const float sv = kSMax * tanh_s(o[t][0][i]);
+                            uq[i] = uq[i] * __expf(sv) + o[t][1][i];
+                            l += sv;
+                        }
                     }
+                    TS->u[q + t][lane] = uq;
+                    TS->l[q + t][lane] = l;
                 }
-                TS->u[q][lane] = uq;
-                TS->l[q][lane] = l;
             }
         }
 #pragma unroll 1
-        for (int q = 0; q < kFlowTiles; ++q) {
-            const f32x4_t uq = TS->u[q][lane];
-            f32x4_t x;
-            float l = TS->l[q][lane];
+        for (int q = 0; q < a.tiles; q += kFlowNT) {
+            f32x4_t x[kFlowNT];
+            float LJ[kFlowNT], fv[kFlowNT];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                x[i] = 1.0f / (1.0f + __expf(-uq[i]));
-                if (4 * g + i < f.D) l += logsigp(uq[i]);
+            for (int t = 0; t < kFlowNT; ++t) {
+                const f32x4_t uq = TS->u[q + t][lane];
+                float l = TS->l[q + t][lane];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    x[t][i] = 1.0f / (1.0f + __expf(-uq[i]));
+                    if (4 * g + i < f.D) l += logsigp(uq[i]);
+                }
+                LJ[t] = group_sum(l);
             }
-            const float LJ = group_sum(l);
-            const float fv = flow_fcn(F, Lc, x, f.D, lane);
-            const uint64_t sl = pb + (uint64_t)(wave * kFlowTiles + q) * 16 + (lane & 15);
-            const bool live = sl < a.n;
-            // f = 0 where the map stretches enough for J to overflow is 0
-            const double fj = (live && fv != 0.f) ? (double)fv * exp((double)LJ) : 0.0;
-            if (fv != fv && live && a.status) atomicOr(a.status, (int32_t)VGX_ENAN);
-            if (g == 0 && live) {
+            flow_fcn<kFlowNT>(F, Lc, x, f.D, lane, fv);
+#pragma unroll
+            for (int t = 0; t < kFlowNT; ++t) {
+                const uint64_t sl = pb + (uint64_t)(wave * a.tiles + q + t) * 16 + (lane & 15);
+                const bool live = sl < a.n;
+                if (fv[t] != fv[t] && live && a.status) atomicOr(a.status, (int32_t)VGX_ENAN);
+                if (a.xout && live) *reinterpret_cast<f32x4_t*>(a.xout + sl * 16 + 4 * g) = x[t];
+                if (g == 0) {
+                    TS->l[q + t][lane] = fv[t];
+                    TS->l[q + t][16 + lane] = LJ[t];
+                }
+            }
+        }
+        // the sums, a sample per lane
+        for (int r = 0; r < a.tiles; r += 4) {
+            const int q = r + (lane >> 4);
+            const uint64_t sl = pb + (uint64_t)(wave * a.tiles + q) * 16 + (lane & 15);
+            if (q < a.tiles && sl < a.n) {
+                const float fl = TS->l[q][lane & 15], lj = TS->l[q][16 + (lane & 15)];
+                // f = 0 where the map stretches enough for J to overflow is 0
+                const double fj = fl != 0.f ? (double)fl * exp_jac((double)lj) : 0.0;
                 dd_add(s1, fj);
                 dd_add(s2, fj * fj);
-            }
-            if (a.xout && live) {
-                *reinterpret_cast<f32x4_t*>(a.xout + sl * 16 + 4 * g) = x;
-                if (g == 0) a.fout[sl] = (float)fj;
+                if (a.xout) a.fout[sl] = (float)fj;
             }
         }
     }
@@ -394,7 +554,7 @@ __global__ __launch_bounds__(kFlowThreads) void flow_sample_kernel(FlowArgs f, F
     __syncthreads();
     if (threadIdx.x == 0) {
         DD t1{0, 0}, t2{0, 0};
-        for (int w = 0; w < kFlowWaves; ++w) {
+        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
             t1 = dd_sum(t1, DD{red[4 * w], red[4 * w + 1]});
             t2 = dd_sum(t2, DD{red[4 * w + 2], red[4 * w + 3]});
         }
@@ -407,19 +567,18 @@ __global__ __launch_bounds__(kFlowThreads) void flow_sample_kernel(FlowArgs f, F
 __global__ __launch_bounds__(256) void flow_eval_kernel(FlowFcn F, int D, const float* x, uint64_t n, float* fout) {
     extern __shared__ __align__(16) unsigned char smem[];
     float* Lc = reinterpret_cast<float*>(smem);
-    const int ncp = F.kind == VGX_FCN_DIAGRIDGE ? 3 * F.ncomp : F.ncomp * (2 + D);
-    for (int i = threadIdx.x; i < ncp; i += blockDim.x)
-        Lc[i] = i < F.ncomp ? F.A[i] : i < 2 * F.ncomp ? F.B[i - F.ncomp] : F.c[i - 2 * F.ncomp];
+    load_fcn(F, D, Lc);
     __syncthreads();
     const int lane = threadIdx.x & 63, g = lane >> 4;
     const uint64_t ntiles = (n + 15) / 16;
     for (uint64_t t = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); t < ntiles;
          t += (uint64_t)gridDim.x * (blockDim.x >> 6)) {
         const uint64_t sl = t * 16 + (lane & 15);
-        f32x4_t xv = {0.5f, 0.5f, 0.5f, 0.5f};
-        if (sl < n) xv = *reinterpret_cast<const f32x4_t*>(x + sl * 16 + 4 * g);
-        const float fv = flow_fcn(F, Lc, xv, D, lane);
-        if (g == 0 && sl < n) fout[sl] = fv;
+        f32x4_t xv[1] = {{0.5f, 0.5f, 0.5f, 0.5f}};
+        if (sl < n) xv[0] = *reinterpret_cast<const f32x4_t*>(x + sl * 16 + 4 * g);
+        float fv[1];
+        flow_fcn<1>(F, Lc, xv, D, lane, fv);
+        if (g == 0 && sl < n) fout[sl] = fv[0];
     }
 }
 
@@ -430,18 +589,23 @@ struct InvArgs {
     float* saved;        // [L][n][16]: input of each layer
     float* u0;           // [n][16]
     float* logq;         // [n]
+    int tiles;           // sample tiles per wave and pass (even, up to kFlowTiles)
 };
 
 __global__ __launch_bounds__(kFlowThreads) void flow_inverse_kernel(FlowArgs f, InvArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     LayerLds* L = reinterpret_cast<LayerLds*>(smem);
-    TileState* TS = reinterpret_cast<TileState*>(smem + ((sizeof(LayerLds) + 15) & ~(size_t)15)) +
+    TileState* TS = reinterpret_cast<TileState*>(smem + kLdsLayer) +
                     (threadIdx.x >> 6);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4;
-    for (uint64_t pb = (uint64_t)blockIdx.x * kFlowPass; pb < a.n; pb += (uint64_t)gridDim.x * kFlowPass) {
+    const int wave = threadIdx.x >> 6;
+    int lane = threadIdx.x & 63;
+    const uint64_t pass = (blockDim.x >> 6) * a.tiles * 16;  // samples per pass of the workgroup
+    for (uint64_t pb = blockIdx.x * pass; pb < a.n; pb += gridDim.x * pass) {
+        asm volatile("" : "+v"(lane));  // addresses are formed when used, not held over the passes
+        const int g = lane >> 4;
 #pragma unroll 1
-        for (int q = 0; q < kFlowTiles; ++q) {
-            const uint64_t sl = pb + (uint64_t)(wave * kFlowTiles + q) * 16 + (lane & 15);
+        for (int q = 0; q < a.tiles; ++q) {
+            const uint64_t sl = pb + (uint64_t)(wave * a.tiles + q) * 16 + (lane & 15);
             f32x4_t xv = {0.5f, 0.5f, 0.5f, 0.5f};
             if (sl < a.n) xv = *reinterpret_cast<const f32x4_t*>(a.x + sl * 16 + 4 * g);
             float l = 0.f;
@@ -449,42 +613,53 @@ __global__ __launch_bounds__(kFlowThreads) void flow_inverse_kernel(FlowArgs f, 
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float xc = fminf(fmaxf(xv[i], 1e-7f), 1.0f - 1e-7f);
-                const float uu = __logf(xc) - __logf(1.0f - xc);
-                uq[i] = (4 * g + i < f.D) ? uu : 0.f;
-                if (4 * g + i < f.D) l -= logsigp(uu);
+                const float l0 = __logf(xc), l1 = __logf(1.0f - xc);
+                uq[i] = (4 * g + i < f.D) ? l0 - l1 : 0.f;
+                if (4 * g + i < f.D) l -= l0 + l1;
             }
             TS->u[q][lane] = uq;
             TS->l[q][lane] = l;
         }
         for (int k = f.L - 1; k >= 0; --k) {
+            asm volatile("" : "+v"(lane));
+            const int g = lane >> 4;
             __syncthreads();
             load_layer(f, k, L, false, nullptr);
             __syncthreads();
             const uint32_t am = f.amask[k];
 #pragma unroll 1
-            for (int q = 0; q < kFlowTiles; ++q) {
-                const uint64_t sl = pb + (uint64_t)(wave * kFlowTiles + q) * 16 + (lane & 15);
-                f32x4_t uq = TS->u[q][lane];
-                float l = TS->l[q][lane];
-                if (sl < a.n) *reinterpret_cast<f32x4_t*>(a.saved + ((size_t)k * a.n + sl) * 16 + 4 * g) = uq;
-                f32x4_t o[2];
-                mlp<false>(L, cond_input(uq, am, f.D, lane), lane, o, nullptr);
+            for (int q = 0; q < a.tiles; q += kFlowNT) {
+                bf16x4_t ain[kFlowNT];
+                f32x4_t o[kFlowNT][2];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int d = 4 * g + i;
-                    if (d < f.D && !((am >> d) & 1u)) {
-                        const float sv = kSMax * tanh_f(o[0][i] / kSMax);
-                        uq[i] = (uq[i] - o[1][i]) * __expf(-sv);
-                        l -= sv;
-                    }
+                for (int t = 0; t < kFlowNT; ++t) {
+                    const uint64_t sl = pb + (uint64_t)(wave * a.tiles + q + t) * 16 + (lane & 15);
+                    const f32x4_t uq = TS->u[q + t][lane];
+                    if (sl < a.n) *reinterpret_cast<f32x4_t*>(a.saved + ((size_t)k * a.n + sl) * 16 + 4 * g) = uq;
+                    ain[t] = cond_input(uq, am, f.D, lane);
                 }
-                TS->u[q][lane] = uq;
-                TS->l[q][lane] = l;
+                mlp<kFlowNT, false>(L, ain, lane, o, nullptr);
+#pragma unroll
+                for (int t = 0; t < kFlowNT; ++t) {
+                    f32x4_t uq = TS->u[q + t][lane];
+                    float l = TS->l[q + t][lane];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int d = 4 * g + i;
+                        if (d < f.D && !((am >> d) & 1u)) {
+                            const float sv = kSMax * tanh_s(o[t][0][i]);
+                            uq[i] = (uq[i] - o[t][1][i]) * __expf(-sv);
+                            l -= sv;
+                        }
+                    }
+                    TS->u[q + t][lane] = uq;
+                    TS->l[q + t][lane] = l;
+                }
             }
         }
 #pragma unroll 1
-        for (int q = 0; q < kFlowTiles; ++q) {
-            const uint64_t sl = pb + (uint64_t)(wave * kFlowTiles + q) * 16 + (lane & 15);
+        for (int q = 0; q < a.tiles; ++q) {
+            const uint64_t sl = pb + (uint64_t)(wave * a.tiles + q) * 16 + (lane & 15);
             const f32x4_t uq = TS->u[q][lane];
             float l = TS->l[q][lane];
 #pragma unroll
@@ -651,7 +826,6 @@ __device__ inline bf16x8_t frag_pair(const uint16_t* S, int j, int row0, int lan
     return cat8(frag_op(s0, row0, lane), frag_op(s0 + kSlot, row0, lane));
 }
 
-constexpr size_t kLdsLayer = (sizeof(LayerLds) + 15) & ~(size_t)15;
 constexpr size_t kLdsBwd = kLdsLayer + sizeof(uint16_t) * kHLayer + sizeof(uint16_t) * (size_t)kBwdWaves * kSlot;
 static_assert(kLdsBwd <= 160 * 1024, "backward LDS plan fits a CU");
 
@@ -714,9 +888,11 @@ __global__ __launch_bounds__(kBwdThreads) void flow_backward_kernel(FlowArgs f, 
                 G[i] = (live && 4 * g + i < f.D) ? -cw * (1.0f - 2.0f / (1.0f + __expf(-graw[i]))) : 0.f;
         }
         const bf16x4_t ain = cond_input(uin, am, f.D, lane);
-        f32x4_t o[2];
+        const bf16x4_t a1[1] = {ain};
+        f32x4_t o1[1][2];
         MlpKeep kp;
-        mlp<true>(L, ain, lane, o, &kp);
+        mlp<1, true>(L, a1, lane, o1, &kp);
+        const f32x4_t (&o)[2] = o1[0];
         // coupling backward (inverse direction)
         f32x4_t dout0, dout1, Gin;
 #pragma unroll
@@ -726,7 +902,7 @@ __global__ __launch_bounds__(kBwdThreads) void flow_backward_kernel(FlowArgs f, 
             dout1[i] = 0.f;
             Gin[i] = G[i];
             if (d < f.D && !((am >> d) & 1u)) {
-                const float th = tanh_f(o[0][i] / kSMax);
+                const float th = tanh_s(o[0][i]);
                 const float sv = kSMax * th;
                 const float es = __expf(-sv);
                 const float uout = (uin[i] - o[1][i]) * es;
@@ -765,7 +941,7 @@ __global__ __launch_bounds__(kBwdThreads) void flow_backward_kernel(FlowArgs f, 
         bf16x4_t dh2[8];
 #pragma unroll
         for (int mt = 0; mt < 8; ++mt) {
-            f32x4_t cc = mfma32(frag_a2(Wt + kTW3, kT3, mt, 0, lane), cat8(do0, do1), zero);
+            f32x4_t cc = mfma32(frag_w(Wt + kTW3, mt, lane), cat8(do0, do1), zero);
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 if (!((kp.m2 >> (4 * mt + i)) & 1u)) cc[i] = 0.f;
@@ -775,10 +951,10 @@ __global__ __launch_bounds__(kBwdThreads) void flow_backward_kernel(FlowArgs f, 
 #pragma unroll
         for (int mt = 0; mt < 8; ++mt) acc[mt] = zero;
 #pragma unroll
-        for (int kt = 0; kt < 8; kt += 2) {
-            const bf16x8_t b = cat8(dh2[kt], dh2[kt + 1]);
+        for (int kp2 = 0; kp2 < 4; ++kp2) {
+            const bf16x8_t b = cat8(dh2[2 * kp2], dh2[2 * kp2 + 1]);
 #pragma unroll
-            for (int mt = 0; mt < 8; ++mt) acc[mt] = mfma32(frag_a2(Wt + kTW2, kT2, mt, kt, lane), b, acc[mt]);
+            for (int mt = 0; mt < 8; ++mt) acc[mt] = mfma32(frag_w(Wt + kTW2, mt * 4 + kp2, lane), b, acc[mt]);
             __builtin_amdgcn_sched_barrier(0);
         }
         bf16x4_t dh1[8];
@@ -791,7 +967,7 @@ __global__ __launch_bounds__(kBwdThreads) void flow_backward_kernel(FlowArgs f, 
         }
         f32x4_t da = zero;
 #pragma unroll
-        for (int kt = 0; kt < 8; kt += 2) da = mfma32(frag_a2(Wt + kTW1, kT1, 0, kt, lane), cat8(dh1[kt], dh1[kt + 1]), da);
+        for (int kt = 0; kt < 8; kt += 2) da = mfma32(frag_w(Wt + kTW1, kt / 2, lane), cat8(dh1[kt], dh1[kt + 1]), da);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int d = 4 * g + i;
@@ -801,12 +977,12 @@ __global__ __launch_bounds__(kBwdThreads) void flow_backward_kernel(FlowArgs f, 
         __syncthreads();
         // ---- phase 2: dh2 | h1 -> dW2, b2
         {
-            bf16x4_t h1[8];
-            layer1(L, ain, lane, h1);
+            bf16x4_t h1[1][8];
+            layer1<1>(L, a1, lane, h1);
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
                 stage(my, 16 * q, dh2[q], ln);
-                stage(my, kFH + 16 * q, h1[q], ln);
+                stage(my, kFH + 16 * q, h1[0][q], ln);
             }
         }
         __syncthreads();
@@ -914,8 +1090,8 @@ __global__ void flow_adam_kernel(AdamArgs a) {
     }
 }
 
-// bf16 copies (and transposes) of the weights after an update, in the
-// padded layouts.
+// bf16 copies (and transposes) of the weights after an update, in fragment
+// order.
 __global__ void flow_cast_kernel(const float* P, uint16_t* H, uint16_t* HT, int L) {
     constexpr int nlog = kFH * kFI + kFH * kFH + kFO * kFH;
     const int total = L * nlog;
@@ -927,18 +1103,18 @@ __global__ void flow_cast_kernel(const float* P, uint16_t* H, uint16_t* HT, int 
         if (r < kFH * kFI) {                 // W1 [128][16] -> W1t [16][128]
             const int o = r / kFI, c = r % kFI;
             v = p[kPW1 + r];
-            rh = kHW1 + o * kS1 + c;
-            rt = kTW1 + c * kT1 + o;
+            rh = kHW1 + frag_pos1(o, c);
+            rt = kTW1 + frag_pos(c, o, 4);
         } else if (r < kFH * kFI + kFH * kFH) {  // W2 [128][128]
             const int q = r - kFH * kFI, o = q / kFH, c = q % kFH;
             v = p[kPW2 + q];
-            rh = kHW2 + o * kS2 + c;
-            rt = kTW2 + c * kT2 + o;
+            rh = kHW2 + frag_pos(o, c, 4);
+            rt = kTW2 + frag_pos(c, o, 4);
         } else {                             // W3 [32][128] -> W3t [128][32]
             const int q = r - kFH * kFI - kFH * kFH, o = q / kFH, c = q % kFH;
             v = p[kPW3 + q];
-            rh = kHW3 + o * kS3 + c;
-            rt = kTW3 + c * kT3 + o;
+            rh = kHW3 + frag_pos(o, c, 4);
+            rt = kTW3 + frag_pos(c, o, 1);
         }
         const uint16_t h = f2bf(v);
         H[(size_t)k * kHLayer + rh] = h;
@@ -980,7 +1156,7 @@ struct vgx_flow {
     uint16_t* H = nullptr;
     uint16_t* HT = nullptr;
     // per-batch scratch (grown on demand)
-    Scratch saved, u0, logq, c, G, wpart, cpart, spart, misc, fpar;
+    Scratch saved, u0, logq, c, G, wpart, cpart, spart, misc;
     int step = 0;
 };
 
@@ -1043,7 +1219,7 @@ extern "C" int vgx_flow_destroy(vgx_flow* fl) {
     for (void* p : ps)
         if (p) (void)hipFree(p);
     Scratch* ss[] = {&fl->saved, &fl->u0, &fl->logq, &fl->c, &fl->G, &fl->wpart, &fl->cpart, &fl->spart,
-                     &fl->misc, &fl->fpar};
+                     &fl->misc};
     for (Scratch* q : ss) q->release();
     delete fl;
     return VGX_OK;
@@ -1079,31 +1255,16 @@ extern "C" int vgx_flow_get_params(const vgx_flow* fl, float* host, float* grad_
     return VGX_OK;
 }
 
-// Device integrand parameters converted to FP32 into fl->fpar.
-static int flow_fcn_params(vgx_flow* fl, const vgx_integrand* fcn, FlowFcn* F, hipStream_t s) {
+// The integrand as the kernels read it (its arrays stay the caller's), and
+// its LDS bytes.
+static int flow_fcn_params(const vgx_flow* fl, const vgx_integrand* fcn, FlowFcn* F, size_t* lds) {
     if (!fcn || (fcn->kind != VGX_FCN_GAUSSMIX && fcn->kind != VGX_FCN_DIAGRIDGE) || fcn->ncomp < 1)
         return VGX_EINVAL;
-    const int nc = fcn->ncomp;
-    const int ncc = fcn->kind == VGX_FCN_GAUSSMIX ? nc * fl->D : nc;
-    const size_t tot = (size_t)2 * nc + ncc;
-    if (tot * 4 > 48 * 1024) return VGX_ERANGE;  // staged in LDS with the layer
-    int rc = fl->fpar.ensure(tot * 4);
-    if (rc) return rc;
-    float* d = (float*)fl->fpar.ptr;
-    std::vector<double> h(tot);
-    VGX_HIP(hipMemcpyAsync(h.data(), fcn->A, nc * 8, hipMemcpyDeviceToHost, s));
-    VGX_HIP(hipMemcpyAsync(h.data() + nc, fcn->B, nc * 8, hipMemcpyDeviceToHost, s));
-    VGX_HIP(hipMemcpyAsync(h.data() + 2 * nc, fcn->c, ncc * 8, hipMemcpyDeviceToHost, s));
-    VGX_HIP(hipStreamSynchronize(s));
-    std::vector<float> hf(tot);
-    for (size_t i = 0; i < tot; ++i) hf[i] = (float)h[i];
-    VGX_HIP(hipMemcpyAsync(d, hf.data(), tot * 4, hipMemcpyHostToDevice, s));
-    VGX_HIP(hipStreamSynchronize(s));
-    F->kind = fcn->kind;
-    F->ncomp = nc;
-    F->A = d;
-    F->B = d + nc;
-    F->c = d + 2 * nc;
+    if (!fcn->A || !fcn->B || !fcn->c) return VGX_EINVAL;
+    const size_t nc = (size_t)fcn->ncomp;
+    *lds = (2 * nc + (fcn->kind == VGX_FCN_GAUSSMIX ? nc * fl->D : nc)) * 4;
+    if (*lds > 48 * 1024) return VGX_ERANGE;  // staged in LDS with the layer
+    *F = FlowFcn{fcn->kind, fcn->ncomp, fcn->A, fcn->B, fcn->c};
     return VGX_OK;
 }
 
@@ -1113,11 +1274,13 @@ extern "C" int vgx_flow_sample(vgx_flow* fl, const vgx_integrand* fcn, int64_t n
     if (!fl || n < 1 || (!sums && (!xout || !fout))) return VGX_EINVAL;
     hipStream_t s = (hipStream_t)stream;
     FlowFcn F{};
-    int rc = flow_fcn_params(fl, fcn, &F, s);
+    size_t fcn_lds;
+    int rc = flow_fcn_params(fl, fcn, &F, &fcn_lds);
     if (rc) return rc;
     DeviceInfo info;
     if ((rc = device_info(&info))) return rc;
-    const int blocks = (int)std::min<int64_t>((int64_t)info.cus, (n + kFlowPass - 1) / kFlowPass);
+    const FlowShape sh = flow_shape(n, info.cus, info.cus, fcn_lds);
+    const int blocks = sh.blocks;
     if ((rc = fl->spart.ensure((size_t)blocks * 4 * 8))) return rc;
     SampleArgs a{};
     a.n = (uint64_t)n;
@@ -1125,21 +1288,21 @@ extern "C" int vgx_flow_sample(vgx_flow* fl, const vgx_integrand* fcn, int64_t n
     a.seed_lo = (uint32_t)seed;
     a.seed_hi = (uint32_t)(seed >> 32);
     a.iteration = iteration;
+    a.tiles = sh.tiles;
     a.part = (double*)fl->spart.ptr;
     a.xout = xout;
     a.fout = fout;
     a.status = status;
-    const size_t ncp = F.kind == VGX_FCN_DIAGRIDGE ? 3 * (size_t)F.ncomp : (size_t)F.ncomp * (2 + fl->D);
-    const size_t lds = lds_layer() + kStateLds + ncp * 4;
+    const size_t lds = lds_layer() + sh.waves * sizeof(TileState) + fcn_lds;
     if (hipFuncSetAttribute((const void*)flow_sample_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)lds) != hipSuccess)
         return VGX_EHIP;
     hipEvent_t e0, e1;
     if (timed_slot(g_timing_ctx, kTimedFlowSample, &e0, &e1))
-        hipExtLaunchKernelGGL(flow_sample_kernel, dim3(blocks), dim3(kFlowThreads), (uint32_t)lds, s, e0, e1, 0,
+        hipExtLaunchKernelGGL(flow_sample_kernel, dim3(blocks), dim3(64 * sh.waves), (uint32_t)lds, s, e0, e1, 0,
                               flow_args(fl), F, a);
     else
-        hipLaunchKernelGGL(flow_sample_kernel, dim3(blocks), dim3(kFlowThreads), lds, s, flow_args(fl), F, a);
+        hipLaunchKernelGGL(flow_sample_kernel, dim3(blocks), dim3(64 * sh.waves), lds, s, flow_args(fl), F, a);
     if ((rc = check_launch())) return rc;
     if (!sums) return VGX_OK;
     std::vector<double> h((size_t)blocks * 4);
@@ -1163,9 +1326,9 @@ static int flow_inverse(vgx_flow* fl, const float* x, int64_t n, hipStream_t s) 
     if ((rc = fl->logq.ensure(nn * 4))) return rc;
     DeviceInfo info;
     if ((rc = device_info(&info))) return rc;
-    const int blocks = (int)std::min<int64_t>((int64_t)info.cus * 2, (n + kFlowPass - 1) / kFlowPass);
-    InvArgs a{(uint64_t)n, x, (float*)fl->saved.ptr, (float*)fl->u0.ptr, (float*)fl->logq.ptr};
-    hipLaunchKernelGGL(flow_inverse_kernel, dim3(blocks), dim3(kFlowThreads), lds_layer() + kStateLds, s,
+    const FlowShape sh = flow_shape(n, info.cus, 2 * info.cus, 0);
+    InvArgs a{(uint64_t)n, x, (float*)fl->saved.ptr, (float*)fl->u0.ptr, (float*)fl->logq.ptr, sh.tiles};
+    hipLaunchKernelGGL(flow_inverse_kernel, dim3(sh.blocks), dim3(64 * sh.waves), lds_layer() + kStateLds, s,
                        flow_args(fl), a);
     return check_launch();
 }
@@ -1267,15 +1430,15 @@ extern "C" int vgx_flow_eval(vgx_flow* fl, const vgx_integrand* fcn, const float
     if (!fl || !x || !f || n < 1) return VGX_EINVAL;
     hipStream_t s = (hipStream_t)stream;
     FlowFcn F{};
-    int rc = flow_fcn_params(fl, fcn, &F, s);
+    size_t fcn_lds;
+    int rc = flow_fcn_params(fl, fcn, &F, &fcn_lds);
     if (rc) return rc;
-    const size_t ncp = F.kind == VGX_FCN_DIAGRIDGE ? 3 * (size_t)F.ncomp : (size_t)F.ncomp * (2 + fl->D);
     const uint64_t ntiles = ((uint64_t)n + 15) / 16;
     const unsigned blocks = (unsigned)std::min<uint64_t>(4096, (ntiles + 3) / 4);
     if (hipFuncSetAttribute((const void*)flow_eval_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)(ncp * 4 + 16)) != hipSuccess)
+                            (int)(fcn_lds + 16)) != hipSuccess)
         return VGX_EHIP;
-    hipLaunchKernelGGL(flow_eval_kernel, dim3(blocks), dim3(256), ncp * 4 + 16, s, F, fl->D, x, (uint64_t)n, f);
+    hipLaunchKernelGGL(flow_eval_kernel, dim3(blocks), dim3(256), fcn_lds + 16, s, F, fl->D, x, (uint64_t)n, f);
     return check_launch();
 }
 
