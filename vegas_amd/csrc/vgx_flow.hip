@@ -186,13 +186,11 @@ __device__ inline bf16x4_t cond_input(const f32x4_t u, uint32_t amask, int D, in
 }
 
 // Layer 1 of the conditioner MLP for NT sample tiles: h1 = relu(W1 a) (bf16
-// fragments, output tile mt = k-step mt of layer 2); m1: tile 0's ReLU mask
-// (bit 4 mt + i: pre-activation > 0).
+// fragments, output tile mt = k-step mt of layer 2).
 template <int NT>
-__device__ inline uint32_t layer1(const LayerLds* s, const bf16x4_t (&a)[NT], int lane, bf16x4_t (&h1)[NT][8]) {
+__device__ inline void layer1(const LayerLds* s, const bf16x4_t (&a)[NT], int lane, bf16x4_t (&h1)[NT][8]) {
     const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
     const float top = relu_top();
-    uint32_t m1 = 0;
 #pragma unroll
     for (int mt = 0; mt < 8; ++mt) {
         const bf16x4_t w = half8(frag_w(s->W + kHW1, mt / 2, lane), mt & 1);
@@ -200,34 +198,24 @@ __device__ inline uint32_t layer1(const LayerLds* s, const bf16x4_t (&a)[NT], in
         for (int t = 0; t < NT; ++t) {
             f32x4_t c = mfma16(w, a[t], zero);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (t == 0) m1 |= (c[i] > 0.f ? 1u : 0u) << (4 * mt + i);
-                c[i] = relu(c[i], top);
-            }
+            for (int i = 0; i < 4; ++i) c[i] = relu(c[i], top);
             h1[t][mt] = pack_bf(c);
         }
     }
-    return m1;
 }
 
 // The conditioner MLP of NT tiles: o[t][0] = raw s, o[t][1] = t rows
-// (l/16)*4+i.  Each weight fragment read serves every tile.  Optionally keeps
-// (tile 0) h2 as bf16 fragments and the ReLU masks of h1 and h2.
-struct MlpKeep {
-    bf16x4_t h2[8];
-    uint32_t m1, m2;   // bit 4 mt + i: pre-activation > 0
-};
-
-template <int NT, bool KEEP>
+// (l/16)*4+i, and h2 as bf16 fragments.  Each weight fragment read serves
+// every tile.
+template <int NT>
 __device__ inline void mlp(const LayerLds* s, const bf16x4_t (&a)[NT], int lane, f32x4_t (&o)[NT][2],
-                           MlpKeep* keep) {
+                           bf16x4_t (&h2)[NT][8]) {
     // layer 2's output tiles accumulate MB at a time side by side
     // (independent MFMA chains), k-step by k-step
     constexpr int MB = NT == 1 ? 8 : 4;
-    bf16x4_t h1[NT][8], h2[NT][8];
+    bf16x4_t h1[NT][8];
     const float top = relu_top();
-    uint32_t m2 = 0;
-    const uint32_t m1 = layer1<NT>(s, a, lane, h1);
+    layer1<NT>(s, a, lane, h1);
 #pragma unroll
     for (int mb = 0; mb < 8; mb += MB) {
         f32x4_t acc[NT][MB];
@@ -258,10 +246,7 @@ __device__ inline void mlp(const LayerLds* s, const bf16x4_t (&a)[NT], int lane,
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    if (t == 0) m2 |= (acc[t][m][i] > 0.f ? 1u : 0u) << (4 * (mb + m) + i);
-                    acc[t][m][i] = relu(acc[t][m][i], top);
-                }
+                for (int i = 0; i < 4; ++i) acc[t][m][i] = relu(acc[t][m][i], top);
                 h2[t][mb + m] = pack_bf(acc[t][m]);
             }
     }
@@ -279,12 +264,6 @@ __device__ inline void mlp(const LayerLds* s, const bf16x4_t (&a)[NT], int lane,
 #pragma unroll
             for (int t = 0; t < NT; ++t) o[t][q] = mfma32(w, cat8(h2[t][2 * kp], h2[t][2 * kp + 1]), o[t][q]);
         }
-    if (KEEP) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) keep->h2[q] = h2[0][q];
-        keep->m1 = m1;
-        keep->m2 = m2;
-    }
 }
 
 // ------------------------------------------------------------- sampling ----
@@ -480,9 +459,10 @@ __global__ __launch_bounds__(kFlowThreads) void flow_sample_kernel(FlowArgs f, F
             for (int q = 0; q < a.tiles; q += kFlowNT) {
                 bf16x4_t a[kFlowNT];
                 f32x4_t o[kFlowNT][2];
+                bf16x4_t h2[kFlowNT][8];
 #pragma unroll
                 for (int t = 0; t < kFlowNT; ++t) a[t] = cond_input(TS->u[q + t][lane], am, f.D, lane);
-                mlp<kFlowNT, false>(L, a, lane, o, nullptr);
+                mlp<kFlowNT>(L, a, lane, o, h2);
 #pragma unroll
                 for (int t = 0; t < kFlowNT; ++t) {
                     f32x4_t uq = TS->u[q + t][lane];
@@ -631,6 +611,7 @@ __global__ __launch_bounds__(kFlowThreads) void flow_inverse_kernel(FlowArgs f, 
             for (int q = 0; q < a.tiles; q += kFlowNT) {
                 bf16x4_t ain[kFlowNT];
                 f32x4_t o[kFlowNT][2];
+                bf16x4_t h2[kFlowNT][8];
 #pragma unroll
                 for (int t = 0; t < kFlowNT; ++t) {
                     const uint64_t sl = pb + (uint64_t)(wave * a.tiles + q + t) * 16 + (lane & 15);
@@ -638,7 +619,7 @@ __global__ __launch_bounds__(kFlowThreads) void flow_inverse_kernel(FlowArgs f, 
                     if (sl < a.n) *reinterpret_cast<f32x4_t*>(a.saved + ((size_t)k * a.n + sl) * 16 + 4 * g) = uq;
                     ain[t] = cond_input(uq, am, f.D, lane);
                 }
-                mlp<kFlowNT, false>(L, ain, lane, o, nullptr);
+                mlp<kFlowNT>(L, ain, lane, o, h2);
 #pragma unroll
                 for (int t = 0; t < kFlowNT; ++t) {
                     f32x4_t uq = TS->u[q + t][lane];
@@ -764,8 +745,8 @@ struct BwdArgs {
 // Backward of one layer together with its weight gradients.  Per round each
 // wave takes one 16-sample tile (tile (round * gridDim.x + block) * 8 +
 // wave), recomputes the layer's MLP, backpropagates through the coupling and
-// the MLP, and the eight waves stage their GEMM operands in LDS (element
-// (row, sample) of a wave's slot at row * 16 + sample) in three phases:
+// the MLP, and the eight waves stage their GEMM operands in LDS in three
+// phases:
 //   1: dout (32 rows) | h2 (128)   -> dW3, b3
 //   2: dh2 (128) | h1 (128)        -> dW2, b2 (h1 recomputed from a: 8 small MFMAs
 //                                     instead of 16 registers held through the
@@ -778,47 +759,58 @@ struct BwdArgs {
 // the CU.  The tile -> workgroup assignment is static, so the sums are
 // reproducible.  Tiles past the end run on zero inputs: their dout is 0, so
 // they add nothing.
+// Two waves per SIMD (the registers of the sums) that meet at every phase:
+// vector work, products and LDS reads mostly add up.  250,000 samples, 9
+// axes: 95 us a layer with operands transposed in registers before staging
+// (eight instructions a fragment, now transposed by the read) and a compare, a
+// select and a bit per relu mask (now two packed instructions per two
+// values), 69 us so; 13 us of it load the weights and write the sums.
+// (Weight fragments read a step ahead, or 32 by 64 blocks of dW2 a wave,
+// which need a third fewer operand reads: no change.)
 constexpr int kBwdThreads = 512;
 constexpr int kBwdWaves = kBwdThreads / 64;
 constexpr int kSlotRows = 2 * kFH;         // the largest phase: dh2 | h1
-constexpr int kSlot = kSlotRows * 16;      // bf16 elements per wave slot
+// A slot is [sample][row], its row stride such that the 16 samples of a write
+// and the 32-byte runs of a transposing read spread over the banks.
+constexpr int kSlotLd = kSlotRows + 16;
+constexpr int kSlot = kSlotLd * 16;        // bf16 elements per wave slot
 constexpr int kNo3 = 2 * 9;                // dW3 output tiles: 2 row tiles x (8 column tiles + bias)
 
-// The C-layout tile v (rows row0 + (l/16)*4 + i, sample l%16) into a slot.
-// Lane (g, 4m + t) holds rows 4g..4g+3 of sample 4m + t; a 4x4 transpose of
-// the 16-bit values within the lane quad (DPP) leaves it row 4g + t of
-// samples 4m..4m+3, which it stores as one 8-byte write (at the permuted
-// chunk position frag_op reads).
+// The C-layout tile v (rows row0 + (l/16)*4 + i, sample l%16) into a slot, as
+// it lies in the registers: one 8-byte write.
 __device__ inline void stage(uint16_t* slot, int row0, const bf16x4_t v, int lane) {
-    typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
-    const u32x2_t d = __builtin_bit_cast(u32x2_t, v);
-    const int t = lane & 3;
-    // dwords with lane t^2: lanes 0,1 keep (x0,x1) and take (x0,x1) of lane
-    // t+2; lanes 2,3 take (x2,x3) of lane t-2 and keep (x2,x3)
-    const uint32_t p0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)d[0], 0x4E, 0xF, 0xF, false);
-    const uint32_t p1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)d[1], 0x4E, 0xF, 0xF, false);
-    const uint32_t a0 = t < 2 ? d[0] : p1, a1 = t < 2 ? p0 : d[1];
-    // 16-bit halves with lane t^1: even lanes lo(own) | lo(odd) << 16, odd
-    // lanes hi(even) | hi(own) << 16
-    const uint32_t q0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)a0, 0xB1, 0xF, 0xF, false);
-    const uint32_t q1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)a1, 0xB1, 0xF, 0xF, false);
-    const uint32_t sel = (t & 1) ? 0x03020706u : 0x05040100u;
-    u32x2_t r;
-    r[0] = __builtin_amdgcn_perm(q0, a0, sel);
-    r[1] = __builtin_amdgcn_perm(q1, a1, sel);
-    const int row = row0 + 4 * (lane >> 4) + t;
-    *reinterpret_cast<u32x2_t*>(slot + row * 16 + 4 * (((lane >> 2) & 3) ^ ((row >> 2) & 3))) = r;
+    *reinterpret_cast<bf16x4_t*>(slot + (lane & 15) * kSlotLd + row0 + 4 * (lane >> 4)) = v;
 }
 // Operand fragment of slot rows row0.. (A and B alike: row row0 + l%16,
-// samples (l/16)*4 .. +3).  In a slot row the four 4-sample chunks are
-// permuted, chunk c at position c ^ ((row >> 2) & 3): the 16 rows that one
-// fragment read (and the 16 that one staging store) touches then fall in
-// distinct LDS banks, where the plain 32-byte rows put every fourth row in
-// the same banks.
+// samples (l/16)*4 .. +3), transposed by the read: in 16 lanes, lane 4 k + q
+// reads rows 4 q .. +3 of sample k, and lane m receives row m of samples
+// 0..3.
 __device__ inline bf16x4_t frag_op(const uint16_t* slot, int row0, int lane) {
-    const int row = row0 + (lane & 15);
-    return *reinterpret_cast<const bf16x4_t*>(slot + row * 16 + 4 * ((lane >> 4) ^ ((row >> 2) & 3)));
+    typedef __attribute__((address_space(3))) bf16x4_t lds_bf16x4_t;
+    const uint16_t* q = slot + (4 * (lane >> 4) + ((lane >> 2) & 3)) * kSlotLd + row0 + 4 * (lane & 3);
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4_t*)q);
 }
+// v where h > 0 (bf16 values, h not negative), 0 elsewhere: two values an
+// instruction (the empty asm keeps the compiler from making a compare and a
+// select of each).
+__device__ inline bf16x4_t where_positive(const bf16x4_t v, const bf16x4_t h) {
+    typedef short s16x2_t __attribute__((ext_vector_type(2)));
+    typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+    const u32x2_t hv = __builtin_bit_cast(u32x2_t, h), vv = __builtin_bit_cast(u32x2_t, v);
+    u32x2_t r;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t hw = hv[i];
+        const s16x2_t hs = __builtin_bit_cast(s16x2_t, hw);
+        uint32_t m = __builtin_bit_cast(uint32_t, (s16x2_t)(-hs));
+        asm("" : "+v"(m));
+        m = __builtin_bit_cast(uint32_t, (s16x2_t)(__builtin_bit_cast(s16x2_t, m) >> 15));
+        asm("" : "+v"(m));
+        r[i] = vv[i] & m;
+    }
+    return __builtin_bit_cast(bf16x4_t, r);
+}
+
 // Rows row0.. of staged tiles j and j+1 as one k = 32 operand (A and B
 // alike: slots 0..3 tile j's samples (l/16)*4.., slots 4..7 tile j+1's).
 __device__ inline bf16x8_t frag_pair(const uint16_t* S, int j, int row0, int lane) {
@@ -890,8 +882,8 @@ __global__ __launch_bounds__(kBwdThreads) void flow_backward_kernel(FlowArgs f, 
         const bf16x4_t ain = cond_input(uin, am, f.D, lane);
         const bf16x4_t a1[1] = {ain};
         f32x4_t o1[1][2];
-        MlpKeep kp;
-        mlp<1, true>(L, a1, lane, o1, &kp);
+        bf16x4_t h2[1][8];
+        mlp<1>(L, a1, lane, o1, h2);
         const f32x4_t (&o)[2] = o1[0];
         // coupling backward (inverse direction)
         f32x4_t dout0, dout1, Gin;
@@ -923,7 +915,7 @@ __global__ __launch_bounds__(kBwdThreads) void flow_backward_kernel(FlowArgs f, 
         stage(my, 0, do0, ln);
         stage(my, 16, do1, ln);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) stage(my, 32 + 16 * q, kp.h2[q], ln);
+        for (int q = 0; q < 8; ++q) stage(my, 32 + 16 * q, h2[0][q], ln);
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < kBwdWaves; j += 2) {
@@ -941,11 +933,7 @@ __global__ __launch_bounds__(kBwdThreads) void flow_backward_kernel(FlowArgs f, 
         bf16x4_t dh2[8];
 #pragma unroll
         for (int mt = 0; mt < 8; ++mt) {
-            f32x4_t cc = mfma32(frag_w(Wt + kTW3, mt, lane), cat8(do0, do1), zero);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (!((kp.m2 >> (4 * mt + i)) & 1u)) cc[i] = 0.f;
-            dh2[mt] = pack_bf(cc);
+            dh2[mt] = where_positive(pack_bf(mfma32(frag_w(Wt + kTW3, mt, lane), cat8(do0, do1), zero)), h2[0][mt]);
         }
         f32x4_t acc[8];
 #pragma unroll
@@ -957,14 +945,10 @@ __global__ __launch_bounds__(kBwdThreads) void flow_backward_kernel(FlowArgs f, 
             for (int mt = 0; mt < 8; ++mt) acc[mt] = mfma32(frag_w(Wt + kTW2, mt * 4 + kp2, lane), b, acc[mt]);
             __builtin_amdgcn_sched_barrier(0);
         }
-        bf16x4_t dh1[8];
+        bf16x4_t h1[1][8], dh1[8];
+        layer1<1>(L, a1, lane, h1);
 #pragma unroll
-        for (int mt = 0; mt < 8; ++mt) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (!((kp.m1 >> (4 * mt + i)) & 1u)) acc[mt][i] = 0.f;
-            dh1[mt] = pack_bf(acc[mt]);
-        }
+        for (int mt = 0; mt < 8; ++mt) dh1[mt] = where_positive(pack_bf(acc[mt]), h1[0][mt]);
         f32x4_t da = zero;
 #pragma unroll
         for (int kt = 0; kt < 8; kt += 2) da = mfma32(frag_w(Wt + kTW1, kt / 2, lane), cat8(dh1[kt], dh1[kt + 1]), da);
@@ -976,14 +960,10 @@ __global__ __launch_bounds__(kBwdThreads) void flow_backward_kernel(FlowArgs f, 
         if (live) *reinterpret_cast<f32x4_t*>(a.G + sl * 16 + 4 * g) = Gin;
         __syncthreads();
         // ---- phase 2: dh2 | h1 -> dW2, b2
-        {
-            bf16x4_t h1[1][8];
-            layer1<1>(L, a1, lane, h1);
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                stage(my, 16 * q, dh2[q], ln);
-                stage(my, kFH + 16 * q, h1[0][q], ln);
-            }
+        for (int q = 0; q < 8; ++q) {
+            stage(my, 16 * q, dh2[q], ln);
+            stage(my, kFH + 16 * q, h1[0][q], ln);
         }
         __syncthreads();
 #pragma unroll
