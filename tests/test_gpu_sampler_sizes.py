@@ -98,3 +98,57 @@ def test_long_mixture(va, nc, dim, neval, kind):
     rb = va.Integrator([[0, 1]] * dim, neval=neval, seed=29, precision='f32')(g, nitn=1).itn_results[0]
     assert abs(ra.mean - rb.mean) <= 2e-5 * abs(rb.mean)
     assert abs(ra.sdev - rb.sdev) <= 1e-3 * rb.sdev
+
+
+@pytest.mark.parametrize("dim,neval,batch", [(1, 1000, 300), (2, 100, 1), (3, 257 * 12, 256), (4, 200000, 50001),
+                                             (8, 300000, 10 ** 9), (16, 5000, 777), (17, 3000, 500), (30, 600, 10 ** 9)])
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_staged_points(va, dim, neval, batch, precision):
+    """Points, weights and hcubes of the staged sampler, over batches that end
+    inside and at a workgroup's 256 points, from their own y (1e-12: a few
+    roundings of the map and the Jacobian)."""
+    integ = va.Integrator([[-1, 2]] * dim, neval=neval, seed=5, min_neval_batch=batch, precision=precision)
+    integ(va.GaussianMixture([1.0], [3.0], [[0.4] * dim]), nitn=2)
+    parts = list(integ.random_batch(yield_hcube=True, yield_y=True))
+    x, y, w, h = (np.concatenate([p[i] for p in parts]) for i in range(4))
+    assert len(x) == integ.last_neval and np.all(np.diff(h) >= 0) and h[0] == 0 and h[-1] == integ.nhcube - 1
+    ns = np.asarray(integ.nstrat, np.int64)
+    own = np.zeros(len(y), np.int64)
+    for d in range(dim)[::-1]:  # axis 0 varies fastest
+        own = own * ns[d] + np.minimum((y[:, d] * ns[d]).astype(np.int64), ns[d] - 1)
+    assert np.mean(own != h) <= 1e-3  # (a y next to a stratum's edge may round over it)
+    xm, jac = (np.empty_like(y), np.empty(len(y)))
+    integ.map.map(y, xm, jac)
+    np.testing.assert_allclose(x, xm, rtol=1e-12, atol=1e-12)
+    n_h = np.bincount(h, minlength=integ.nhcube)
+    np.testing.assert_allclose(w, jac / integ.nhcube / n_h[h], rtol=1e-12)
+
+
+@pytest.mark.parametrize("per", [2, 31, 32, 33, 64, 65, 2048, 2049, 5000])
+def test_covariance_components(va, per):
+    """Every number of components that has its own kernel (1-6) against the
+    pairwise kernel (7) and the scalar path, with hcubes on both sides of each
+    thread, wave and workgroup border.  The sums differ in their order only
+    (per points: 1e-12 covers 5000 roundings of terms that do not cancel)."""
+    import torch
+    ns = [5, 3]
+
+    def run(m):
+        def f(x):
+            g = torch.exp(-3.0 * ((x - 0.4) ** 2).sum(1))
+            return torch.stack([g * (1 + x[:, 0] * k) * (1 + 0.5 * x[:, 1]) ** k for k in range(m)], 1) if m else g
+        integ = va.Integrator([[0, 1], [0, 2]], neval=15 * per, nstrat=ns, beta=0.0, seed=3)
+        r = integ(va.gpu_lbatchintegrand(f), nitn=1).itn_results[0]
+        assert integ.last_neval == 15 * per
+        return r
+
+    full = run(7)
+    cov, scale = np.asarray(full.cov), np.sqrt(np.diag(full.cov))
+    for m in range(1, 7):
+        r = run(m)
+        np.testing.assert_allclose(np.asarray(r.mean), np.asarray(full.mean)[:m], rtol=1e-12)
+        np.testing.assert_allclose(np.asarray(r.cov) / np.outer(scale[:m], scale[:m]),
+                                   cov[:m, :m] / np.outer(scale[:m], scale[:m]), atol=1e-11)
+    one = run(0)
+    assert abs(one.mean - full.mean[0]) <= 1e-12 * one.mean
+    assert abs(one.var - cov[0, 0]) <= 1e-10 * one.var

@@ -687,24 +687,27 @@ __global__ void sigf_reset_kernel(double* sigf, int64_t n, Scalars* sc) {
 
 // eval_point for hcube h with the stratum->bin path the fused sampler takes
 // for this geometry (staged and error-training kernels).
-template <bool R32>
+template <int DIM, bool R32>
 __device__ inline void eval_point_h(const IterGeom& g, const AxisC* axes, const double* grid, uint32_t h,
                                     uint32_t p, double* x, double& J, int* kb) {
-    PackedCoords<0> pc;
+    PackedCoords<DIM> pc;
     uint32_t zmin = 0xFFFFFFFFu;
     if constexpr (R32) {
         if (g.per_all) {
             pc.set(axes, g.dim, h);
-            eval_point<0, true, true>(tile_geom(g), axes, grid, pc, h, p, x, J, kb, zmin);
+            eval_point<DIM, true, true>(tile_geom(g), axes, grid, pc, h, p, x, J, kb, zmin);
             if (zmin == 0) {
-                const uint64_t zm = per_zero_axes<0>(tile_geom(g), pc, p);
-                for (int d = 0; d < g.dim; ++d)
+                const uint64_t zm = per_zero_axes<DIM>(tile_geom(g), pc, p);
+#pragma unroll
+                for (int d = 0; d < nd_max(DIM); ++d) {
+                    if (DIM <= 0 && d >= g.dim) break;
                     if ((zm >> d) & 1) kb[d] = -1;
+                }
             }
             return;
         }
     }
-    eval_point<0, R32, false>(tile_geom(g), axes, grid, pc, h, p, x, J, kb, zmin);
+    eval_point<DIM, R32, false>(tile_geom(g), axes, grid, pc, h, p, x, J, kb, zmin);
 }
 
 // adapt_to_errors: training entry |var_h| at the last point of every hcube
@@ -719,7 +722,7 @@ __global__ __launch_bounds__(256) void errors_train_kernel(IterGeom g, const Axi
         double x[VGX_MAXDIM];
         int kb[VGX_MAXDIM];
         double J;
-        eval_point_h<R32>(g, axes, grid, (uint32_t)h, off[h + 1] - 1, x, J, kb);
+        eval_point_h<0, R32>(g, axes, grid, (uint32_t)h, off[h + 1] - 1, x, J, kb);
         for (int d = 0; d < g.dim; ++d)
             if (kb[d] >= 0) {
                 unsafeAtomicAdd(&sum_f[d * g.nb + kb[d]], errv[h]);
@@ -755,30 +758,99 @@ __global__ __launch_bounds__(1024) void max_exponent_kernel(const double* A, int
 }
 
 // Staged path: x, y, weight and hcube of points [p0, p1) (pyx:1731-1759).
-template <bool R32>
-__global__ __launch_bounds__(256) void sample_kernel(IterGeom g, const AxisC* axes, const double* grid,
-                                                     const uint32_t* off, uint32_t h0, uint32_t h1,
-                                                     uint32_t p0, uint32_t p1, double* x, double* y,
-                                                     double* wgt, int64_t* hcube, const Scalars* sc) {
+// 256 consecutive points a step: the workgroup finds the hcube of the first
+// (256 probes at a time) and takes the boundaries after it into LDS, where
+// each point finds its own; with the dimension known x stays in registers,
+// and goes out in whole rows through LDS.  Bound by its writes and by Philox.
+// 2e6 points, 8 axes: 130 us with a search over all boundaries per point, the
+// axes in scratch and x written axis by axis, 71 so (144 MB; 29 us at copy
+// rate).
+constexpr int kSampThreads = 256;
+template <int DIM, bool R32>
+__global__ __launch_bounds__(kSampThreads) void sample_kernel(IterGeom g, const AxisC* axes, const double* grid,
+                                                              const uint32_t* off, uint32_t h0, uint32_t h1,
+                                                              uint32_t p0, uint32_t p1, double* x, double* y,
+                                                              double* wgt, int64_t* hcube, const Scalars* sc) {
     if (sc->status) return;
-    const int dim = g.dim;
-    for (uint32_t p = p0 + blockIdx.x * blockDim.x + threadIdx.x; p < p1; p += gridDim.x * blockDim.x) {
-        uint32_t lo = h0, hi = h1 - 1;  // largest h with off[h] <= p
-        while (lo < hi) {
-            uint32_t mid = (lo + hi + 1) >> 1;
-            if (off[mid] <= p) lo = mid; else hi = mid - 1;
+    const int dim = DIM > 0 ? DIM : g.dim;
+    constexpr int kRow = DIM > 0 ? (DIM | 1) : 1;  // odd: lanes' rows start in different banks
+    __shared__ double xs[DIM > 0 ? kSampThreads * kRow : 1];
+    __shared__ uint32_t so[kSampThreads + 2];
+    const int t = threadIdx.x;
+    for (uint64_t pb = (uint64_t)p0 + (uint64_t)blockIdx.x * kSampThreads; pb < p1;
+         pb += (uint64_t)gridDim.x * kSampThreads) {
+        uint32_t hlo = h0, hhi = h1 - 1;  // largest h with off[h] <= pb
+        while (hlo < hhi) {
+            const uint32_t step = (hhi - hlo) / kSampThreads + 1;
+            const uint64_t m = hlo + (uint64_t)t * step;
+            const int c = __syncthreads_count(m <= hhi && off[m] <= pb);
+            if (c > 0) hlo += (uint32_t)(c - 1) * step;
+            hhi = min(hhi, hlo + (step - 1));
         }
-        const uint32_t h = lo;
-        const uint32_t n = off[h + 1] - off[h];
-        double xx[VGX_MAXDIM];
-        int kb[VGX_MAXDIM];
+        for (int i = t; i < kSampThreads + 2; i += kSampThreads) so[i] = off[min((uint64_t)hlo + i, (uint64_t)h1)];
+        __syncthreads();
+        const bool live = pb + t < p1;
+        const uint32_t p = live ? (uint32_t)(pb + t) : (uint32_t)pb;
+        uint32_t a = 0, b = min((uint32_t)kSampThreads, h1 - 1 - hlo);
+        while (a < b) {
+            const uint32_t mid = (a + b + 1) >> 1;
+            if (so[mid] <= p) a = mid; else b = mid - 1;
+        }
+        uint32_t h = hlo + a, beg = so[a], end = so[a + 1];
+        if (end <= p && h + 1 < h1) {  // beyond the table (empty hcubes only)
+            uint32_t lo = h, hi = h1 - 1;
+            while (lo < hi) {
+                const uint32_t mid = lo + (hi - lo + 1) / 2;
+                if (off[mid] <= p) lo = mid; else hi = mid - 1;
+            }
+            h = lo;
+            beg = off[h];
+            end = off[h + 1];
+        }
+        double xx[nd_max(DIM)];
+        int kb[nd_max(DIM)];
         double J;
-        eval_point_h<R32>(g, axes, grid, h, p, xx, J, kb);
+        eval_point_h<DIM, R32>(g, axes, grid, h, p, xx, J, kb);
         const int64_t i = (int64_t)(p - p0);
-        for (int d = 0; d < dim; ++d) x[i * dim + d] = xx[d];
-        if (y) point_y<R32>(tile_geom(g), axes, h, p, y + i * dim);
-        if (wgt) wgt[i] = J * (g.dv_y / (double)n);
-        if (hcube) hcube[i] = (int64_t)h;
+        if constexpr (DIM > 0) {
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) xs[t * kRow + d] = xx[d];
+            __syncthreads();
+            double* xo = x + (pb - p0) * DIM;
+            const int tot = (int)min((uint64_t)kSampThreads, p1 - pb) * DIM;
+            for (int e = t; e < tot; e += kSampThreads) xo[e] = xs[(e / DIM) * kRow + e % DIM];
+        } else if (live) {
+            for (int d = 0; d < dim; ++d) x[i * dim + d] = xx[d];
+        }
+        if (live) {
+            if (y) point_y<R32>(tile_geom(g), axes, h, p, y + i * dim);
+            if (wgt) wgt[i] = J * (g.dv_y / (double)(end - beg));
+            if (hcube) hcube[i] = (int64_t)h;
+        }
+        __syncthreads();  // so and xs are written again
+    }
+}
+
+template <bool R32>
+static auto sample_kernel_of(int dim) {
+    switch (dim) {
+        case 1: return sample_kernel<1, R32>;
+        case 2: return sample_kernel<2, R32>;
+        case 3: return sample_kernel<3, R32>;
+        case 4: return sample_kernel<4, R32>;
+        case 5: return sample_kernel<5, R32>;
+        case 6: return sample_kernel<6, R32>;
+        case 7: return sample_kernel<7, R32>;
+        case 8: return sample_kernel<8, R32>;
+        case 9: return sample_kernel<9, R32>;
+        case 10: return sample_kernel<10, R32>;
+        case 11: return sample_kernel<11, R32>;
+        case 12: return sample_kernel<12, R32>;
+        case 13: return sample_kernel<13, R32>;
+        case 14: return sample_kernel<14, R32>;
+        case 15: return sample_kernel<15, R32>;
+        case 16: return sample_kernel<16, R32>;
+        default: return sample_kernel<0, R32>;
     }
 }
 
@@ -1240,17 +1312,11 @@ extern "C" int vgx_iter_sample(vgx_ctx* ctx, const vgx_config* c, vgx_state* st,
     if (rc) return rc;
     if ((rc = init_axes(&R, s))) return rc;
     set_iter(&R, c, it);
-    const int64_t n = p1 - p0;
-    int64_t b = (n + 255) / 256;
-    if (b > 4096) b = 4096;
-    if (R.g.rng32)
-        hipLaunchKernelGGL(sample_kernel<true>, dim3((unsigned)b), dim3(256), 0, s, R.g, (const AxisC*)R.axes,
-                           (const double*)st->grid, (const uint32_t*)ctx->off.ptr, (uint32_t)h0, (uint32_t)h1,
-                           (uint32_t)p0, (uint32_t)p1, x, y, wgt, hcube, (const Scalars*)R.sc);
-    else
-        hipLaunchKernelGGL(sample_kernel<false>, dim3((unsigned)b), dim3(256), 0, s, R.g, (const AxisC*)R.axes,
-                           (const double*)st->grid, (const uint32_t*)ctx->off.ptr, (uint32_t)h0, (uint32_t)h1,
-                           (uint32_t)p0, (uint32_t)p1, x, y, wgt, hcube, (const Scalars*)R.sc);
+    const int64_t b = std::min<int64_t>((p1 - p0 + kSampThreads - 1) / kSampThreads, 1 << 20);
+    const auto k = R.g.rng32 ? sample_kernel_of<true>(c->dim) : sample_kernel_of<false>(c->dim);
+    hipLaunchKernelGGL(k, dim3((unsigned)b), dim3(kSampThreads), 0, s, R.g, (const AxisC*)R.axes,
+                       (const double*)st->grid, (const uint32_t*)ctx->off.ptr, (uint32_t)h0, (uint32_t)h1,
+                       (uint32_t)p0, (uint32_t)p1, x, y, wgt, hcube, (const Scalars*)R.sc);
     return check_launch();
 }
 
