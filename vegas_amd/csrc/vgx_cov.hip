@@ -2,7 +2,7 @@
 // the mean vector and the covariance (or the variances) of one iteration,
 // src/vegas/_vegas.pyx:2136-2183 with correlate_integrals on or off.
 //
-// Work item: (hcube h, component pair q, or all pairs for m <= 4).  A thread
+// Work item: (hcube h, component pair q, or all pairs for m <= 6).  A thread
 // owns a strided set of the batch's hcubes (the long ones are shared by its
 // workgroup); for each hcube it makes the reference's two passes over the
 // hcube's points: S = sum w f (per component), then the deviations
@@ -18,7 +18,12 @@ namespace vgx {
 constexpr int kCovThreads = 256;
 constexpr int kCovWaves = kCovThreads / 64;
 constexpr int kCovMaxBlocks = 8192;  // workgroups per pair (one thread per hcube up to 2M hcubes)
-constexpr uint32_t kCovLong = 32;    // hcubes with more points are summed by the whole workgroup
+// A hcube of up to kCovShort points is summed by a thread, of up to kCovLong by
+// a wave, a longer one by the workgroup.  (Everything above 32 by the workgroup
+// in turn: up to 375 us a batch of 2e6 points in adapted strata, 8 axes, four
+// components, now up to 170.  From 16 by a wave: 5-15 % slower where most
+// hcubes are that short; from 8 twice the time.)
+constexpr uint32_t kCovShort = 32, kCovLong = 2048;
 
 // Pair q of the lower triangle (t <= s), row-major: (0,0) (1,0) (1,1) (2,0) ...
 __device__ inline void cov_pair(int q, int correlate, int& s, int& t) {
@@ -54,13 +59,67 @@ __device__ inline void block_sum(double (&v)[K], double* red) {
     __syncthreads();
 }
 
+__device__ inline double lane_value(double v, int lane) {
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)u, lane), hi = __builtin_amdgcn_readlane((uint32_t)(u >> 32), lane);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+// v from lane (l & ~15) | ((l + N) & 15): a rotation within 16 lanes.
+template <int N>
+__device__ inline double row_ror(double v) {
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (uint32_t)u, 0x120 + N, 0xF, 0xF, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (uint32_t)(u >> 32), 0x120 + N, 0xF, 0xF, true);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+// a + b of the halves (SIXTEEN: the odd and even rows of 16 lanes) of the wave:
+// the lower (even) lanes receive a's, the upper (odd) lanes b's.
+template <bool SIXTEEN>
+__device__ inline double fold2(double a, double b) {
+    const uint64_t ua = (uint64_t)__double_as_longlong(a), ub = (uint64_t)__double_as_longlong(b);
+    uint32_t x[2], y[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t wa = (uint32_t)(ua >> (32 * i)), wb = (uint32_t)(ub >> (32 * i));
+        const auto r = SIXTEEN ? __builtin_amdgcn_permlane16_swap(wa, wb, false, false)
+                               : __builtin_amdgcn_permlane32_swap(wa, wb, false, false);
+        x[i] = r[0];
+        y[i] = r[1];
+    }
+    return __longlong_as_double((long long)(((uint64_t)x[1] << 32) | x[0])) +
+           __longlong_as_double((long long)(((uint64_t)y[1] << 32) | y[0]));
+}
+// Wave sum of K values per lane, in a fixed order; every lane receives the
+// totals.  Two foldings leave a quarter of the values in each 16 lanes, which
+// add theirs: a third of the instructions of K butterflies.
+template <int K>
+__device__ inline void wave_total(double (&v)[K]) {
+    constexpr int Q = (K + 3) / 4;
+    double z[4 * Q];
+#pragma unroll
+    for (int k = 0; k < 4 * Q; ++k) z[k] = k < K ? v[k] : 0.0;
+#pragma unroll
+    for (int k = 0; k < 2 * Q; ++k) z[k] = fold2<false>(z[k], z[2 * Q + k]);
+#pragma unroll
+    for (int k = 0; k < Q; ++k) {
+        z[k] = fold2<true>(z[k], z[Q + k]);
+        z[k] += row_ror<8>(z[k]);
+        z[k] += row_ror<4>(z[k]);
+        z[k] += row_ror<2>(z[k]);
+        z[k] += row_ror<1>(z[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = lane_value(z[k % Q], 16 * (k / Q));
+}
+
 // The hcubes [h0, h1) in rounds of gridDim.x * blockDim.x: thread t of
 // workgroup b takes hcube h0 + r0 + t * gridDim.x + b (neighbouring hcubes,
 // which tend to be large together near a peak, land in different
-// workgroups).  A hcube of at most kCovLong points is summed by its thread
-// (wk.thread_hcube); longer ones are summed after the round by the whole
-// workgroup, in thread order (wk.block_hcube), so the work per thread stays
-// bounded however the points are spread.  A hcube whose points are not the
+// workgroups).  A hcube of at most kCovShort points is summed by its thread
+// (wk.thread_hcube), a longer one after that by the thread's wave
+// (wk.wave_hcube), and those of more than kCovLong points after the round by
+// the whole workgroup, in thread order (wk.block_hcube), so the work per
+// thread stays bounded however the points are spread.  A hcube whose points are not the
 // batch's [p0, p1) (or that has fewer than two) sets VGX_ERANGE and is not read.
 template <class Work>
 __device__ inline void cov_rounds(const uint32_t* off, uint32_t h0, uint32_t h1, uint32_t p0, uint32_t p1,
@@ -70,18 +129,26 @@ __device__ inline void cov_rounds(const uint32_t* off, uint32_t h0, uint32_t h1,
     const uint32_t nh = h1 - h0, stride = gridDim.x * blockDim.x;
     for (uint32_t r0 = 0; r0 < nh; r0 += stride) {
         const uint32_t idx = r0 + threadIdx.x * gridDim.x + blockIdx.x;
-        bool lng = false;
+        bool lng = false, mid = false;
+        uint32_t oa = 0, ob = 0;
         if (idx < nh) {
-            const uint32_t oa = off[h0 + idx], ob = off[h0 + idx + 1];
+            oa = off[h0 + idx];
+            ob = off[h0 + idx + 1];
             if (oa < p0 || ob > p1 || ob < oa + 2) {
                 if (status) atomicOr(status, VGX_ERANGE);
             } else if (ob - oa > kCovLong) {
                 lng = true;
                 la[threadIdx.x] = oa - p0;
                 lb[threadIdx.x] = ob - p0;
+            } else if (ob - oa > kCovShort) {
+                mid = true;
             } else {
                 wk.thread_hcube(oa - p0, ob - p0);
             }
+        }
+        for (uint64_t mk = __ballot(mid); mk; mk &= mk - 1) {
+            const int src = __builtin_ctzll(mk);
+            wk.wave_hcube(__builtin_amdgcn_readlane(oa, src) - p0, __builtin_amdgcn_readlane(ob, src) - p0, src);
         }
         const uint64_t bal = __ballot(lng);
         if ((threadIdx.x & 63) == 0) lmask[threadIdx.x >> 6] = bal;
@@ -117,6 +184,21 @@ struct PairWork {
         double v[3] = {0.0, 0.0, 0.0};
         pass2(a, b, 1, Ss / n, St / n, v);
         close(n, Ss, v);
+    }
+    // by the wave, into lane src's sums
+    __device__ void wave_hcube(uint32_t a, uint32_t b, int src) {
+        const int lane = threadIdx.x & 63;
+        const double n = (double)(b - a);
+        double S[2] = {0.0, 0.0};
+        for (uint32_t j = a + lane; j < b; j += 64) {
+            S[0] += w[j] * f[(size_t)j * m + s];
+            S[1] += w[j] * f[(size_t)j * m + t];
+        }
+        wave_total<2>(S);
+        double v[3] = {0.0, 0.0, 0.0};
+        pass2(a + lane, b, 64, S[0] / n, S[1] / n, v);
+        wave_total<3>(v);
+        if (lane == src) close(n, S[0], v);
     }
     __device__ void block_hcube(uint32_t a, uint32_t b) {
         const double n = (double)(b - a);
@@ -197,10 +279,11 @@ __global__ __launch_bounds__(kCovThreads) void cov_hcube_kernel(const uint32_t* 
 }
 
 // Up to kCovAllMax components: every pair at once from the hcube's
-// contiguous rows of f (each row read once per pass), plain FP64 sums per
-// thread, then the same fixed-order double-double reduction and partial
+// contiguous rows of f (each row read once per pass), then the same fixed-order double-double reduction and partial
 // layout as cov_hcube_kernel.
-constexpr int kCovAllMax = 4;
+// (Pair by pair, six components took 980-4400 us a batch of 2e6 points, 12
+// axes, now 142-324; 250 registers.)
+constexpr int kCovAllMax = 6;
 
 template <int M>
 struct AllWork {
@@ -208,7 +291,7 @@ struct AllWork {
     const double* w;
     const double* f;
     double eps;
-    double am[M], av[NP];
+    DD am[M], av[NP];
     double* red;
 
     __device__ void thread_hcube(uint32_t a, uint32_t b) {
@@ -219,6 +302,19 @@ struct AllWork {
         double v[M + NP];
         pass2(a, b, 1, S, (double)(b - a), v);
         close((double)(b - a), S, v);
+    }
+    // by the wave, into lane src's sums
+    __device__ void wave_hcube(uint32_t a, uint32_t b, int src) {
+        const int lane = threadIdx.x & 63;
+        double S[M];
+#pragma unroll
+        for (int s = 0; s < M; ++s) S[s] = 0.0;
+        pass1(a + lane, b, 64, S);
+        wave_total<M>(S);
+        double v[M + NP];
+        pass2(a + lane, b, 64, S, (double)(b - a), v);
+        wave_total<M + NP>(v);
+        if (lane == src) close((double)(b - a), S, v);
     }
     __device__ void block_hcube(uint32_t a, uint32_t b) {
         double S[M];
@@ -270,14 +366,21 @@ struct AllWork {
                 for (int t = 0; t < s; ++t) v[M + s * (s + 1) / 2 + t] += d[s] * d[t];
         }
     }
+    // double-double beyond four components, as PairWork; plain up to four
+    static __device__ void add(DD& a, double v) {
+        if constexpr (M > 4)
+            dd_add(a, v);
+        else
+            a.hi += v;
+    }
     __device__ void close(double n, const double (&S)[M], const double (&v)[M + NP]) {
 #pragma unroll
         for (int s = 0; s < M; ++s) {
-            am[s] += S[s] + v[s];
+            add(am[s], S[s] + v[s]);
 #pragma unroll
             for (int t = 0; t <= s; ++t) {
                 const int q = s * (s + 1) / 2 + t;
-                av[q] += (n * v[M + q] - v[s] * v[t]) / (n - 1.);
+                add(av[q], (n * v[M + q] - v[s] * v[t]) / (n - 1.));
             }
         }
     }
@@ -296,15 +399,15 @@ __global__ __launch_bounds__(kCovThreads) void cov_hcube_all_kernel(const uint32
     wk.eps = kEpsilon;
     wk.red = red;
 #pragma unroll
-    for (int s = 0; s < M; ++s) wk.am[s] = 0.0;
+    for (int s = 0; s < M; ++s) wk.am[s] = DD{0, 0};
 #pragma unroll
-    for (int q = 0; q < NP; ++q) wk.av[q] = 0.0;
+    for (int q = 0; q < NP; ++q) wk.av[q] = DD{0, 0};
     cov_rounds(off, h0, h1, p0, p1, status, wk);
     // workgroup partials: mean entries then pair entries, DD per wave
     const int wv = threadIdx.x >> 6;
 #pragma unroll
     for (int k = 0; k < M + NP; ++k) {
-        const DD r = wave_sum_dd(DD{k < M ? wk.am[k] : wk.av[k - M], 0.0});
+        const DD r = wave_sum_dd(k < M ? wk.am[k] : wk.av[k - M]);
         if ((threadIdx.x & 63) == 0) {
             red[2 * ((size_t)wv * (M + NP) + k)] = r.hi;
             red[2 * ((size_t)wv * (M + NP) + k) + 1] = r.lo;
@@ -403,6 +506,10 @@ extern "C" int vgx_iter_accumulate_cov(vgx_ctx* ctx, const vgx_config* c, int64_
         case 3: hipLaunchKernelGGL(cov_hcube_all_kernel<3>, dim3(nbx), dim3(kCovThreads), 0, s, off, (uint32_t)h0,
                                    (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, part, status); break;
         case 4: hipLaunchKernelGGL(cov_hcube_all_kernel<4>, dim3(nbx), dim3(kCovThreads), 0, s, off, (uint32_t)h0,
+                                   (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, part, status); break;
+        case 5: hipLaunchKernelGGL(cov_hcube_all_kernel<5>, dim3(nbx), dim3(kCovThreads), 0, s, off, (uint32_t)h0,
+                                   (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, part, status); break;
+        case 6: hipLaunchKernelGGL(cov_hcube_all_kernel<6>, dim3(nbx), dim3(kCovThreads), 0, s, off, (uint32_t)h0,
                                    (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, part, status); break;
         default:
             hipLaunchKernelGGL(cov_hcube_kernel, dim3(nbx, npairs), dim3(kCovThreads), 0, s, off, (uint32_t)h0,
