@@ -186,8 +186,15 @@ int vgx_integrate(vgx_ctx* ctx, const vgx_config* cfg, const vgx_integrand* fcn,
  * vgx_iter_begin    allocation + scan; writes n_h (device int32[nhcube]) so
  *                   the caller can cut batches at hcube boundaries exactly
  *                   as _random_batch does (pyx:1692-1710);
+ * vgx_iter_batches  or those batches themselves, with one wait for the
+ *                   stream: out (host int64[3 + 2 max], max <= 4096) = {points,
+ *                   0, batches, then h1 and p1 of each}; VGX_ERANGE when there
+ *                   are more than max;
  * vgx_iter_sample   x (and optionally y, wgt, hcube) for the hcubes
  *                   [h0, h1) (pyx:1731-1759);
+ * vgx_iter_values   component 0 (f0, device double[n], may be NULL) of a
+ *                   batch's values f (device double[n][m]), and *nan (device
+ *                   int32) |= 1 if any of them is a NaN;
  * vgx_iter_accumulate  per-hcube sums and training data for the same batch
  *                   given f (device double[n]) (pyx:2136-2197);
  * vgx_iter_end      closes the iteration: estimate, sum_sigf, running
@@ -195,6 +202,9 @@ int vgx_integrate(vgx_ctx* ctx, const vgx_config* cfg, const vgx_integrand* fcn,
  *                   index within cfg->nitn.                              */
 int vgx_iter_begin(vgx_ctx* ctx, const vgx_config* cfg, vgx_state* st, int it,
                    int32_t* n_h, int64_t* total_host, void* stream);
+int vgx_iter_batches(vgx_ctx* ctx, const vgx_config* cfg, vgx_state* st, int64_t min_batch, int max,
+                     int64_t* out, void* stream);
+int vgx_iter_values(const double* f, int64_t n, int m, double* f0, int32_t* nan, void* stream);
 int vgx_iter_sample(vgx_ctx* ctx, const vgx_config* cfg, vgx_state* st, int it,
                     int64_t h0, int64_t h1, int64_t p0, int64_t p1,
                     double* x, double* y, double* wgt, int64_t* hcube, void* stream);

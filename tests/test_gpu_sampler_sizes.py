@@ -152,3 +152,41 @@ def test_covariance_components(va, per):
     one = run(0)
     assert abs(one.mean - full.mean[0]) <= 1e-12 * one.mean
     assert abs(one.var - cov[0, 0]) <= 1e-10 * one.var
+
+
+@pytest.mark.parametrize("dim,neval,batch", [(1, 50, 10 ** 9), (2, 1000, 1), (2, 1000, 2.5), (3, 30000, 7),
+                                             (3, 30000, 8), (4, 200000, 49999), (4, 200000, 0), (5, 100000, float('inf')),
+                                             (8, 900000, 100000)])
+def test_batch_cuts(va, dim, neval, batch):
+    """The device's batches (and those of the host beyond its limit) against
+    the reference's cut of the same counts."""
+    from vegas_amd import _geometry
+    integ = va.Integrator([[0, 1]] * dim, neval=neval, seed=5)
+    integ(va.GaussianMixture([1.0], [30.0], [[0.4] * dim]), nitn=2)
+    integ.min_neval_batch = batch
+    parts = [p[2] for p in integ.random_batch(yield_hcube=True)]
+    h = np.concatenate(parts)
+    cuts = _geometry.batches(np.bincount(h, minlength=integ.nhcube), batch)
+    assert [len(p) for p in parts] == [p1 - p0 for _, _, p0, p1 in cuts]
+    assert [int(p[0]) for p in parts] == [h0 for h0, _, _, _ in cuts]
+
+
+@pytest.mark.parametrize("n", [1, 255, 1025, 4096 * 256 + 3])
+@pytest.mark.parametrize("m", [1, 2, 3, 7, 300])
+def test_batch_values(va, n, m):
+    """Component 0 and the NaN flag of a batch, with a NaN in the last value."""
+    import torch
+    from vegas_amd import _lib
+    n = min(n, 4 * 10 ** 6 // m)
+    f = torch.rand((n, m), dtype=torch.float64, device='cuda')
+    f[n // 2, m // 2] = float('inf')
+    f0, flag = torch.empty(n, dtype=torch.float64, device='cuda'), torch.zeros(1, dtype=torch.int32, device='cuda')
+
+    def run(out):
+        _lib.check(_lib.lib().vgx_iter_values(_lib.ptr(f), n, m, out, _lib.ptr(flag), _lib.stream_ptr()))
+
+    run(_lib.ptr(f0))
+    assert torch.equal(f0, f[:, 0]) and int(flag.item()) == 0
+    f[n - 1, m - 1] = float('nan')
+    run(None)
+    assert int(flag.item()) == 1

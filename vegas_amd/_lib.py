@@ -76,6 +76,8 @@ def lib():
                                 C.POINTER(VgxState), vp]
     L.vgx_iter_begin.argtypes = [vp, C.POINTER(VgxConfig), C.POINTER(VgxState), C.c_int, vp,
                                  C.POINTER(C.c_int64), vp]
+    L.vgx_iter_batches.argtypes = [vp, C.POINTER(VgxConfig), C.POINTER(VgxState), C.c_int64, C.c_int, vp, vp]
+    L.vgx_iter_values.argtypes = [vp, C.c_int64, C.c_int, vp, vp, vp]
     L.vgx_iter_sample.argtypes = [vp, C.POINTER(VgxConfig), C.POINTER(VgxState), C.c_int,
                                   C.c_int64, C.c_int64, C.c_int64, C.c_int64, vp, vp, vp, vp, vp]
     L.vgx_iter_accumulate.argtypes = [vp, C.POINTER(VgxConfig), C.POINTER(VgxState), C.c_int,

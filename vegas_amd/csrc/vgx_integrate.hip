@@ -831,6 +831,67 @@ __global__ __launch_bounds__(kSampThreads) void sample_kernel(IterGeom g, const 
     }
 }
 
+// Batch boundaries of an iteration (pyx:1692-1710): a batch closes at the
+// first hcube where its points reach min_batch, or at the last hcube.  out =
+// {total, overflow, batches or -1, (h1, p1) per batch}; one workgroup, each
+// boundary found with 256 probes at a time, a serial chain of a few memory
+// latencies each.  (Copying the counts of 260,000 hcubes to the host and
+// summing them there took 250 us an iteration.)
+__global__ __launch_bounds__(256) void batch_cuts_kernel(const uint32_t* off, uint32_t nh, uint64_t min_batch, int max,
+                                                         const Scalars* sc, int64_t* out) {
+    uint32_t h0 = 0;
+    int n = 0;
+    while (h0 < nh && !sc->overflow) {
+        if (n == max) {
+            n = -1;
+            break;
+        }
+        const uint64_t p0 = off[h0];
+        uint32_t lo = h0, hi = nh;  // largest i with off[i] - p0 < min_batch
+        while (lo < hi) {
+            const uint32_t step = (hi - lo) / 256 + 1;
+            const uint64_t m = lo + (uint64_t)threadIdx.x * step;
+            const int c = __syncthreads_count(m <= hi && off[m] - p0 < min_batch);
+            lo += (uint32_t)(c - 1) * step;  // c > 0: m = lo is one
+            hi = min(hi, lo + (step - 1));
+        }
+        h0 = min(lo + 1, nh);
+        if (threadIdx.x == 0) {
+            out[3 + 2 * n] = h0;
+            out[4 + 2 * n] = off[h0];
+        }
+        ++n;
+    }
+    if (threadIdx.x == 0) {
+        out[0] = sc->total;
+        out[1] = sc->overflow;
+        out[2] = n;
+    }
+}
+
+// A batch's integrand values f [n][m]: component 0 into f0 (unless NULL) and
+// *nan |= 1 where any is a NaN, in one pass bound by the read (four library
+// launches before, one with a flag per value).
+__global__ __launch_bounds__(256) void values_kernel(const double* f, int64_t n, int m, double* f0, int32_t* nan) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x, tot = n * m;
+    int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t row = e / m, srow = stride / m;
+    int col = (int)(e - row * m), scol = (int)(stride - srow * m);
+    bool bad = false;
+    for (; e < tot; e += stride) {
+        const double v = f[e];
+        bad |= v != v;
+        if (f0 && col == 0) f0[row] = v;
+        row += srow;
+        col += scol;
+        if (col >= m) {
+            col -= m;
+            ++row;
+        }
+    }
+    if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(nan, 1);
+}
+
 template <bool R32>
 static auto sample_kernel_of(int dim) {
     switch (dim) {
@@ -1299,6 +1360,29 @@ extern "C" int vgx_iter_begin(vgx_ctx* ctx, const vgx_config* c, vgx_state* st, 
         *total_host = (int64_t)tmp.total;
     }
     return VGX_OK;
+}
+
+extern "C" int vgx_iter_batches(vgx_ctx* ctx, const vgx_config* c, vgx_state* st, int64_t min_batch, int max,
+                                int64_t* out, void* stream) {
+    if (!ctx || !c || !st || !out || min_batch < 1 || max < 1 || max > 4096) return VGX_EINVAL;
+    hipStream_t s = (hipStream_t)stream;
+    Run R;
+    int rc = prepare(ctx, c, st, &R);
+    if (rc) return rc;
+    int64_t* d = (int64_t*)R.fparams;  // (no integrand parameters between vgx_iter_begin and a batch)
+    hipLaunchKernelGGL(batch_cuts_kernel, dim3(1), dim3(256), 0, s, (const uint32_t*)ctx->off.ptr,
+                       (uint32_t)c->nhcube, (uint64_t)min_batch, max, (const Scalars*)R.sc, d);
+    if ((rc = check_launch())) return rc;
+    VGX_HIP(hipMemcpyAsync(out, d, (3 + 2 * (size_t)max) * 8, hipMemcpyDeviceToHost, s));
+    VGX_HIP(hipStreamSynchronize(s));
+    return out[1] || out[2] < 0 ? VGX_ERANGE : VGX_OK;
+}
+
+extern "C" int vgx_iter_values(const double* f, int64_t n, int m, double* f0, int32_t* nan, void* stream) {
+    if (!f || !nan || n < 1 || m < 1) return VGX_EINVAL;
+    const int64_t b = std::min<int64_t>((n * m + 1023) / 1024, 4096);
+    hipLaunchKernelGGL(values_kernel, dim3((unsigned)b), dim3(256), 0, (hipStream_t)stream, f, n, m, f0, nan);
+    return check_launch();
 }
 
 extern "C" int vgx_iter_sample(vgx_ctx* ctx, const vgx_config* c, vgx_state* st, int it, int64_t h0,

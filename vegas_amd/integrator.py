@@ -612,6 +612,28 @@ class Integrator:
         call.layout = None
         return call
 
+    def _begin_staged(self, torch, cfg, st):
+        """Allocate a staged iteration: its number of points and its batches
+        [(h0, h1, p0, p1), ...].  The device cuts them (the strata counts of a
+        large run took longer to copy and sum on the host than the sampler),
+        unless they may be more than its limit of 4096."""
+        L, cx, sp = _lib.lib(), _lib.ctx(), _lib.stream_ptr()
+        most = 0
+        if 1 <= self.min_neval_batch < 2 ** 62:
+            mnb = math.ceil(self.min_neval_batch)
+            most = (self.neval + self.nhcube * int(self.min_neval_hcube) + 2) // mnb + 2
+        if not 1 <= most <= 4096:
+            nh = torch.empty(self.nhcube, dtype=torch.int32, device='cuda')
+            total = C.c_int64()
+            _lib.check(L.vgx_iter_begin(cx, C.byref(cfg), C.byref(st), 0, _lib.ptr(nh), C.byref(total), sp),
+                       'iter_begin')
+            return int(total.value), _geometry.batches(nh.cpu().numpy(), self.min_neval_batch)
+        out = np.empty(3 + 2 * most, np.int64)
+        _lib.check(L.vgx_iter_begin(cx, C.byref(cfg), C.byref(st), 0, None, None, sp), 'iter_begin')
+        _lib.check(L.vgx_iter_batches(cx, C.byref(cfg), C.byref(st), mnb, most, out.ctypes.data, sp), 'iter_begin')
+        cuts = [(0, 0)] + [tuple(c) for c in out[3:3 + 2 * out[2]].reshape(-1, 2).tolist()]
+        return int(out[0]), [(a[0], b[0], a[1], b[1]) for a, b in zip(cuts, cuts[1:])]
+
     def _probe_layout(self, torch, std):
         """Output structure of a Python integrand: one call on a batch of one
         point (the centre of the y box) with jac = 1, as the reference's
@@ -626,26 +648,23 @@ class Integrator:
         L = _lib.lib()
         st, bufs = self._state(torch, 1)
         cfg = self._config(1, self._rng_iter, prec)
-        nh = torch.empty(self.nhcube, dtype=torch.int32, device='cuda')
-        total = C.c_int64()
         cx, sp = _lib.ctx(), _lib.stream_ptr()
         m = std.layout[-1][3] if std.layout else 1
         multi = bool(getattr(std, 'multi', m > 1))
         corr = 1 if self.correlate_integrals else 0
         if multi:
             # per iteration: mean[m] and the covariance lower triangle (or
-            # the variances), double-double pairs
+            # the variances), double-double pairs, and the status word
             npairs = m * (m + 1) // 2 if corr else m
-            acc = torch.zeros(2 * (m + npairs), dtype=torch.float64, device='cuda')
-            cstat = torch.zeros(1, dtype=torch.int32, device='cuda')
-        _lib.check(L.vgx_iter_begin(cx, C.byref(cfg), C.byref(st), 0, _lib.ptr(nh), C.byref(total),
-                                    sp), 'iter_begin')
-        ubuf = self._uniforms(torch, cfg, total.value)
+            acc = torch.zeros(2 * (m + npairs) + 1, dtype=torch.float64, device='cuda')
+            cstat = acc[-1:].view(torch.int32)
+        total, batches = self._begin_staged(torch, cfg, st)
+        ubuf = self._uniforms(torch, cfg, total)
         # NaN in any component: flagged on the device batch by batch and read
         # once, before the iteration closes (no adapt), instead of a host
         # synchronisation per batch (pyx:2133-2134 raises at the batch)
-        nan_seen = torch.zeros((), dtype=torch.bool, device='cuda')
-        for h0, h1, p0, p1 in _geometry.batches(nh.cpu().numpy(), self.min_neval_batch):
+        nan_seen = torch.zeros(1, dtype=torch.int32, device='cuda')
+        for h0, h1, p0, p1 in batches:
             n = p1 - p0
             self._draw(torch, ubuf, p0, p1)
             x = torch.empty((n, self.dim), dtype=torch.float64, device='cuda')
@@ -657,16 +676,17 @@ class Integrator:
             f = std(x, jac)
             if f.shape[1] != m:
                 raise ValueError('integrand output changed shape (%d values, not %d)' % (f.shape[1], m))
-            nan_seen |= torch.isnan(f).any()
             # component 0 steers sigf and the training data (pyx:2173, 2185)
-            f0 = f[:, 0].contiguous()
+            f0 = f if m == 1 else torch.empty(n, dtype=torch.float64, device='cuda')
+            _lib.check(L.vgx_iter_values(_lib.ptr(f), n, m, None if m == 1 else _lib.ptr(f0), _lib.ptr(nan_seen), sp),
+                       'iter_values')
             _lib.check(L.vgx_iter_accumulate(cx, C.byref(cfg), C.byref(st), 0, h0, h1, p0, p1,
                                              _lib.ptr(f0), sp), 'iter_accumulate')
             if multi:
                 _lib.check(L.vgx_iter_accumulate_cov(cx, C.byref(cfg), h0, h1, p0, p1, _lib.ptr(f), _lib.ptr(w),
                                                      m, corr, _lib.ptr(acc), _lib.ptr(cstat), sp),
                            'iter_accumulate_cov')
-        if bool(nan_seen):
+        if int(nan_seen.item()):
             raise ValueError('integrand evaluates to nan')
         _lib.check(L.vgx_iter_end(cx, C.byref(cfg), C.byref(st), 0, sp), 'iter_end')
         status, res = self._read_back(bufs)
@@ -674,11 +694,11 @@ class Integrator:
         if not multi:
             self._finish(status, res, 1, result)
             return
-        if int(cstat.item()):
-            _lib.check(int(cstat.item()), 'iter_accumulate_cov')
+        a = acc.cpu().numpy()
+        _lib.check(int(a[-1:].view(np.int32)[0]), 'iter_accumulate_cov')
         scalar = RAvg(weighted=self.adapt)
         self._finish(status, res, 1, scalar)
-        a = acc.cpu().numpy()
+        a = a[:-1]
         mean = a[0:2 * m:2] + a[1:2 * m:2]
         cv = a[2 * m::2] + a[2 * m + 1::2]
         cov = np.zeros((m, m))
@@ -700,16 +720,11 @@ class Integrator:
         L = _lib.lib()
         st, bufs = self._state(torch, 1)
         cfg = self._config(1, self._rng_iter, self._precision(False))
-        nh = torch.empty(self.nhcube, dtype=torch.int32, device='cuda')
-        total = C.c_int64()
         cx, sp = _lib.ctx(), _lib.stream_ptr()
-        _lib.check(L.vgx_iter_begin(cx, C.byref(cfg), C.byref(st), 0, _lib.ptr(nh), C.byref(total), sp),
-                   'iter_begin')
+        self.last_neval, batches = self._begin_staged(torch, cfg, st)
         self._rng_iter += 1
-        nhh = nh.cpu().numpy()
-        self.last_neval = int(total.value)
-        ubuf = self._uniforms(torch, cfg, total.value)
-        for h0, h1, p0, p1 in _geometry.batches(nhh, self.min_neval_batch):
+        ubuf = self._uniforms(torch, cfg, self.last_neval)
+        for h0, h1, p0, p1 in batches:
             n = p1 - p0
             self._draw(torch, ubuf, p0, p1)
             x = torch.empty((n, self.dim), dtype=torch.float64, device='cuda')
