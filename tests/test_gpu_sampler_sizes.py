@@ -190,3 +190,28 @@ def test_batch_values(va, n, m):
     f[n - 1, m - 1] = float('nan')
     run(None)
     assert int(flag.item()) == 1
+
+
+@pytest.mark.parametrize("nhcube", [992, 1024, 1056, 8190, 8281])
+@pytest.mark.parametrize("beta", [0.75, 0.0])
+def test_hcube_counts(va, orc, nhcube, beta):
+    """Allocation by one workgroup (up to 8192 hcubes) and by many, on both
+    sides of its 1024 threads, with adaptive and equal counts."""
+    kw = dict(neval=(8 if beta else 2) * (nhcube + 1), seed=37, beta=beta)
+    c = [[0.45, 0.55]]
+    f, fo = va.GaussianMixture([1.0], [30.0], c), orc.GaussMix([1.0], [30.0], c)
+    integ = va.Integrator([[0, 1]] * 2, precision='f64', exact=True, **kw)
+    assert integ.nhcube == nhcube
+    r = integ(f, nitn=3)
+    o = orc.OracleIntegrator([(0, 1)] * 2, **kw)
+    mean, var, nev = o.run(fo, 3)
+    for k, m in enumerate(r.itn_results):
+        assert abs(m.mean - mean[k]) <= 1e-12 * abs(mean[k])
+        assert abs(m.var - var[k]) <= 1e-10 * var[k]
+    assert integ.last_neval == nev[-1]
+    # the counts of the next iteration, whole numbers, from the weights themselves
+    h = np.concatenate([p[2] for p in integ.random_batch(yield_hcube=True)])
+    want = np.full(nhcube, 2) if not beta else np.minimum(
+        (integ.sigf * (integ.neval_frac * integ.neval / integ.sum_sigf)).astype(np.int64) + integ.min_neval_hcube,
+        integ.max_neval_hcube)
+    np.testing.assert_array_equal(np.bincount(h, minlength=nhcube), want)

@@ -47,6 +47,20 @@ __global__ void iter_init_kernel(IterGeom g, double* sum_f, double* n_f, Scalars
 // The iteration's training data start empty (AdaptiveMap.clear, pyx:596-599):
 // they are cleared here rather than after the adapt reads them, so the last
 // iteration's histogram stays readable after a run.
+// n_h of hcube h, and sigf's reset where the previous iteration found its sum 0.
+__device__ __forceinline__ int32_t alloc_one(const IterGeom& g, double* sigf, int64_t h, int reset, double neval_sigf) {
+    if (!g.adaptive_sampler) return g.avg_nh;
+    double sv = 1.0;
+    if (reset)
+        sigf[h] = 1.0;
+    else
+        sv = sigf[h];
+    double v = sv * neval_sigf;
+    v = v < 2147483647.0 ? v : 2147483647.0;
+    const int64_t nn = (int64_t)(int32_t)v + g.nmin;
+    return (int32_t)(nn > g.nmax ? g.nmax : nn);
+}
+
 __global__ __launch_bounds__(kAllocThreads) void alloc_kernel(IterGeom g, double* sigf,
                                                               const double* sum_sigf, int32_t* nh,
                                                               uint64_t* stat, const Scalars* sc,
@@ -70,24 +84,10 @@ __global__ __launch_bounds__(kAllocThreads) void alloc_kernel(IterGeom g, double
     for (int i = 0; i < kAllocItems; ++i) {
         const int64_t h = base + (int64_t)i * kAllocThreads + threadIdx.x;
         if (h >= g.nhcube) break;
-        int32_t n;
+        const int32_t n = alloc_one(g, sigf, h, reset, neval_sigf);
         if (g.adaptive_sampler) {
-            double sv;
-            if (reset) {
-                sv = 1.0;
-                sigf[h] = 1.0;
-            } else {
-                sv = sigf[h];
-            }
-            double v = sv * neval_sigf;
-            v = v < 2147483647.0 ? v : 2147483647.0;
-            int64_t nn = (int64_t)(int32_t)v + g.nmin;
-            if (nn > g.nmax) nn = g.nmax;
-            n = (int32_t)nn;
             mn = n < mn ? n : mn;
             mx = n > mx ? n : mx;
-        } else {
-            n = g.avg_nh;
         }
         nh[h] = n;
         sum += (uint64_t)n;
@@ -227,6 +227,98 @@ __global__ __launch_bounds__(kAllocThreads) void offsets_kernel(IterGeom g, cons
         if (h < g.nhcube) off[h] = ln[lds_pad(i)];
     }
     if (last && threadIdx.x == 0) off[g.nhcube] = (uint32_t)tot;
+}
+
+// alloc_kernel and offsets_kernel by one workgroup, for up to kOneMax hcubes:
+// the same numbers from one launch.  Bound by latency.  Ten iterations in 2 to
+// 4 dimensions: 121 hcubes 505 -> 490 us, 1225 to 4608 hcubes 5-9 % less;
+// with 12,100 hcubes one workgroup loses 2 % to the two launches' many.
+constexpr int kOneThreads = 1024, kOneMax = kOneThreads * 8;
+__global__ __launch_bounds__(kOneThreads) void alloc_offsets_kernel(IterGeom g, double* sigf, const double* sum_sigf,
+                                                                    int32_t* nh, Scalars* sc, double* sum_f,
+                                                                    double* n_f, uint32_t* off, int32_t* tile_h,
+                                                                    uint64_t capacity) {
+    __shared__ uint32_t one_n[kOneMax + kOneMax / 8];
+    __shared__ uint64_t wsum[kOneThreads / 64];
+    __shared__ int32_t wmm[2 * (kOneThreads / 64)];
+    if (sc->status) return;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nhc = (int)g.nhcube;
+    if (g.train_points || g.train_errors) {
+        const int tot = g.dim * g.nb;
+        for (int i = threadIdx.x; i < tot; i += kOneThreads) {
+            sum_f[i] = 0.0;
+            n_f[i] = kTiny;
+        }
+    }
+    const int reset = sc->reset_sigf;
+    const double ss = *sum_sigf;
+    const double neval_sigf = (g.beta > 0 && ss > 0 && g.adaptive_sampler) ? g.neval_frac * g.neval / ss : 0.0;
+    const int items = (nhc + kOneThreads - 1) / kOneThreads;
+    int32_t mn = g.nmin, mx = g.nmin;
+    for (int i = 0; i < items; ++i) {
+        const int h = i * kOneThreads + (int)threadIdx.x;
+        int32_t n = 0;
+        if (h < nhc) {
+            n = alloc_one(g, sigf, h, reset, neval_sigf);
+            nh[h] = n;
+            if (g.adaptive_sampler) {
+                mn = min(mn, n);
+                mx = max(mx, n);
+            }
+        }
+        one_n[lds_pad(h)] = (uint32_t)n;
+    }
+    __syncthreads();
+    uint64_t run = 0;
+    for (int i = 0; i < items; ++i) run += one_n[lds_pad(threadIdx.x * items + i)];
+    uint64_t incl = run;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint64_t t = __shfl_up(incl, o, kWave);
+        if (lane >= o) incl += t;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        mn = min(mn, __shfl_xor(mn, o, kWave));
+        mx = max(mx, __shfl_xor(mx, o, kWave));
+    }
+    if (lane == 63) {
+        wsum[w] = incl;
+        wmm[2 * w] = mn;
+        wmm[2 * w + 1] = mx;
+    }
+    __syncthreads();
+    uint64_t wbase = 0, tot = 0;
+    for (int k = 0; k < kOneThreads / 64; ++k) {
+        if (k < w) wbase += wsum[k];
+        tot += wsum[k];
+        mn = min(mn, wmm[2 * k]);
+        mx = max(mx, wmm[2 * k + 1]);
+    }
+    const bool ok = tot <= capacity && tot < 0xFFFFFFFFull;
+    if (threadIdx.x == 0) {
+        sc->overflow = ok ? 0u : 1u;
+        sc->total = ok ? (uint32_t)tot : 0u;
+        sc->nh_min = mn;
+        sc->nh_max = mx;
+        sc->b_p0 = 0;
+        sc->b_p1 = sc->total;
+        sc->b_h0 = 0;
+        sc->b_h1 = (uint32_t)g.nhcube;
+        sc->b_ntiles = (sc->total + kT - 1) / kT;
+    }
+    if (!ok) return;
+    uint32_t lo = (uint32_t)(wbase + incl - run);
+    for (int i = 0; i < items; ++i) {
+        const int h = threadIdx.x * items + i;
+        const uint32_t hi = lo + one_n[lds_pad(h)];
+        for (uint32_t t = (lo + kT - 1) / kT; t < (hi + kT - 1) / kT; ++t) tile_h[t] = (int32_t)h;
+        one_n[lds_pad(h)] = lo;  // (a hcube beyond the last has no points)
+        lo = hi;
+    }
+    __syncthreads();
+    for (int h = threadIdx.x; h < nhc; h += kOneThreads) off[h] = one_n[lds_pad(h)];
+    if (threadIdx.x == 0) off[nhc] = (uint32_t)tot;
 }
 
 // Staged batches: tiles of points [p0, p1) covering hcubes [h0, h1).
@@ -1159,6 +1251,12 @@ static int run_init(Run* R, vgx_state* st, hipStream_t s, int new_run) {
 
 static int alloc_kernels(vgx_ctx* ctx, Run* R, vgx_state* st, hipStream_t s) {
     const IterGeom& g = R->g;
+    if (g.nhcube <= kOneMax) {
+        hipLaunchKernelGGL(alloc_offsets_kernel, dim3(1), dim3(kOneThreads), 0, s, g, st->sigf,
+                           (const double*)st->sum_sigf, R->nh, R->sc, st->sum_f, st->n_f, (uint32_t*)ctx->off.ptr,
+                           (int32_t*)ctx->tile_h.ptr, R->cap);
+        return check_launch();
+    }
     hipLaunchKernelGGL(alloc_kernel, dim3(R->nblk_alloc), dim3(kAllocThreads), 0, s, g, st->sigf,
                        (const double*)st->sum_sigf, R->nh, R->stat, (const Scalars*)R->sc, st->sum_f, st->n_f);
     hipLaunchKernelGGL(offsets_kernel, dim3(R->nblk_alloc), dim3(kAllocThreads), 0, s, g,
