@@ -13,7 +13,7 @@
 //                         (pyx:2392-2410); resets the per-iteration scalars
 //   adapt                 AdaptiveMap.adapt(alpha) in place (pyx:2216-2217);
 //                         clears the training data for the next iteration
-// The run starts with iter_init and ends with sigf_reset.
+// The run starts with run_begin and ends with sigf_reset.
 #include <math.h>
 #include <string.h>
 
@@ -23,30 +23,32 @@
 
 namespace vgx {
 
-// Resets the per-iteration scalars (the NaN flag too on a new run) and
-// clears the training data (AdaptiveMap.clear, pyx:596-599).
-__global__ void iter_init_kernel(IterGeom g, double* sum_f, double* n_f, Scalars* sc, int new_run) {
+// The start of a run: the axes' constants, the scalars (the NaN flag is sticky
+// within one run only), empty training data (AdaptiveMap.clear, pyx:596-599)
+// and the FP32 copies p32 = A [nc] | B [nc] | c [ncc] of an integrand's
+// parameters (none: nc = ncc = 0).  One launch (five before: 10 us of a call
+// of 455 with ten iterations in two dimensions).
+__global__ __launch_bounds__(256) void run_begin_kernel(IterGeom g, AxisC* axes, double* sum_f, double* n_f,
+                                                        Scalars* sc, const double* A, const double* B, const double* c,
+                                                        int nc, int ncc, float* p32) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
     const int tot = g.dim * g.nb;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < tot; i += gridDim.x * blockDim.x) {
+    for (int i = t; i < tot; i += stride) {
         sum_f[i] = 0.0;
         n_f[i] = kTiny;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        if (new_run) {
-            sc->status = 0;  // the NaN flag is sticky within one run only
-            sc->reset_sigf = 0;
-        }
+    for (int i = t; i < 2 * nc + ncc; i += stride)
+        p32[i] = (float)(i < nc ? A[i] : i < 2 * nc ? B[i - nc] : c[i - 2 * nc]);
+    if (t < g.dim) axes[t] = make_axis(g, t);
+    if (t == 0) {
+        sc->status = 0;
+        sc->reset_sigf = 0;
         for (int k = 0; k < 6; ++k) sc->acc[k] = 0.0;
         sc->overflow = 0;
     }
 }
 
 // ------------------------------------------------------------ allocation ----
-// n_h = min(int(sigf_h * neval_sigf) + nmin, max(nmax, nmin))   (pyx:1696-1698)
-// Per-workgroup total, min and max go to stat[3 * blockIdx.x + {0,1,2}].
-// The iteration's training data start empty (AdaptiveMap.clear, pyx:596-599):
-// they are cleared here rather than after the adapt reads them, so the last
-// iteration's histogram stays readable after a run.
 // n_h of hcube h, and sigf's reset where the previous iteration found its sum 0.
 __device__ __forceinline__ int32_t alloc_one(const IterGeom& g, double* sigf, int64_t h, int reset, double neval_sigf) {
     if (!g.adaptive_sampler) return g.avg_nh;
@@ -61,6 +63,11 @@ __device__ __forceinline__ int32_t alloc_one(const IterGeom& g, double* sigf, in
     return (int32_t)(nn > g.nmax ? g.nmax : nn);
 }
 
+// n_h = min(int(sigf_h * neval_sigf) + nmin, max(nmax, nmin))   (pyx:1696-1698)
+// Per-workgroup total, min and max go to stat[3 * blockIdx.x + {0,1,2}].
+// The iteration's training data start empty (AdaptiveMap.clear, pyx:596-599):
+// they are cleared here rather than after the adapt reads them, so the last
+// iteration's histogram stays readable after a run.
 __global__ __launch_bounds__(kAllocThreads) void alloc_kernel(IterGeom g, double* sigf,
                                                               const double* sum_sigf, int32_t* nh,
                                                               uint64_t* stat, const Scalars* sc,
@@ -827,10 +834,6 @@ __global__ void axes_init_kernel(IterGeom g, AxisC* axes) {
     if (threadIdx.x < (unsigned)g.dim) axes[threadIdx.x] = make_axis(g, threadIdx.x);
 }
 
-__global__ void to_float_kernel(const double* a, float* b, int n) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) b[i] = (float)a[i];
-}
-
 // out[0]: the least integer e (as a float) with every A[i] < 2^e; infinity
 // when one is negative or not finite.
 __global__ __launch_bounds__(1024) void max_exponent_kernel(const double* A, int n, float* out) {
@@ -1235,17 +1238,29 @@ static void set_iter(Run* R, const vgx_config* c, int it) {
     R->g.itn = (uint32_t)it;
 }
 
+// Whether FP32 copies of the integrand's parameters are taken, and fit.
+static int fcn_params32(const vgx_config* c, const vgx_integrand* f) {
+    if (c->precision != VGX_PREC_F32 || (f->kind != VGX_FCN_GAUSSMIX && f->kind != VGX_FCN_DIAGRIDGE)) return VGX_EINVAL;
+    if (f->ncomp < 1 || !f->A || !f->B || !f->c) return VGX_EINVAL;
+    const int64_t nc = f->ncomp, ncc = f->kind == VGX_FCN_GAUSSMIX ? nc * c->dim : nc;
+    return (2 * nc + ncc) * 4 > 1024 * 1024 ? VGX_ERANGE : VGX_OK;
+}
 static int init_axes(Run* R, hipStream_t s) {
     hipLaunchKernelGGL(axes_init_kernel, dim3(1), dim3(64), 0, s, R->g, R->axes);
     return check_launch();
 }
 
-static int run_init(Run* R, vgx_state* st, hipStream_t s, int new_run) {
+// Axes and state of a run; f: the integrand whose FP32 parameters it takes.
+static int run_begin(Run* R, const vgx_config* c, const vgx_integrand* f, vgx_state* st, hipStream_t s) {
     const IterGeom& g = R->g;
-    const int tot = g.dim * g.nb;
-    const int nb = (tot + 255) / 256 < 64 ? (tot + 255) / 256 : 64;
-    hipLaunchKernelGGL(iter_init_kernel, dim3(nb > 0 ? nb : 1), dim3(256), 0, s, g, st->sum_f, st->n_f,
-                       R->sc, new_run);
+    int nc = 0, ncc = 0;
+    if (f && fcn_params32(c, f) == VGX_OK) {
+        nc = f->ncomp;
+        ncc = f->kind == VGX_FCN_GAUSSMIX ? nc * c->dim : nc;
+    }
+    const int tot = std::max(g.dim * g.nb, 2 * nc + ncc), nb = std::min((tot + 255) / 256, 64);
+    hipLaunchKernelGGL(run_begin_kernel, dim3(nb > 0 ? nb : 1), dim3(256), 0, s, g, R->axes, st->sum_f, st->n_f, R->sc,
+                       nc ? f->A : nullptr, nc ? f->B : nullptr, nc ? f->c : nullptr, nc, ncc, R->fparams);
     return check_launch();
 }
 
@@ -1369,7 +1384,7 @@ static int run_end(Run* R, const vgx_config* c, vgx_state* st, hipStream_t s) {
 }
 
 static int make_fcn_and_run(vgx_ctx* ctx, Run* R, const vgx_config* c, const vgx_integrand* f,
-                            hipStream_t s, int timed, int convert, int reduce) {
+                            hipStream_t s, int timed, int first, int reduce) {
     const bool f32 = c->precision == VGX_PREC_F32;
     if (f->kind == VGX_FCN_BUFFER) {
         if (f32) {
@@ -1382,19 +1397,14 @@ static int make_fcn_and_run(vgx_ctx* ctx, Run* R, const vgx_config* c, const vgx
     if (f->kind == VGX_FCN_GAUSSMIX || f->kind == VGX_FCN_DIAGRIDGE) {
         const int nc = f->ncomp;
         if (nc < 1 || !f->A || !f->B || !f->c) return VGX_EINVAL;
-        const int ncc = f->kind == VGX_FCN_GAUSSMIX ? nc * c->dim : nc;
         if (f32) {
-            if ((size_t)(2 * nc + ncc) * 4 > 1024 * 1024) return VGX_ERANGE;
+            const int rc = fcn_params32(c, f);
+            if (rc) return rc;
             float* A = R->fparams;
             float* B = A + nc;
             float* C = B + nc;
-            if (convert) {
-                hipLaunchKernelGGL(to_float_kernel, dim3(64), dim3(256), 0, s, f->A, A, nc);
-                hipLaunchKernelGGL(to_float_kernel, dim3(64), dim3(256), 0, s, f->B, B, nc);
-                hipLaunchKernelGGL(to_float_kernel, dim3(64), dim3(256), 0, s, f->c, C, ncc);
-            }
             if (f->kind == VGX_FCN_GAUSSMIX && many_pays(nc, c->dim, c->neval)) {
-                if (convert) hipLaunchKernelGGL(max_exponent_kernel, dim3(1), dim3(1024), 0, s, f->A, nc, R->fmax);
+                if (first) hipLaunchKernelGGL(max_exponent_kernel, dim3(1), dim3(1024), 0, s, f->A, nc, R->fmax);
                 GaussMany32 fn{nc, A, B, C, R->fmax};
                 return accumulate_kernels(ctx, R, fn, s, timed, reduce);
             }
@@ -1427,8 +1437,7 @@ extern "C" int vgx_integrate(vgx_ctx* ctx, const vgx_config* c, const vgx_integr
     Run R;
     int rc = prepare(ctx, c, st, &R);
     if (rc) return rc;
-    if ((rc = init_axes(&R, s))) return rc;
-    if ((rc = run_init(&R, st, s, 1))) return rc;
+    if ((rc = run_begin(&R, c, c->nitn > 0 ? f : nullptr, st, s))) return rc;
     for (int it = 0; it < c->nitn; ++it) {
         set_iter(&R, c, it);
         if ((rc = alloc_kernels(ctx, &R, st, s))) return rc;
@@ -1445,9 +1454,8 @@ extern "C" int vgx_iter_begin(vgx_ctx* ctx, const vgx_config* c, vgx_state* st, 
     Run R;
     int rc = prepare(ctx, c, st, &R);
     if (rc) return rc;
-    if ((rc = init_axes(&R, s))) return rc;
     set_iter(&R, c, it);
-    if ((rc = run_init(&R, st, s, 1))) return rc;
+    if ((rc = run_begin(&R, c, nullptr, st, s))) return rc;
     if ((rc = alloc_kernels(ctx, &R, st, s))) return rc;
     if (n_h) VGX_HIP(hipMemcpyAsync(n_h, R.nh, (size_t)c->nhcube * 4, hipMemcpyDeviceToDevice, s));
     if (total_host) {
