@@ -3,7 +3,7 @@
 // src/vegas/_vegas.pyx:2136-2183 with correlate_integrals on or off.
 //
 // Work item: (hcube h, component pair q, or all pairs for m <= 6).  A thread
-// owns a strided set of the batch's hcubes (the long ones are shared by its
+// owns a strided set of the batch's hcubes (longer ones are shared by its wave or
 // workgroup); for each hcube it makes the reference's two passes over the
 // hcube's points: S = sum w f (per component), then the deviations
 // d = w f - S/n with the EPSILON guard (a guarded deviation adds
