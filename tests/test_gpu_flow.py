@@ -302,3 +302,25 @@ def test_ridge_component_counts(torch, nc):
     want = f1.double().cpu().numpy() / one(xs) * f(xs)
     np.testing.assert_allclose(fj.double().cpu().numpy(), want, rtol=1e-4, atol=0)
     np.testing.assert_allclose(flow.eval_fcn(f, x).double().cpu().numpy(), f(xs), rtol=1e-4, atol=0)
+
+
+@pytest.mark.parametrize("n", [1, 300000])
+def test_largest_uniform(torch, orc, n):
+    """The largest 24-bit uniform, 1 - 2^-25, is no float: it must not become
+    z = 1, whose f J is a NaN that reaches the sums.  Sample 286585 has it on
+    axis 3.  The untrained flow is the identity: x = z and f J = f, up to the
+    logs of u (16.6 there, an error of 2^-20 in it: held to 1e-5)."""
+    import vegas_amd as va
+    from vegas_amd.flow import CouplingFlow
+    i, dim = 286585, 5
+    z = (np.concatenate([orc.philox([i, 0, 2, g], [7, 0]) for g in range(2)])[:dim].astype(np.int64) >> 8) + 0.5
+    assert z[3] == 2 ** 24 - 0.5
+    f = va.DiagonalRidge([1.0], [0.5], [0.4], dim)
+    base, at = (i, 0) if n == 1 else (0, i)
+    s1, s2, x, fj = CouplingFlow(dim, 4, seed=3).sample(f, n, seed=7, iteration=2, base=base, keep_points=True)
+    assert torch.isfinite(fj).all() and np.isfinite(s1) and np.isfinite(s2)
+    np.testing.assert_allclose(x[at, :dim].cpu().numpy(), z / 2 ** 24, rtol=1e-5)
+    np.testing.assert_allclose(fj[at].item(), f(z[None] / 2 ** 24)[0], rtol=1e-5)
+    # sums are of f J before the rounding to FP32 (2^-24 a term)
+    np.testing.assert_allclose(s1, fj.double().sum().item(), rtol=6e-8, equal_nan=False)
+    np.testing.assert_allclose(s2, (fj.double() ** 2).sum().item(), rtol=1.2e-7, equal_nan=False)

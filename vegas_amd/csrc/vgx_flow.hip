@@ -440,7 +440,10 @@ __global__ __launch_bounds__(kFlowThreads) void flow_sample_kernel(FlowArgs f, F
             f32x4_t uq;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float z = (float)(ws[i] >> 8) * (1.0f / 16777216.0f) + (1.0f / 33554432.0f);
+                // below 1: the last of the 2^24 values rounds to it, and its
+                // logit and Jacobian would be infinite, f J a NaN
+                const float z = fminf((float)(ws[i] >> 8) * (1.0f / 16777216.0f) + (1.0f / 33554432.0f),
+                                      1.0f - 1.0f / 16777216.0f);
                 const float l0 = __logf(z), l1 = __logf(1.0f - z);
                 uq[i] = l0 - l1;
                 if (4 * g + i < f.D) l -= l0 + l1;  // dz/du = z (1 - z)
