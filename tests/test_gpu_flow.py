@@ -324,3 +324,24 @@ def test_largest_uniform(torch, orc, n):
     # sums are of f J before the rounding to FP32 (2^-24 a term)
     np.testing.assert_allclose(s1, fj.double().sum().item(), rtol=6e-8, equal_nan=False)
     np.testing.assert_allclose(s2, (fj.double() ** 2).sum().item(), rtol=1.2e-7, equal_nan=False)
+
+
+@pytest.mark.parametrize("waves,tiles", [(4, 2), (8, 2), (12, 2), (12, 6)])
+@pytest.mark.parametrize("over", [-15, 0, 1, 17, 33])
+def test_sums_of_other_lanes_values(torch, waves, tiles, over):
+    """The lane that sums a sample reads f and log J that other lanes of its
+    wave stored: f J of every sample at each launch shape, its tiles full and
+    cut, and over more than one pass.  The untrained flow is the identity, so
+    f J is f at the sample's own point, up to the logs (10 terms of at most 17,
+    2^-24 each: 1e-5; held to 1e-4)."""
+    import vegas_amd as va
+    from vegas_amd.flow import CouplingFlow
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    n = (2 if tiles > 2 else 1) * waves * tiles * 16 * cus + over
+    f = va.DiagonalRidge([1.0, 3.0], [2.0, 20.0], [0.3, 0.6], 5)
+    flow = CouplingFlow(5, 2, seed=3)
+    s1, s2, x, fj = flow.sample(f, n, seed=11, iteration=1, keep_points=True)
+    fx = flow.eval_fcn(f, x).double()
+    assert ((fj.double() - fx).abs() <= 1e-4 * fx).all()
+    np.testing.assert_allclose(s1, fj.double().sum().item(), rtol=6e-8, equal_nan=False)
+    np.testing.assert_allclose(s2, (fj.double() ** 2).sum().item(), rtol=1.2e-7, equal_nan=False)

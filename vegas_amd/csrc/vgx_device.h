@@ -155,6 +155,15 @@ __device__ inline DD wave_sum_dd(DD v) {
     return v;
 }
 
+// Between the LDS stores of a wave's lanes and its other lanes' loads (or the
+// other way round).  A wave's LDS instructions execute in order: this only
+// keeps the compiler from moving them across.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---- DPP lane movement (gfx9 encodings): another lane's value through the
 // VALU's data-parallel-primitive path instead of an LDS permute.
 constexpr int kDppRowShl = 0x100;     // + n: row_shl:n (within 16-lane rows)

@@ -512,7 +512,8 @@ __global__ __launch_bounds__(kFlowThreads) void flow_sample_kernel(FlowArgs f, F
                 }
             }
         }
-        // the sums, a sample per lane
+        // the sums, a sample per lane, from what other lanes stored
+        wave_lds_fence();
         for (int r = 0; r < a.tiles; r += 4) {
             const int q = r + (lane >> 4);
             const uint64_t sl = pb + (uint64_t)(wave * a.tiles + q) * 16 + (lane & 15);
@@ -525,6 +526,7 @@ __global__ __launch_bounds__(kFlowThreads) void flow_sample_kernel(FlowArgs f, F
                 if (a.xout) a.fout[sl] = (float)fj;
             }
         }
+        wave_lds_fence();  // read before the next pass stores
     }
     s1 = wave_sum_dd(s1);
     s2 = wave_sum_dd(s2);
