@@ -345,3 +345,44 @@ def test_sums_of_other_lanes_values(torch, waves, tiles, over):
     assert ((fj.double() - fx).abs() <= 1e-4 * fx).all()
     np.testing.assert_allclose(s1, fj.double().sum().item(), rtol=6e-8, equal_nan=False)
     np.testing.assert_allclose(s2, (fj.double() ** 2).sum().item(), rtol=1.2e-7, equal_nan=False)
+
+
+@pytest.mark.parametrize("call", ["sample", "eval"])
+def test_parameters_are_the_callers_after_the_call(torch, call):
+    """A call that does not wait for its kernel has read the integrand's arrays
+    when it returns: another stream may then overwrite them, with the call's
+    stream still busy, and the values are those of the arrays before.  The next
+    call, on that other stream, does not disturb them either."""
+    import vegas_amd as va
+    from vegas_amd.flow import CouplingFlow
+    flow, n = CouplingFlow(5, 2, seed=3), 20000
+    x = torch.rand((n, 16), dtype=torch.float32, device='cuda')
+    status = torch.zeros(1, dtype=torch.int32, device='cuda')
+
+    def go(f):
+        if call == "eval":
+            return flow.eval_fcn(f, x)
+        return flow.sample(f, n, seed=5, keep_points=True, status=status)[3]
+
+    def integrand():
+        return va.DiagonalRidge([1.0] * 7, [20.0] * 7, np.linspace(0.3, 0.7, 7), 5)
+
+    want, half = go(integrand()).clone(), va.DiagonalRidge([0.5], [2.0], [0.5], 5)
+    want2 = go(half).clone()
+    f = integrand()
+    arrays = f.vgx_integrand(torch, torch.device('cuda'))[1]
+    torch.cuda.synchronize()
+    # (several, as two streams may share a hardware queue)
+    busy, others = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(6)]
+    for other in others:
+        with torch.cuda.stream(busy):
+            torch.cuda._sleep(10 ** 7)
+            got = go(f)
+        with torch.cuda.stream(other):
+            for a in arrays:
+                a.zero_()
+            got2 = go(half)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and torch.equal(got2, want2)
+        for a, v in zip(arrays, f._param_arrays()):
+            a.copy_(torch.as_tensor(v))

@@ -288,6 +288,13 @@ __device__ inline void load_fcn(const FlowFcn& F, int D, float* Lc) {
         Lc[i] = (float)(i < F.ncomp ? F.A[i] : i < 2 * F.ncomp ? F.B[i - F.ncomp] : F.c[i - 2 * F.ncomp]);
 }
 
+// A copy of them that a kernel can read after the caller's arrays are gone:
+// out = A [na] | B [na] | c [nc].
+__global__ __launch_bounds__(256) void flow_hold_kernel(FlowFcn F, int na, int nc, double* out) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < 2 * na + nc; i += gridDim.x * blockDim.x)
+        out[i] = i < na ? F.A[i] : i < 2 * na ? F.B[i - na] : F.c[i - 2 * na];
+}
+
 struct SampleArgs {
     uint64_t n;          // samples
     uint64_t base;       // first sample index (Philox counter)
@@ -1141,7 +1148,9 @@ struct vgx_flow {
     uint16_t* H = nullptr;
     uint16_t* HT = nullptr;
     // per-batch scratch (grown on demand)
-    Scratch saved, u0, logq, c, G, wpart, cpart, spart, misc;
+    Scratch saved, u0, logq, c, G, wpart, cpart, spart, misc, fpar;
+    hipEvent_t held = nullptr;  // fpar has been written
+    hipEvent_t used = nullptr;  // and read
     int step = 0;
 };
 
@@ -1189,7 +1198,9 @@ extern "C" int vgx_flow_create(int dim, int nlayers, const uint32_t* amask, vgx_
     if (hipFuncSetAttribute((const void*)flow_backward_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)lds_bwd()) != hipSuccess ||
         hipFuncSetAttribute((const void*)flow_inverse_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)(lds_layer() + kStateLds)) != hipSuccess) {
+                            (int)(lds_layer() + kStateLds)) != hipSuccess ||
+        hipEventCreateWithFlags(&fl->held, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&fl->used, hipEventDisableTiming) != hipSuccess) {
         vgx_flow_destroy(fl);
         return VGX_EHIP;
     }
@@ -1204,8 +1215,10 @@ extern "C" int vgx_flow_destroy(vgx_flow* fl) {
     for (void* p : ps)
         if (p) (void)hipFree(p);
     Scratch* ss[] = {&fl->saved, &fl->u0, &fl->logq, &fl->c, &fl->G, &fl->wpart, &fl->cpart, &fl->spart,
-                     &fl->misc};
+                     &fl->misc, &fl->fpar};
     for (Scratch* q : ss) q->release();
+    for (hipEvent_t e : {fl->held, fl->used})
+        if (e) (void)hipEventDestroy(e);
     delete fl;
     return VGX_OK;
 }
@@ -1240,8 +1253,8 @@ extern "C" int vgx_flow_get_params(const vgx_flow* fl, float* host, float* grad_
     return VGX_OK;
 }
 
-// The integrand as the kernels read it (its arrays stay the caller's), and
-// its LDS bytes.
+// The integrand as the kernels read it (its arrays are the caller's), and its
+// LDS bytes.
 static int flow_fcn_params(const vgx_flow* fl, const vgx_integrand* fcn, FlowFcn* F, size_t* lds) {
     if (!fcn || (fcn->kind != VGX_FCN_GAUSSMIX && fcn->kind != VGX_FCN_DIAGRIDGE) || fcn->ncomp < 1)
         return VGX_EINVAL;
@@ -1250,6 +1263,32 @@ static int flow_fcn_params(const vgx_flow* fl, const vgx_integrand* fcn, FlowFcn
     *lds = (2 * nc + (fcn->kind == VGX_FCN_GAUSSMIX ? nc * fl->D : nc)) * 4;
     if (*lds > 48 * 1024) return VGX_ERANGE;  // staged in LDS with the layer
     *F = FlowFcn{fcn->kind, fcn->ncomp, fcn->A, fcn->B, fcn->c};
+    return VGX_OK;
+}
+
+// For a call that returns before its kernel has run: the kernel reads a copy of
+// the arrays, and flow_params_held, after its launch, waits until that has been
+// taken, so that the caller may reuse or free them.  (The kernel is then
+// already in the queue: waiting for the copy before the launch would leave
+// the GPU idle for the launch.)  A second stream's copy waits for the first's
+// reader.
+static int flow_hold_params(vgx_flow* fl, FlowFcn* F, size_t lds, hipStream_t s) {
+    const int na = F->ncomp, nc = (int)(lds / 4) - 2 * na;
+    int rc = fl->fpar.ensure(lds * 2);
+    if (rc) return rc;
+    double* d = (double*)fl->fpar.ptr;
+    VGX_HIP(hipStreamWaitEvent(s, fl->used, 0));
+    hipLaunchKernelGGL(flow_hold_kernel, dim3((2 * na + nc + 1023) / 1024), dim3(256), 0, s, *F, na, nc, d);
+    if ((rc = check_launch())) return rc;
+    VGX_HIP(hipEventRecord(fl->held, s));
+    F->A = d;
+    F->B = d + na;
+    F->c = d + 2 * na;
+    return VGX_OK;
+}
+static int flow_params_held(vgx_flow* fl, hipStream_t s) {
+    VGX_HIP(hipEventRecord(fl->used, s));
+    VGX_HIP(hipEventSynchronize(fl->held));
     return VGX_OK;
 }
 
@@ -1262,6 +1301,7 @@ extern "C" int vgx_flow_sample(vgx_flow* fl, const vgx_integrand* fcn, int64_t n
     size_t fcn_lds;
     int rc = flow_fcn_params(fl, fcn, &F, &fcn_lds);
     if (rc) return rc;
+    if (!sums && (rc = flow_hold_params(fl, &F, fcn_lds, s))) return rc;
     DeviceInfo info;
     if ((rc = device_info(&info))) return rc;
     const FlowShape sh = flow_shape(n, info.cus, info.cus, fcn_lds);
@@ -1289,7 +1329,7 @@ extern "C" int vgx_flow_sample(vgx_flow* fl, const vgx_integrand* fcn, int64_t n
     else
         hipLaunchKernelGGL(flow_sample_kernel, dim3(blocks), dim3(64 * sh.waves), lds, s, flow_args(fl), F, a);
     if ((rc = check_launch())) return rc;
-    if (!sums) return VGX_OK;
+    if (!sums) return flow_params_held(fl, s);
     std::vector<double> h((size_t)blocks * 4);
     VGX_HIP(hipMemcpyAsync(h.data(), a.part, h.size() * 8, hipMemcpyDeviceToHost, s));
     VGX_HIP(hipStreamSynchronize(s));
@@ -1423,8 +1463,10 @@ extern "C" int vgx_flow_eval(vgx_flow* fl, const vgx_integrand* fcn, const float
     if (hipFuncSetAttribute((const void*)flow_eval_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)(fcn_lds + 16)) != hipSuccess)
         return VGX_EHIP;
+    if ((rc = flow_hold_params(fl, &F, fcn_lds, s))) return rc;
     hipLaunchKernelGGL(flow_eval_kernel, dim3(blocks), dim3(256), fcn_lds + 16, s, F, fl->D, x, (uint64_t)n, f);
-    return check_launch();
+    if ((rc = check_launch())) return rc;
+    return flow_params_held(fl, s);
 }
 
 extern "C" int vgx_flow_mfma_probe(const uint16_t* A, const uint16_t* B, float* D, void* stream) {

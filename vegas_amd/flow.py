@@ -189,20 +189,10 @@ class CouplingFlow:
         _lib.check(self._L.vgx_flow_adam(self._h, lr, beta1, beta2, eps, clip, _lib.stream_ptr()), 'vgx_flow_adam')
         self.steps += 1
 
-    def _integrand(self, fcn):
-        """The integrand for a launch on the current stream.  The kernel reads
-        its arrays, which may belong to another stream, after the call
-        returns: they are not reused before."""
-        torch = self._torch
-        vf, keep = fcn.vgx_integrand(torch, torch.device('cuda'))
-        for t in keep:
-            t.record_stream(torch.cuda.current_stream())
-        return vf
-
     def eval_fcn(self, fcn, x):
         """f(x) of a device integrand at device points x float [n][16]."""
         torch = self._torch
-        vf = self._integrand(fcn)
+        vf, keep = fcn.vgx_integrand(torch, torch.device('cuda'))
         n = x.shape[0]
         out = torch.empty(n, dtype=torch.float32, device='cuda')
         _lib.check(self._L.vgx_flow_eval(self._h, C.byref(vf), _lib.ptr(x), n, _lib.ptr(out), _lib.stream_ptr()),
@@ -216,7 +206,7 @@ class CouplingFlow:
         sums are None, the call does not wait for the GPU, and a NaN integrand
         shows as VGX_ENAN in ``status`` for the caller to check."""
         torch = self._torch
-        vf = self._integrand(fcn)
+        vf, keep = fcn.vgx_integrand(torch, torch.device('cuda'))
         lazy = status is not None
         if lazy and not keep_points:
             raise ValueError('a lazy sample needs keep_points')
