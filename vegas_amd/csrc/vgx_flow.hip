@@ -447,10 +447,7 @@ __global__ __launch_bounds__(kFlowThreads) void flow_sample_kernel(FlowArgs f, F
             f32x4_t uq;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                // below 1: the last of the 2^24 values rounds to it, and its
-                // logit and Jacobian would be infinite, f J a NaN
-                const float z = fminf((float)(ws[i] >> 8) * (1.0f / 16777216.0f) + (1.0f / 33554432.0f),
-                                      1.0f - 1.0f / 16777216.0f);
+                const float z = (float)(ws[i] >> 8) * (1.0f / 16777216.0f) + (1.0f / 33554432.0f);
                 const float l0 = __logf(z), l1 = __logf(1.0f - z);
                 uq[i] = l0 - l1;
                 if (4 * g + i < f.D) l -= l0 + l1;  // dz/du = z (1 - z)
@@ -526,8 +523,12 @@ __global__ __launch_bounds__(kFlowThreads) void flow_sample_kernel(FlowArgs f, F
             const uint64_t sl = pb + (uint64_t)(wave * a.tiles + q) * 16 + (lane & 15);
             if (q < a.tiles && sl < a.n) {
                 const float fl = TS->l[q][lane & 15], lj = TS->l[q][16 + (lane & 15)];
-                // f = 0 where the map stretches enough for J to overflow is 0
-                const double fj = fl != 0.f ? (double)fl * exp_jac((double)lj) : 0.0;
+                // f = 0 where the map stretches enough for J to overflow is 0,
+                // and so is a sample at the end of the unit interval: the last
+                // of the 2^24 values of a z rounds to 1, whose u is infinite and
+                // whose log J is a NaN where f is none
+                const bool in = fl != 0.f && (lj == lj || fl != fl);
+                const double fj = in ? (double)fl * exp_jac((double)lj) : 0.0;
                 dd_add(s1, fj);
                 dd_add(s2, fj * fj);
                 if (a.xout) a.fout[sl] = (float)fj;
