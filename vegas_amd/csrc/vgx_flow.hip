@@ -1149,9 +1149,9 @@ struct vgx_flow {
     uint16_t* H = nullptr;
     uint16_t* HT = nullptr;
     // per-batch scratch (grown on demand)
-    Scratch saved, u0, logq, c, G, wpart, cpart, spart, misc, fpar;
-    hipEvent_t held = nullptr;  // fpar has been written
-    hipEvent_t used = nullptr;  // and read
+    Scratch saved, u0, logq, c, G, wpart, cpart, spart, misc;
+    hipEvent_t held = nullptr;  // an integrand's parameters have been copied
+    hipEvent_t used = nullptr;  // and the copy read
     int step = 0;
 };
 
@@ -1216,7 +1216,7 @@ extern "C" int vgx_flow_destroy(vgx_flow* fl) {
     for (void* p : ps)
         if (p) (void)hipFree(p);
     Scratch* ss[] = {&fl->saved, &fl->u0, &fl->logq, &fl->c, &fl->G, &fl->wpart, &fl->cpart, &fl->spart,
-                     &fl->misc, &fl->fpar};
+                     &fl->misc};
     for (Scratch* q : ss) q->release();
     for (hipEvent_t e : {fl->held, fl->used})
         if (e) (void)hipEventDestroy(e);
@@ -1254,6 +1254,13 @@ extern "C" int vgx_flow_get_params(const vgx_flow* fl, float* host, float* grad_
     return VGX_OK;
 }
 
+// Sampling scratch: a workgroup's sums (one workgroup per CU) | a copy of an
+// integrand's FP64 parameters (kFlowFcnMax bytes as FP32).
+constexpr size_t kFlowFcnMax = 48 * 1024;
+static int flow_spart(vgx_flow* fl, const DeviceInfo& info) {
+    return fl->spart.ensure((size_t)info.cus * 4 * 8 + 2 * kFlowFcnMax);
+}
+
 // The integrand as the kernels read it (its arrays are the caller's), and its
 // LDS bytes.
 static int flow_fcn_params(const vgx_flow* fl, const vgx_integrand* fcn, FlowFcn* F, size_t* lds) {
@@ -1262,7 +1269,7 @@ static int flow_fcn_params(const vgx_flow* fl, const vgx_integrand* fcn, FlowFcn
     if (!fcn->A || !fcn->B || !fcn->c) return VGX_EINVAL;
     const size_t nc = (size_t)fcn->ncomp;
     *lds = (2 * nc + (fcn->kind == VGX_FCN_GAUSSMIX ? nc * fl->D : nc)) * 4;
-    if (*lds > 48 * 1024) return VGX_ERANGE;  // staged in LDS with the layer
+    if (*lds > kFlowFcnMax) return VGX_ERANGE;  // staged in LDS with the layer
     *F = FlowFcn{fcn->kind, fcn->ncomp, fcn->A, fcn->B, fcn->c};
     return VGX_OK;
 }
@@ -1275,9 +1282,10 @@ static int flow_fcn_params(const vgx_flow* fl, const vgx_integrand* fcn, FlowFcn
 // reader.
 static int flow_hold_params(vgx_flow* fl, FlowFcn* F, size_t lds, hipStream_t s) {
     const int na = F->ncomp, nc = (int)(lds / 4) - 2 * na;
-    int rc = fl->fpar.ensure(lds * 2);
-    if (rc) return rc;
-    double* d = (double*)fl->fpar.ptr;
+    DeviceInfo info;
+    int rc = device_info(&info);
+    if (rc || (rc = flow_spart(fl, info))) return rc;
+    double* d = (double*)fl->spart.ptr + 4 * (size_t)info.cus;
     VGX_HIP(hipStreamWaitEvent(s, fl->used, 0));
     hipLaunchKernelGGL(flow_hold_kernel, dim3((2 * na + nc + 1023) / 1024), dim3(256), 0, s, *F, na, nc, d);
     if ((rc = check_launch())) return rc;
@@ -1307,7 +1315,7 @@ extern "C" int vgx_flow_sample(vgx_flow* fl, const vgx_integrand* fcn, int64_t n
     if ((rc = device_info(&info))) return rc;
     const FlowShape sh = flow_shape(n, info.cus, info.cus, fcn_lds);
     const int blocks = sh.blocks;
-    if ((rc = fl->spart.ensure((size_t)blocks * 4 * 8))) return rc;
+    if ((rc = flow_spart(fl, info))) return rc;
     SampleArgs a{};
     a.n = (uint64_t)n;
     a.base = base;
