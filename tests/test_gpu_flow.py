@@ -390,3 +390,22 @@ def test_parameters_are_the_callers_after_the_call(torch, call):
         assert torch.equal(got, want) and torch.equal(got2, want2)
         for a, v in zip(arrays, f._param_arrays()):
             a.copy_(torch.as_tensor(v))
+
+
+@pytest.mark.parametrize("nc", [1750, 1770, 2200, 2900, 3500, 4096])
+def test_long_integrands_in_large_calls(torch, nc):
+    """Parameters that leave LDS for 12, 11, 10, 9 and 8 waves: the points and
+    values of a call of several passes are the bits of a small call's, where 4
+    waves fit always."""
+    import vegas_amd as va
+    from vegas_amd.flow import CouplingFlow
+    f = va.DiagonalRidge([1.0] * nc, [20.0] * nc, np.linspace(0.3, 0.7, nc), 5)
+    flow = CouplingFlow(5, 4, seed=3)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    n = 2 * 72 * 16 * cus + 3
+    s1, s2, x, fj = flow.sample(f, n, seed=8, iteration=1, keep_points=True)
+    for base in (0, 3000, n - 1000):
+        _, _, xs, fs = flow.sample(f, 1000, seed=8, iteration=1, base=base, keep_points=True)
+        assert torch.equal(xs, x[base:base + 1000]) and torch.equal(fs, fj[base:base + 1000])
+    np.testing.assert_allclose(s1, fj.double().sum().item(), rtol=6e-8, equal_nan=False)
+    np.testing.assert_allclose(s2, (fj.double() ** 2).sum().item(), rtol=1.2e-7, equal_nan=False)
