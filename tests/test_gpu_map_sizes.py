@@ -74,3 +74,36 @@ def test_map_invmap_sizes(va, orc, dim, ninc, n):
     yr, jr = o.invmap(xo)
     assert np.array_equal(yi.cpu().numpy(), yr)
     assert np.array_equal(ji.cpu().numpy(), jr)
+
+
+@pytest.mark.parametrize("dim", [1, 3, 16])
+@pytest.mark.parametrize("ninc", [1, 2, 10, 400])
+@pytest.mark.parametrize("kind", ["plain", "equal", "tiny", "huge"])
+def test_invmap_table_and_search(va, dim, ninc, kind):
+    """The search within a table's cell (from 65536 points) and over all nodes
+    give the same bits for any x, NaN and infinities among them, on grids with
+    equal nodes, denormal increments and lengths that overflow."""
+    import torch
+    rng = np.random.default_rng(ninc)
+    inc = np.exp(rng.normal(0, 2, (dim, ninc)))
+    if kind == "equal":
+        inc[:, ::2] = 0.0
+    grid = np.concatenate([np.zeros((dim, 1)), np.cumsum(inc, axis=1)], axis=1)
+    if kind == "tiny":
+        grid *= 5e-324 * 64 / inc.mean()
+    if kind == "huge":
+        grid = (grid / grid.max() * 2.0 - 1.0) * 1.7e308
+    m = va.AdaptiveMap(grid.tolist())
+    n = 1000
+    x = grid[:, rng.integers(0, ninc + 1, n)].T.copy()
+    with np.errstate(over='ignore'):
+        x[::2] = x[::2] + rng.uniform(-0.1, 1.1, x[::2].shape) * (grid[:, 1] - grid[:, 0]).max()
+    x[3::11] = np.nan
+    x[4::11] = np.inf
+    x[5::11] = -np.inf
+    x[6::11] = np.nextafter(x[6::11], np.inf)
+    x = torch.as_tensor(x, device='cuda')
+    y, jac = m.invmap(x)
+    yt, jt = m.invmap(x.repeat(70, 1))
+    assert torch.equal(yt.view(torch.int64), y.view(torch.int64).repeat(70, 1))
+    assert torch.equal(jt.view(torch.int64), jac.view(torch.int64).repeat(70))

@@ -25,7 +25,9 @@ constexpr size_t kMapTileMax = 56 * 1024;   // of it, a tile's Jacobian factors,
 constexpr size_t kMapGridMax = 136 * 1024;  // a larger grid is read from global memory
 constexpr int kMapCells = 512;              // cells per axis of invmap's table, at most
 // points from which the table saves more probes than it costs (1e6 points of 8
-// axes: 50 us with it, 65 without; 5e4: no gain)
+// axes of 1000: 50 us with it, 65 without; 5e4: no gain; with 10 increments
+// it gains from 1e6 elements on and costs up to 1 us below, where 65,536 points
+// of 24 axes cost 80 us with a table filled axis by axis)
 constexpr int64_t kMapLutMin = 1 << 16;
 
 struct MapArgs {
@@ -64,15 +66,25 @@ __device__ inline int map_cell(double xv, double g0, double scale, int cells) {
     return c >= (double)(cells - 1) ? cells - 1 : c > 0.0 ? (int)c : 0;
 }
 
-// lut[c]: the first node whose cell is c or more (ni + 1 past the last), so
-// that the nodes before lut[c] are below every x of cell c and those from
-// lut[c + 1] on are above: the search of all nodes ends in between.
-__device__ inline void fill_lut(const double* g, int ni, double scale, int cells, uint16_t* lut) {
-    for (int i = threadIdx.x; i <= ni + 1; i += kMapThreads) {
-        const int c0 = i > 0 ? map_cell(g[i - 1], g[0], scale, cells) : -1;
-        const int c1 = i <= ni ? map_cell(g[i], g[0], scale, cells) : cells;
-        for (int c = c0 + 1; c <= c1; ++c) lut[c] = (uint16_t)i;
+// Row d of lut, [c]: the first node of axis d whose cell is c or more (ni + 1
+// past the last), so that the nodes before [c] are below every x of cell c and
+// those from [c + 1] on are above: the search of all nodes ends in between.
+// All axes at once (one after the other, each with its division and few busy
+// lanes, 24 axes of 10 increments took 64 us of the call's 81, now 17 in all).
+__device__ inline void fill_lut(const MapArgs& a, const double* G, const int32_t* ninc, double* sc, uint16_t* lut) {
+    for (int d = threadIdx.x; d < a.dim; d += kMapThreads)
+        sc[d] = (double)a.cells / (G[d * a.ld + ninc[d]] - G[d * a.ld]);
+    __syncthreads();
+    const int row = a.ld + 1;
+    for (int e = threadIdx.x; e < a.dim * row; e += kMapThreads) {
+        const int d = e / row, i = e - d * row, ni = ninc[d];
+        if (i > ni + 1) continue;
+        const double* g = G + d * a.ld;
+        const int c0 = i > 0 ? map_cell(g[i - 1], g[0], sc[d], a.cells) : -1;
+        const int c1 = i <= ni ? map_cell(g[i], g[0], sc[d], a.cells) : a.cells;
+        for (int c = c0 + 1; c <= c1; ++c) lut[d * (a.cells + 1) + c] = (uint16_t)i;
     }
+    __syncthreads();
 }
 
 // AdaptiveMap.invmap (pyx:362-416) of a thread's elements together: for
@@ -164,15 +176,7 @@ __global__ __launch_bounds__(kMapThreads) void map_kernel(MapArgs a, const T* __
     };
     if ((int64_t)blockIdx.x < ntiles) load(blockIdx.x, cur);
     __syncthreads();
-    if (OP == 1 && a.cells) {
-        for (int d = 0; d < dim; ++d) {
-            const double* g = G + d * a.ld;
-            const double scale = (double)a.cells / (g[a.ninc[d]] - g[0]);
-            if (threadIdx.x == 0) sc[d] = scale;
-            fill_lut(g, a.ninc[d], scale, a.cells, lut + d * (a.cells + 1));
-        }
-        __syncthreads();
-    }
+    if (OP == 1 && a.cells) fill_lut(a, G, ni, sc, lut);
     for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
         // the next tile's loads are in flight while this one is mapped
         if (t + gridDim.x < ntiles) load(t + gridDim.x, nxt);
@@ -254,6 +258,12 @@ static int launch_map(MapArgs a, const T* in, T* out, T* jac, void* stream) {
     const int64_t split = 256 * (OP == 1 ? 1 : 4);
     const int64_t share = std::max<int64_t>((a.n + split - 1) / split, kMapThreads / a.dim);
     a.pts = (int)std::max<int64_t>(1, std::min(most, (share + 63) & ~(int64_t)63));
+    if (OP == 1 && share > most) {
+        // as many points in each of a workgroup's tiles (300,000 points of 5
+        // axes: 1.4 tiles of 819 a workgroup 14.0 us, 2 of 592 13.2)
+        const int64_t rounds = (share + most - 1) / most;
+        a.pts = (int)std::min(most, ((share + rounds - 1) / rounds + 7) & ~(int64_t)7);
+    }
     if (OP != 2) lds += (size_t)a.pts * a.pad * sizeof(double);
     lds = (lds + 15) & ~(size_t)15;
     auto kern = a.use_lds ? map_kernel<OP, true, T> : map_kernel<OP, false, T>;
