@@ -215,3 +215,43 @@ def test_hcube_counts(va, orc, nhcube, beta):
         (integ.sigf * (integ.neval_frac * integ.neval / integ.sum_sigf)).astype(np.int64) + integ.min_neval_hcube,
         integ.max_neval_hcube)
     np.testing.assert_array_equal(np.bincount(h, minlength=nhcube), want)
+
+
+@pytest.mark.parametrize("ns,per", [([1, 1], 33000), ([5, 1], 10000), ([5, 1], 128), ([5, 1], 129), ([40, 26], 32),
+                                    ([40, 26], 33), ([40, 26], 130), ([64, 64], 40), ([300, 10], 2100),
+                                    ([300, 220], 33)])
+def test_covariance_plans(va, ns, per):
+    """The launch plans of the covariance kernels (a workgroup per hcube, a few
+    hcubes per workgroup, many; all pairs at once or pair by pair) against the
+    points' own sums, hcube by hcube, in 64 bits: the sums differ in their
+    order only (1e-12 for means; deviations are at least 0.01 of the values, so
+    1e-10 for covariances, on the scale of the variances)."""
+    import torch
+    nh = ns[0] * ns[1]
+    kw = dict(neval=nh * per, nstrat=ns, beta=0.0, seed=3, min_neval_batch=10 ** 9)
+    region = [[0, 1], [0, 2]]
+
+    def values(x, m):
+        g = torch.exp(-3.0 * ((x - 0.4) ** 2).sum(1))
+        return torch.stack([g * (1 + x[:, 0] * k) * (1 + 0.5 * x[:, 1]) ** k for k in range(m)], 1)
+
+    for m in (1, 3, 4, 5, 6, 7):
+        seen = []
+
+        def f(x):
+            seen.append(x.clone())
+            return values(x, m)
+
+        integ = va.Integrator(region, **kw)
+        r = integ(va.gpu_lbatchintegrand(f), nitn=1).itn_results[0]
+        x = seen[-1]
+        assert x.shape[0] == nh * per
+        # a uniform grid: every weight is the region's volume over the points
+        wf = (values(x, m) * (2.0 / (nh * per))).reshape(nh, per, m)
+        S = wf.sum(1)
+        d = wf - (S / per)[:, None, :]
+        mean = S.sum(0)
+        cov = (torch.matmul(d.transpose(1, 2).contiguous(), d).sum(0) * (per / (per - 1.0))).cpu().numpy()
+        sd = np.sqrt(np.diag(cov))
+        np.testing.assert_allclose(np.asarray(r.mean), mean.cpu().numpy(), rtol=1e-12)
+        np.testing.assert_allclose(np.asarray(r.cov) / np.outer(sd, sd), cov / np.outer(sd, sd), atol=1e-10)

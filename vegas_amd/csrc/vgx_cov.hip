@@ -24,6 +24,24 @@ constexpr int kCovMaxBlocks = 8192;  // workgroups per pair (one thread per hcub
 // components, now up to 170.  From 16 by a wave: 5-15 % slower where most
 // hcubes are that short; from 8 twice the time.)
 constexpr uint32_t kCovShort = 32, kCovLong = 2048;
+// A batch of hcubes that are long on average (above kCovShort) has few of them:
+// with a workgroup for 256 they would be the work of a few waves.  As long as
+// that gives fewer workgroups than CUs, it has a workgroup for each hcube, up to
+// kCovFew in all, the hcubes of a workgroup are spread over its waves, and a
+// workgroup with one hcube sums it together from kCovAlone points on.  (56
+// hcubes of 2000 points, six components: 1306 us by one wave, 361 by one
+// workgroup in turn, 36 so.  kCovFew = 2048: 40,000 hcubes of 40, 231 us for 178.)
+constexpr int kCovFew = 1024;
+constexpr uint32_t kCovAlone = 128;
+// Five and six components: pair by pair for few points or hcubes, where the
+// kernel of all pairs is one long chain.  (us a call, all pairs / pair by pair:
+// 256 hcubes of 4 points 25 / 17, 56 of 500 33 / 17, one of 100,000 349 / 299.)
+constexpr int64_t kCovPairPoints = 32768, kCovPairHcubes = 4;
+
+struct CovPlan {
+    uint32_t lng;  // hcubes with more points are summed by the workgroup
+    uint32_t few;  // spread a workgroup's hcubes over its waves
+};
 
 // Pair q of the lower triangle (t <= s), row-major: (0,0) (1,0) (1,1) (2,0) ...
 __device__ inline void cov_pair(int q, int correlate, int& s, int& t) {
@@ -115,29 +133,30 @@ __device__ inline void wave_total(double (&v)[K]) {
 // The hcubes [h0, h1) in rounds of gridDim.x * blockDim.x: thread t of
 // workgroup b takes hcube h0 + r0 + t * gridDim.x + b (neighbouring hcubes,
 // which tend to be large together near a peak, land in different
-// workgroups).  A hcube of at most kCovShort points is summed by its thread
+// workgroups; with `few` also in different waves).  A hcube of at most kCovShort points is summed by its thread
 // (wk.thread_hcube), a longer one after that by the thread's wave
-// (wk.wave_hcube), and those of more than kCovLong points after the round by
+// (wk.wave_hcube), and those of more than pl.lng points after the round by
 // the whole workgroup, in thread order (wk.block_hcube), so the work per
 // thread stays bounded however the points are spread.  A hcube whose points are not the
 // batch's [p0, p1) (or that has fewer than two) sets VGX_ERANGE and is not read.
 template <class Work>
 __device__ inline void cov_rounds(const uint32_t* off, uint32_t h0, uint32_t h1, uint32_t p0, uint32_t p1,
-                                  int32_t* status, Work& wk) {
+                                  CovPlan pl, int32_t* status, Work& wk) {
     __shared__ uint64_t lmask[kCovWaves];
     __shared__ uint32_t la[kCovThreads], lb[kCovThreads];
     const uint32_t nh = h1 - h0, stride = gridDim.x * blockDim.x;
     for (uint32_t r0 = 0; r0 < nh; r0 += stride) {
-        const uint32_t idx = r0 + threadIdx.x * gridDim.x + blockIdx.x;
-        bool lng = false, mid = false;
+        const uint32_t slot = pl.few ? (threadIdx.x & 63) * kCovWaves + (threadIdx.x >> 6) : threadIdx.x;
+        const uint32_t idx = r0 + slot * gridDim.x + blockIdx.x;
+        bool block = false, mid = false;
         uint32_t oa = 0, ob = 0;
         if (idx < nh) {
             oa = off[h0 + idx];
             ob = off[h0 + idx + 1];
             if (oa < p0 || ob > p1 || ob < oa + 2) {
                 if (status) atomicOr(status, VGX_ERANGE);
-            } else if (ob - oa > kCovLong) {
-                lng = true;
+            } else if (ob - oa > pl.lng) {
+                block = true;
                 la[threadIdx.x] = oa - p0;
                 lb[threadIdx.x] = ob - p0;
             } else if (ob - oa > kCovShort) {
@@ -150,7 +169,7 @@ __device__ inline void cov_rounds(const uint32_t* off, uint32_t h0, uint32_t h1,
             const int src = __builtin_ctzll(mk);
             wk.wave_hcube(__builtin_amdgcn_readlane(oa, src) - p0, __builtin_amdgcn_readlane(ob, src) - p0, src);
         }
-        const uint64_t bal = __ballot(lng);
+        const uint64_t bal = __ballot(block);
         if ((threadIdx.x & 63) == 0) lmask[threadIdx.x >> 6] = bal;
         __syncthreads();
         for (int wv = 0; wv < kCovWaves; ++wv) {
@@ -248,12 +267,12 @@ struct PairWork {
 
 __global__ __launch_bounds__(kCovThreads) void cov_hcube_kernel(const uint32_t* off, uint32_t h0, uint32_t h1,
                                                                  uint32_t p0, uint32_t p1, const double* w,
-                                                                 const double* f, int m, int correlate,
+                                                                 const double* f, int m, int correlate, CovPlan pl,
                                                                  double* part, int32_t* status) {
     __shared__ double red[4 * kCovWaves];
     PairWork wk{w, f, m, 0, 0, kEpsilon, DD{0, 0}, DD{0, 0}, red};
     cov_pair((int)blockIdx.y, correlate, wk.s, wk.t);
-    cov_rounds(off, h0, h1, p0, p1, status, wk);
+    cov_rounds(off, h0, h1, p0, p1, pl, status, wk);
     DD am = wave_sum_dd(wk.am);
     DD av = wave_sum_dd(wk.av);
     const int wv = threadIdx.x >> 6;
@@ -389,7 +408,7 @@ struct AllWork {
 template <int M>
 __global__ __launch_bounds__(kCovThreads) void cov_hcube_all_kernel(const uint32_t* off, uint32_t h0, uint32_t h1,
                                                                      uint32_t p0, uint32_t p1, const double* w,
-                                                                     const double* f, int correlate,
+                                                                     const double* f, int correlate, CovPlan pl,
                                                                      double* part, int32_t* status) {
     constexpr int NP = M * (M + 1) / 2;
     __shared__ double red[kCovWaves * 2 * (M + NP)];
@@ -402,7 +421,7 @@ __global__ __launch_bounds__(kCovThreads) void cov_hcube_all_kernel(const uint32
     for (int s = 0; s < M; ++s) wk.am[s] = DD{0, 0};
 #pragma unroll
     for (int q = 0; q < NP; ++q) wk.av[q] = DD{0, 0};
-    cov_rounds(off, h0, h1, p0, p1, status, wk);
+    cov_rounds(off, h0, h1, p0, p1, pl, status, wk);
     // workgroup partials: mean entries then pair entries, DD per wave
     const int wv = threadIdx.x >> 6;
 #pragma unroll
@@ -489,7 +508,16 @@ extern "C" int vgx_iter_accumulate_cov(vgx_ctx* ctx, const vgx_config* c, int64_
     hipStream_t s = (hipStream_t)stream;
     const int npairs = correlate ? m * (m + 1) / 2 : m;
     const int64_t nh = h1 - h0;
-    const int nbx = (int)std::min<int64_t>(kCovMaxBlocks, (nh + kCovThreads - 1) / kCovThreads);
+    const int64_t np = p1 - p0;
+    const bool all = m <= kCovAllMax && (m <= 4 || (np > kCovPairPoints && nh > kCovPairHcubes));
+    const int rows = all ? 1 : npairs;  // workgroups per block of hcubes
+    int64_t blocks = std::min<int64_t>(kCovMaxBlocks, (nh + kCovThreads - 1) / kCovThreads);
+    CovPlan pl{kCovLong, 0};
+    if (np > nh * (int64_t)kCovShort && blocks * rows < ctx->info.cus) {
+        blocks = std::min<int64_t>(nh, std::max<int64_t>(blocks, kCovFew / rows));
+        pl = CovPlan{blocks == nh ? kCovAlone : kCovLong, 1};
+    }
+    const int nbx = (int)blocks;
     int rc;
     if ((rc = ctx->cov_part.ensure((size_t)npairs * nbx * 4 * sizeof(double)))) return rc;
     const uint32_t* off = (const uint32_t*)ctx->off.ptr;
@@ -498,22 +526,22 @@ extern "C" int vgx_iter_accumulate_cov(vgx_ctx* ctx, const vgx_config* c, int64_
     hipEvent_t e0 = nullptr, e1 = nullptr;
     const bool timed = timed_slot(ctx, kTimedCov, &e0, &e1);
     if (timed) VGX_HIP(hipEventRecord(e0, s));
-    switch (m <= kCovAllMax ? m : 0) {
+    switch (all ? m : 0) {
         case 1: hipLaunchKernelGGL(cov_hcube_all_kernel<1>, dim3(nbx), dim3(kCovThreads), 0, s, off, (uint32_t)h0,
-                                   (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, part, status); break;
+                                   (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, pl, part, status); break;
         case 2: hipLaunchKernelGGL(cov_hcube_all_kernel<2>, dim3(nbx), dim3(kCovThreads), 0, s, off, (uint32_t)h0,
-                                   (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, part, status); break;
+                                   (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, pl, part, status); break;
         case 3: hipLaunchKernelGGL(cov_hcube_all_kernel<3>, dim3(nbx), dim3(kCovThreads), 0, s, off, (uint32_t)h0,
-                                   (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, part, status); break;
+                                   (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, pl, part, status); break;
         case 4: hipLaunchKernelGGL(cov_hcube_all_kernel<4>, dim3(nbx), dim3(kCovThreads), 0, s, off, (uint32_t)h0,
-                                   (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, part, status); break;
+                                   (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, pl, part, status); break;
         case 5: hipLaunchKernelGGL(cov_hcube_all_kernel<5>, dim3(nbx), dim3(kCovThreads), 0, s, off, (uint32_t)h0,
-                                   (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, part, status); break;
+                                   (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, pl, part, status); break;
         case 6: hipLaunchKernelGGL(cov_hcube_all_kernel<6>, dim3(nbx), dim3(kCovThreads), 0, s, off, (uint32_t)h0,
-                                   (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, part, status); break;
+                                   (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, correlate, pl, part, status); break;
         default:
             hipLaunchKernelGGL(cov_hcube_kernel, dim3(nbx, npairs), dim3(kCovThreads), 0, s, off, (uint32_t)h0,
-                               (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, m, correlate, part, status);
+                               (uint32_t)h1, (uint32_t)p0, (uint32_t)p1, wgt, f, m, correlate, pl, part, status);
     }
     hipLaunchKernelGGL(cov_reduce_kernel, dim3(npairs), dim3(kCovThreads), 0, s,
                        (const double*)ctx->cov_part.ptr, nbx, npairs, m, correlate, acc);
