@@ -107,3 +107,22 @@ def test_invmap_table_and_search(va, dim, ninc, kind):
     yt, jt = m.invmap(x.repeat(70, 1))
     assert torch.equal(yt.view(torch.int64), y.view(torch.int64).repeat(70, 1))
     assert torch.equal(jt.view(torch.int64), jac.view(torch.int64).repeat(70))
+
+
+@pytest.mark.parametrize("n", [2, 2047, 4095, 4096, 4097, 5 * 1024 + 64, 17 * 1024 - 1])
+@pytest.mark.parametrize("ninc", [[1], [40, 3], [1000] * 3, [3000]])
+def test_train_hist_few_tiles(va, orc, n, ninc):
+    """The ordered histogram on both sides of its few tiles (up to 4 of 1024
+    points), with whole and cut groups of 64 points in the last."""
+    rng = np.random.default_rng(n)
+    dim = len(ninc)
+    m, o = va.AdaptiveMap([[0, 1]] * dim, ninc=ninc), orc.OracleMap([[0, 1]] * dim, ninc=ninc)
+    y = rng.uniform(0, 1, (n, dim)) ** 3
+    y[::5, 0] = 1.0
+    f = rng.normal(size=n) * np.exp(rng.uniform(-20, 20, n))
+    for _ in range(2):
+        m.add_training_data(y, f)
+        o.add_training_data(y, f)
+    for d, k in enumerate(ninc):
+        assert np.array_equal(m.sum_f[d, :k], o.sum_f[d, :k])
+        assert np.array_equal(m.n_f[d, :k], o.n_f[d, :k])
