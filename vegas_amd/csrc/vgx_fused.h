@@ -153,7 +153,8 @@ struct CoordWalk {
 //   between the grid reads (a scalar load shares the LDS reads' wait counter
 //   and returns out of order, which would wait out every grid read at once).
 //   DIM > 0: that dimension; DIM <= 0: runtime g.dim, at most nd_max(DIM).
-template <int DIM, bool R32, bool PER>
+//   XJ false: the bins only (the grid is not read, x and J are not set).
+template <int DIM, bool R32, bool PER, bool XJ = true>
 __device__ __forceinline__ void eval_point(const TileGeom& g, const AxisC* __restrict__ ax,
                                            const double* __restrict__ G, const PackedCoords<DIM>& pc,
                                            uint32_t h, uint32_t p, double* x, double& J, int* kbin,
@@ -207,6 +208,8 @@ __device__ __forceinline__ void eval_point(const TileGeom& g, const AxisC* __res
             dl = tt - (double)k;
             kv = (yv > 0 && yv < 1) ? (k < ni ? k : ni - 1) : -1;
         }
+        kbin[d] = kv;
+        if constexpr (!XJ) continue;
         const double* gd = G + d * g.ld;
         if (PER) {
             // k < ninc always: no branch, the loads can be issued early; x by
@@ -225,7 +228,6 @@ __device__ __forceinline__ void eval_point(const TileGeom& g, const AxisC* __res
             x[d] = in ? g0 + inc * dl : g1;
             J *= inc * (double)ni;
         }
-        kbin[d] = kv;
         if (!PER) {
             // formed here: left to the compiler, bin and Jacobian are computed
             // where they are used, after the integrand, and every axis' y,

@@ -786,7 +786,7 @@ __global__ void sigf_reset_kernel(double* sigf, int64_t n, Scalars* sc) {
 
 // eval_point for hcube h with the stratum->bin path the fused sampler takes
 // for this geometry (staged and error-training kernels).
-template <int DIM, bool R32>
+template <int DIM, bool R32, bool XJ = true>
 __device__ inline void eval_point_h(const IterGeom& g, const AxisC* axes, const double* grid, uint32_t h,
                                     uint32_t p, double* x, double& J, int* kb) {
     PackedCoords<DIM> pc;
@@ -794,7 +794,7 @@ __device__ inline void eval_point_h(const IterGeom& g, const AxisC* axes, const 
     if constexpr (R32) {
         if (g.per_all) {
             pc.set(axes, g.dim, h);
-            eval_point<DIM, true, true>(tile_geom(g), axes, grid, pc, h, p, x, J, kb, zmin);
+            eval_point<DIM, true, true, XJ>(tile_geom(g), axes, grid, pc, h, p, x, J, kb, zmin);
             if (zmin == 0) {
                 const uint64_t zm = per_zero_axes<DIM>(tile_geom(g), pc, p);
 #pragma unroll
@@ -806,7 +806,7 @@ __device__ inline void eval_point_h(const IterGeom& g, const AxisC* axes, const 
             return;
         }
     }
-    eval_point<DIM, R32, false>(tile_geom(g), axes, grid, pc, h, p, x, J, kb, zmin);
+    eval_point<DIM, R32, false, XJ>(tile_geom(g), axes, grid, pc, h, p, x, J, kb, zmin);
 }
 
 // adapt_to_errors: training entry |var_h| at the last point of every hcube
@@ -818,10 +818,9 @@ __global__ __launch_bounds__(256) void errors_train_kernel(IterGeom g, const Axi
     if (sc->status || sc->overflow) return;
     for (int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; h < g.nhcube;
          h += (int64_t)gridDim.x * blockDim.x) {
-        double x[VGX_MAXDIM];
         int kb[VGX_MAXDIM];
         double J;
-        eval_point_h<0, R32>(g, axes, grid, (uint32_t)h, off[h + 1] - 1, x, J, kb);
+        eval_point_h<0, R32, false>(g, axes, grid, (uint32_t)h, off[h + 1] - 1, nullptr, J, kb);
         for (int d = 0; d < g.dim; ++d)
             if (kb[d] >= 0) {
                 unsafeAtomicAdd(&sum_f[d * g.nb + kb[d]], errv[h]);
