@@ -952,7 +952,8 @@ __device__ inline void block_close_tiles(const TileAcc& acc, const double* tpart
 // vector registers: besides the time, this compiler places some of the spill
 // stores before the exec mask is restored at the end of a branch, and the
 // lanes that skipped the branch then lose the value (the 9-axis FP64 sampler's
-// sums came out wrong so).  us per launch of 1e6 points, 1024 threads with
+// sums came out wrong so).  The build fails where a kernel spills them, the
+// batched sampler among them (the Makefile's kernel-resource-usage).  us per launch of 1e6 points, 1024 threads with
 // spills / without: 9 axes f64 49 / 41, 13 axes 91 / 61.
 constexpr int sampler_threads(int dim, bool per) {
     if (dim > 16) dim = 0;
