@@ -255,3 +255,50 @@ def test_covariance_plans(va, ns, per):
         sd = np.sqrt(np.diag(cov))
         np.testing.assert_allclose(np.asarray(r.mean), mean.cpu().numpy(), rtol=1e-12)
         np.testing.assert_allclose(np.asarray(r.cov) / np.outer(sd, sd), cov / np.outer(sd, sd), atol=1e-10)
+
+
+@pytest.mark.parametrize("dim", [5, 6, 7, 8, 9, 10, 11, 12])
+@pytest.mark.parametrize("kind", ["narrow", "wide", "spread"])
+def test_long_mixture_same_bits(va, dim, kind):
+    """Components of weight 0 change nothing, so 255 of them (the plain loop)
+    and the same with 1 to 4 more of weight 0 (the long mixtures' loop, its
+    remainders) are one integrand: mean, variance, per-hcube sums, training
+    histogram and grid are the same bits, with terms left out or not."""
+    rng = np.random.default_rng(dim)
+    nc, neval = 255, 4200000
+    sigma = 0.4 if kind == "wide" else 0.02 * np.sqrt(dim)
+    A = rng.uniform(0.5, 1.5, nc) * (np.exp(rng.uniform(-40, 40, nc)) if kind == "spread" else 1.0)
+    B = 0.5 / (sigma * rng.uniform(0.7, 1.3, nc)) ** 2
+    c = rng.permutation(np.linspace(0.25, 0.75, nc))[:, None] + rng.uniform(-0.02, 0.02, (nc, dim))
+
+    def run(zeros):
+        # the zeros first, in the middle and last
+        at = np.sort(rng.integers(0, nc + 1, zeros)) if zeros else []
+        f = va.GaussianMixture(np.insert(A, at, 0.0), np.insert(B, at, 50.0), np.insert(c, at, 0.5, axis=0))
+        integ = va.Integrator([[0, 1]] * dim, neval=neval, seed=31, precision='f32')
+        r = integ(f, nitn=1).itn_results[0]
+        return r.mean, r.var, integ.sigf.copy(), integ.map.grid, integ._last_training()
+
+    plain = run(0)
+    for zeros in (1, 2, 3, 4):
+        many = run(zeros)
+        assert many[:2] == plain[:2]
+        for a, b in zip(many[2:4] + many[4], plain[2:4] + plain[4]):
+            assert np.array_equal(np.asarray(a), np.asarray(b))
+
+
+def test_long_mixture_few_points(va):
+    """A long mixture whose launch has few tiles after all (only 2 points in
+    each of 256 hcubes) runs the sampler of few tiles."""
+    rng = np.random.default_rng(3)
+    c = rng.uniform(0.3, 0.7, (256, 8))
+
+    def run(zeros):
+        f = va.GaussianMixture([1.0] * 256 + [0.0] * zeros, [30.0] * (256 + zeros), np.concatenate([c, c[:zeros]]))
+        integ = va.Integrator([[0, 1]] * 8, neval=4200000, nstrat=[2] * 8, seed=31, precision='f32', nitn=2)
+        integ.neval_frac, integ.min_neval_hcube = 0.0, 2
+        r = integ(f).itn_results[-1]
+        assert integ.last_neval == 512
+        return r.mean, r.var
+
+    assert run(0) == run(3)

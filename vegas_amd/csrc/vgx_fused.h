@@ -12,6 +12,8 @@
 // builds the histogram in a fixed order; the batched sampler, which calls the same tile
 // body, keeps an LDS-privatised histogram (FP64 sums, packed u16 counts) instead.
 #pragma once
+#include <type_traits>
+
 #include "vgx_iter.h"
 
 namespace vgx {
@@ -1297,26 +1299,26 @@ __global__ __launch_bounds__(sampler_threads(DIM, PER)) void split_kernel(IterGe
     block_close_tiles(acc, io.tile_part, tb, te, io.blk_part + 6 * (size_t)blockIdx.x, sc);
 }
 
+// One launch of either sampler; GaussMany32, which large launches take, has
+// fused_kernel only.
 template <int DIM, class Fcn>
 int launch_fused_dim(const IterGeom& g, const FusedPtrs& io, const Fcn& fcn, int blocks, size_t lds,
                      hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
-    auto kern = g.split ? split_kernel<DIM, false, Fcn> : fused_kernel<DIM, false, Fcn>;
-    if constexpr (Fcn::kRng32) {
-        if (g.per_all) kern = g.split ? split_kernel<DIM, true, Fcn> : fused_kernel<DIM, true, Fcn>;
-    }
-    // the LDS limit of this instantiation is raised once, to the largest
+    constexpr bool kSplit = !std::is_same_v<Fcn, GaussMany32>;
+    if (g.split && !kSplit) return VGX_EINVAL;
+    using Kernel = void (*)(IterGeom, FusedPtrs, Fcn);
+    Kernel kerns[4] = {fused_kernel<DIM, false, Fcn>};  // [2 split + PER]
+    if constexpr (Fcn::kRng32) kerns[1] = fused_kernel<DIM, true, Fcn>;
+    if constexpr (kSplit) kerns[2] = split_kernel<DIM, false, Fcn>;
+    if constexpr (kSplit && Fcn::kRng32) kerns[3] = split_kernel<DIM, true, Fcn>;
+    const Kernel kern = kerns[(g.split ? 2 : 0) + (Fcn::kRng32 && g.per_all ? 1 : 0)];
+    // the LDS limit of these instantiations is raised once, to the largest
     // request seen (a host-side attribute, not a per-launch cost)
     static size_t lds_set = 64 * 1024;
     if (lds > lds_set) {
-        auto raise = [&](const void* k) {
-            return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
-        };
-        if (!raise((const void*)fused_kernel<DIM, false, Fcn>) || !raise((const void*)split_kernel<DIM, false, Fcn>))
-            return VGX_EHIP;
-        if constexpr (Fcn::kRng32) {
-            if (!raise((const void*)fused_kernel<DIM, true, Fcn>) || !raise((const void*)split_kernel<DIM, true, Fcn>))
+        for (const Kernel k : kerns)
+            if (k && hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
                 return VGX_EHIP;
-        }
         lds_set = lds;
     }
     const int threads = sampler_threads(DIM, g.per_all && Fcn::kRng32);
