@@ -302,3 +302,27 @@ def test_long_mixture_few_points(va):
         return r.mean, r.var
 
     assert run(0) == run(3)
+
+
+@pytest.mark.parametrize("dim", [9, 10, 11, 12, 13])
+@pytest.mark.parametrize("nc", [1, 3, 4, 5, 15, 16, 17, 33])
+@pytest.mark.parametrize("kind", ["mixture", "ridge"])
+def test_component_steps_same_bits(va, dim, nc, kind):
+    """Components of weight 0 in any place change no bit, whatever step of the
+    components' loop (one, 4, 8 or 16 at a time) or its remainder they fall in."""
+    rng = np.random.default_rng(nc)
+    A, B = rng.uniform(0.5, 1.5, nc), rng.uniform(5.0, 20.0, nc)
+    t = np.linspace(0.3, 0.7, nc)
+
+    def run(at):
+        a, b, c = (np.insert(v, at, z) for v, z in ((A, 0.0), (B, 9.0), (t, 0.5)))
+        f = va.DiagonalRidge(a, b, c, dim) if kind == "ridge" else \
+            va.GaussianMixture(a, b, c[:, None] * np.linspace(0.8, 1.2, dim)[None, :])
+        integ = va.Integrator([[0, 1]] * dim, neval=20000, seed=31, precision='f32')
+        r = integ(f, nitn=2)
+        return [(g.mean, g.var) for g in r.itn_results], integ.map.grid
+
+    plain = run([])
+    for zeros in (1, 2, 3, 15):
+        more = run(np.sort(rng.integers(0, nc + 1, zeros)))
+        assert more[0] == plain[0] and np.array_equal(more[1], plain[1])

@@ -308,7 +308,7 @@ constexpr size_t kBLds = kBLdsGrid + kBLdsSums + kBLdsCnts + kBLdsOffs;
 // order at the item's close.
 template <int DIM, bool PER>
 __device__ __forceinline__ void b_item_tiles(const BArgs& a, const TileGeom& tg, const TileIO& tio,
-                                             const GaussMix32& fcn, const AxisC* ax, const double* G, double* Ls,
+                                             const GaussOne32& fcn, const AxisC* ax, const double* G, double* Ls,
                                              uint32_t* Lc, uint32_t* offs, uint32_t t0, uint32_t ntl, uint32_t hend,
                                              uint32_t off_end, uint32_t hbase, uint32_t pshift, uint32_t* s_tile,
                                              int lane, TileAcc& acc) {
@@ -389,7 +389,7 @@ __global__ __launch_bounds__(kFusedThreads) void b_fused_kernel(BArgs a, int it,
         for (int k = threadIdx.x; k < tot; k += blockDim.x) Ls[k] = 0.0;
         for (int k = threadIdx.x; k < (tot + 1) / 2; k += blockDim.x) Lc[k] = 0u;
         __syncthreads();
-        const GaussMix32 fcn{1, a.fA + i, a.fB + i, a.fc + (size_t)i * kBD};
+        const GaussOne32 fcn{1, a.fA + i, a.fB + i, a.fc + (size_t)i * kBD};
         const TileIO tio{a.off, a.sigf, a.slots, nullptr, nullptr, nullptr, 0u, 0u};  // LDS histogram
         TileAcc acc{{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, 0};
         const uint32_t hend = q.hbase + (uint32_t)q.nhcube, off_end = pl.P + pl.T;

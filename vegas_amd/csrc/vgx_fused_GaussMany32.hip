@@ -13,9 +13,6 @@ int launch_fused<GaussMany32>(const IterGeom& g, const FusedPtrs& io, const Gaus
         case 7: return launch_fused_dim<7>(g, io, fcn, blocks, lds, st, ev0, ev1);
         case 8: return launch_fused_dim<8>(g, io, fcn, blocks, lds, st, ev0, ev1);
         case 9: return launch_fused_dim<9>(g, io, fcn, blocks, lds, st, ev0, ev1);
-        case 10: return launch_fused_dim<10>(g, io, fcn, blocks, lds, st, ev0, ev1);
-        case 11: return launch_fused_dim<11>(g, io, fcn, blocks, lds, st, ev0, ev1);
-        case 12: return launch_fused_dim<12>(g, io, fcn, blocks, lds, st, ev0, ev1);
         default: return VGX_EINVAL;
     }
 }

@@ -155,7 +155,14 @@ __device__ __forceinline__ double scaled_exp2(float A, float y) {
     return ldexp((double)(A * __builtin_amdgcn_exp2f(y - fl)), (int)fl);
 }
 
-struct GaussMix32 {
+// STEPS: four components at a time, their constants loaded first (one wait
+// for scalar loads instead of one per component), where the sampler has 12
+// waves, 10 to 12 axes: with 16 the others cover those waits, and a short
+// mixture pays for the registers (8 axes, two components: 1-2 % of its launch).
+// 1e7 points, 250 components of 10 axes, two iterations: 4155 us one by one
+// (3523 with 16 waves, which spilled), 3297 so; two or three at a time 3469, 3409.
+template <bool STEPS>
+struct GaussMix32T {
     static constexpr bool kRng32 = true;
     int ncomp;
     const float* A;
@@ -170,9 +177,34 @@ struct GaussMix32 {
             if (DIM <= 0 && d >= nd) break;
             xf[d] = (float)x[d];
         }
-        // the components' values, each with the FP64 exponent range, summed in FP64
+        // the components' values, each with the FP64 exponent range, summed in
+        // FP64 in component order
         double acc = 0.0;
-        for (int k = 0; k < ncomp; ++k) {
+        int k = 0;
+        if constexpr (STEPS && DIM >= 10 && DIM <= 12) {
+            constexpr int kStep = 4;
+            for (; k + kStep <= ncomp; k += kStep) {
+                float cc[kStep][DIM], aa[kStep], bb[kStep];
+#pragma unroll
+                for (int i = 0; i < kStep; ++i) {
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) cc[i][d] = ldc(c, (k + i) * DIM + d);
+                    aa[i] = ldc(A, k + i);
+                    bb[i] = ldc(B, k + i);
+                }
+#pragma unroll
+                for (int i = 0; i < kStep; ++i) {
+                    float r2 = 0.0f;
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) {
+                        const float t = xf[d] - cc[i][d];
+                        r2 = __builtin_fmaf(t, t, r2);
+                    }
+                    acc += scaled_exp2(aa[i], (-bb[i] * r2) * 1.44269504088896341f);
+                }
+            }
+        }
+        for (; k < ncomp; ++k) {
             float r2 = 0.0f;
 #pragma unroll
             for (int d = 0; d < nd_max(DIM); ++d) {
@@ -185,6 +217,8 @@ struct GaussMix32 {
         return acc;
     }
 };
+using GaussMix32 = GaussMix32T<true>;
+using GaussOne32 = GaussMix32T<false>;  // the batched sampler's (16 waves for every dimension)
 
 // GaussMix32 for long mixtures (many_pays below): the same operations in the
 // same order, so the same bits, but two components at a time, and a pair whose
@@ -260,13 +294,15 @@ struct GaussMany32 {
 };
 
 // Where GaussMany32 takes GaussMix32's place (one pair against the other, 256
-// to 1000 components, FP32 samples): with 5 to 12 axes and 4.2e6 or 8e6 points
-// it is 0.98-1.24 times as fast where every term counts (sigma 0.2) and
-// 1.18-1.52 where few do (0.005).  With 4 axes wide mixtures lose 2-5 %, with 1.2e6
+// to 1000 components, FP32 samples): with 5 to 9 axes and 4.2e6 or 8e6 points
+// it is 1.00-1.11 times as fast where every term counts (sigma 0.2) and
+// 1.05-1.18 where few do (0.02).  With 10 to 12 axes GaussMix32 takes four at a
+// time itself, and is faster; with 4 axes wide mixtures lose 2-5 %, with 1.2e6
 // points (few tiles to a wave) up to 11 %; a short mixture loses its whole
 // kernel 1-2 % (two components, 8 axes, 9.8e6 points: 259 -> 261-265 us).
+// Above 12 axes it was not measured.
 inline bool many_pays(int ncomp, int dim, int64_t neval) {
-    return ncomp >= 256 && dim >= 5 && dim <= 12 && neval >= (1 << 22);
+    return ncomp >= 256 && dim >= 5 && dim <= 9 && neval >= (1 << 22);
 }
 
 // Mixture with centres t_k (1,...,1): |x - c_k|^2 = P + dim (xbar - t_k)^2,
@@ -300,8 +336,10 @@ struct DiagRidge32 {
         float acc = 0.0f;
         // eight components per step with their constants loaded first (wide
         // scalar loads, one wait instead of two per component); the sum runs
-        // in component order as in the remainder loop
-        constexpr int kStep = 8;
+        // in component order as in the remainder loop.  Sixteen where the
+        // sampler has 12 waves (4e6 points, 1000 components of 11 axes: 1900
+        // us with eight, 1684; with 16 waves, which spilled, 1716).
+        constexpr int kStep = DIM >= 10 && DIM <= 12 ? 16 : 8;
         int k = 0;
         for (; k + kStep <= ncomp; k += kStep) {
             float cc[kStep], aa[kStep], bb[kStep];
