@@ -12,8 +12,6 @@
 // builds the histogram in a fixed order; the batched sampler, which calls the same tile
 // body, keeps an LDS-privatised histogram (FP64 sums, packed u16 counts) instead.
 #pragma once
-#include <type_traits>
-
 #include "vgx_iter.h"
 
 namespace vgx {
@@ -407,6 +405,21 @@ __device__ __forceinline__ void store_offsets(uint32_t* offs, int lane, const ui
         if (lane + kWave * q < kNoff) offs[lane + kWave * q] = v[q];
 }
 
+// Threads of a sampler workgroup (one per CU): 16 waves as long as the kernel
+// fits their 128 registers, else 12 (168) or 8 (256).  No sampler may spill
+// vector registers: besides the time, this compiler places some of the spill
+// stores before the exec mask is restored at the end of a branch, and the
+// lanes that skipped the branch then lose the value (the 9-axis FP64 sampler's
+// sums came out wrong so).  The build fails where a kernel spills them, the
+// batched sampler among them (the Makefile's kernel-resource-usage).  us per launch of 1e6 points, 1024 threads with
+// spills / without: 9 axes f64 49 / 41, 13 axes 91 / 61.
+constexpr int sampler_threads(int dim, bool per) {
+    if (dim > 16) dim = 0;
+    if (dim <= 0) return per ? 768 : kFusedThreads;  // (runtime dimension: its arrays are in scratch)
+    if (dim <= (per ? 9 : 6)) return kFusedThreads;
+    return dim <= (per ? 14 : 10) ? 768 : 512;
+}
+
 // One point: hcube h (integral-local) of ncur points, weight factor wdiv =
 // dv_y / ncur, point index pj.  Samples, maps, evaluates, and stores or adds
 // the training data.  Returns w f.
@@ -425,7 +438,8 @@ __device__ __forceinline__ double tile_point(const TileGeom& g, const TileIO& io
     uint32_t zmin = 0xFFFFFFFFu;
     eval_point<DIM, R32, PER>(g, ax, G, pc, h, pj - tp.pshift, x, J, kb, zmin, perv);
     const double w = J * wdiv;
-    const double f = fcn.template eval<DIM>(x, dim, pj);
+    constexpr bool kFew = DIM > 0 && sampler_threads(DIM, PER) < kFusedThreads;
+    const double f = fcn.template eval<DIM, kFew>(x, dim, pj);
     if (f != f) acc.nan_seen = 1;
     const double vj = w * f;
     const double tn = vj * (double)ncur;
@@ -947,21 +961,6 @@ __device__ inline void block_close_tiles(const TileAcc& acc, const double* tpart
             out[0] = m.hi; out[1] = m.lo; out[2] = v.hi; out[3] = v.lo; out[4] = q.hi; out[5] = q.lo;
         }
     }
-}
-
-// Threads of a sampler workgroup (one per CU): 16 waves as long as the kernel
-// fits their 128 registers, else 12 (168) or 8 (256).  No sampler may spill
-// vector registers: besides the time, this compiler places some of the spill
-// stores before the exec mask is restored at the end of a branch, and the
-// lanes that skipped the branch then lose the value (the 9-axis FP64 sampler's
-// sums came out wrong so).  The build fails where a kernel spills them, the
-// batched sampler among them (the Makefile's kernel-resource-usage).  us per launch of 1e6 points, 1024 threads with
-// spills / without: 9 axes f64 49 / 41, 13 axes 91 / 61.
-constexpr int sampler_threads(int dim, bool per) {
-    if (dim > 16) dim = 0;
-    if (dim <= 0) return per ? 768 : kFusedThreads;  // (runtime dimension: its arrays are in scratch)
-    if (dim <= (per ? 9 : 6)) return kFusedThreads;
-    return dim <= (per ? 14 : 10) ? 768 : 512;
 }
 
 template <int DIM, bool PER, class Fcn>

@@ -1,5 +1,7 @@
 // vgx_iter.h -- shared definitions of the vegas+ iteration kernels.
 #pragma once
+#include <type_traits>
+
 #include "vgx_internal.h"
 
 namespace vgx {
@@ -125,7 +127,7 @@ struct GaussMix64 {
     const double* A;
     const double* B;
     const double* c;
-    template <int DIM>
+    template <int DIM, bool FEW>
     __device__ double eval(const double* x, int dim, uint32_t) const {
         const int nd = DIM > 0 ? DIM : dim;
         double acc = 0.0;
@@ -155,12 +157,14 @@ __device__ __forceinline__ double scaled_exp2(float A, float y) {
     return ldexp((double)(A * __builtin_amdgcn_exp2f(y - fl)), (int)fl);
 }
 
-// STEPS: four components at a time, their constants loaded first (one wait
-// for scalar loads instead of one per component), where the sampler has 12
-// waves, 10 to 12 axes: with 16 the others cover those waits, and a short
-// mixture pays for the registers (8 axes, two components: 1-2 % of its launch).
+// An integrand's eval: FEW where the sampler has fewer than 16 waves.
+// STEPS: four components at a time there, their constants loaded first (one
+// wait for scalar loads instead of one per component): 16 waves cover those
+// waits, and a short mixture pays for the registers (8 axes, two components:
+// 1-2 % of its launch).
 // 1e7 points, 250 components of 10 axes, two iterations: 4155 us one by one
-// (3523 with 16 waves, which spilled), 3297 so; two or three at a time 3469, 3409.
+// (3523 with 16 waves, which spilled), 3297 so; two or three at a time 3469,
+// 3409.  (FP64 two at a time: short mixtures of 12 and 13 axes lose 10 %.)
 template <bool STEPS>
 struct GaussMix32T {
     static constexpr bool kRng32 = true;
@@ -168,7 +172,7 @@ struct GaussMix32T {
     const float* A;
     const float* B;
     const float* c;
-    template <int DIM>
+    template <int DIM, bool FEW>
     __device__ double eval(const double* x, int dim, uint32_t) const {
         const int nd = DIM > 0 ? DIM : dim;
         float xf[nd_max(DIM)];
@@ -181,7 +185,7 @@ struct GaussMix32T {
         // FP64 in component order
         double acc = 0.0;
         int k = 0;
-        if constexpr (STEPS && DIM >= 10 && DIM <= 12) {
+        if constexpr (STEPS && FEW) {
             constexpr int kStep = 4;
             for (; k + kStep <= ncomp; k += kStep) {
                 float cc[kStep][DIM], aa[kStep], bb[kStep];
@@ -235,7 +239,7 @@ struct GaussMany32 {
     const float* B;
     const float* c;
     const float* ea;  // [1]: an integer, every A[k] < 2^ea (max_exponent_kernel)
-    template <int DIM>
+    template <int DIM, bool FEW>
     __device__ double eval(const double* x, int dim, uint32_t) const {
         const int nd = DIM > 0 ? DIM : dim;
         float xf[nd_max(DIM)];
@@ -313,7 +317,7 @@ struct DiagRidge32 {
     const float* A;
     const float* B;
     const float* c;  // t_k
-    template <int DIM>
+    template <int DIM, bool FEW>
     __device__ double eval(const double* x, int dim, uint32_t) const {
         const int nd = DIM > 0 ? DIM : dim;
         float xf[nd_max(DIM)];
@@ -336,12 +340,13 @@ struct DiagRidge32 {
         float acc = 0.0f;
         // eight components per step with their constants loaded first (wide
         // scalar loads, one wait instead of two per component); the sum runs
-        // in component order as in the remainder loop.  Sixteen where the
-        // sampler has 12 waves (4e6 points, 1000 components of 11 axes: 1900
-        // us with eight, 1684; with 16 waves, which spilled, 1716).
-        constexpr int kStep = DIM >= 10 && DIM <= 12 ? 16 : 8;
+        // in component order as in the remainder loop.  Sixteen, then eight, on
+        // 10 to 12 axes, where the sampler has 12 waves (4e6 points, 1000
+        // components of 11 axes: 1900 us with eight, 1684; with 16 waves, which
+        // spilled, 1716).
         int k = 0;
-        for (; k + kStep <= ncomp; k += kStep) {
+        auto step = [&](auto n) {
+            constexpr int kStep = decltype(n)::value;
             float cc[kStep], aa[kStep], bb[kStep];
 #pragma unroll
             for (int i = 0; i < kStep; ++i) {
@@ -355,7 +360,11 @@ struct DiagRidge32 {
                 float r2 = __builtin_fmaf(fd * t, t, P);
                 acc = __builtin_fmaf(aa[i], __expf(-bb[i] * r2), acc);
             }
-        }
+            k += kStep;
+        };
+        if constexpr (DIM >= 10 && DIM <= 12)
+            while (k + 16 <= ncomp) step(std::integral_constant<int, 16>{});
+        while (k + 8 <= ncomp) step(std::integral_constant<int, 8>{});
         for (; k < ncomp; ++k) {
             float t = xbar - ldc(c, k);
             float r2 = __builtin_fmaf(fd * t, t, P);
@@ -371,7 +380,7 @@ struct DiagRidge64 {
     const double* A;
     const double* B;
     const double* c;
-    template <int DIM>
+    template <int DIM, bool FEW>
     __device__ double eval(const double* x, int dim, uint32_t) const {
         const int nd = DIM > 0 ? DIM : dim;
         double s = 0.0;
@@ -403,7 +412,7 @@ struct BufferFcn {
     static constexpr bool kRng32 = R32;
     const double* f;
     int64_t base;
-    template <int DIM>
+    template <int DIM, bool FEW>
     __device__ double eval(const double*, int, uint32_t p) const {
         return f[(int64_t)p - base];
     }
