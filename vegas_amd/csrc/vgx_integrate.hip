@@ -1402,7 +1402,7 @@ static int make_fcn_and_run(vgx_ctx* ctx, Run* R, const vgx_config* c, const vgx
             float* A = R->fparams;
             float* B = A + nc;
             float* C = B + nc;
-            if (f->kind == VGX_FCN_GAUSSMIX && many_pays(nc, c->dim, c->neval) && !R->g.split) {
+            if (f->kind == VGX_FCN_GAUSSMIX && many_pays(nc, c->dim, c->neval, R->g.per_all) && !R->g.split) {
                 if (first) hipLaunchKernelGGL(max_exponent_kernel, dim3(1), dim3(1024), 0, s, f->A, nc, R->fmax);
                 GaussMany32 fn{nc, A, B, C, R->fmax};
                 return accumulate_kernels(ctx, R, fn, s, timed, reduce);

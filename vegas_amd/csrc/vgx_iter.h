@@ -164,7 +164,8 @@ __device__ __forceinline__ double scaled_exp2(float A, float y) {
 // 1-2 % of its launch).
 // 1e7 points, 250 components of 10 axes, two iterations: 4155 us one by one
 // (3523 with 16 waves, which spilled), 3297 so; two or three at a time 3469,
-// 3409.  (FP64 two at a time: short mixtures of 12 and 13 axes lose 10 %.)
+// 3409.  (FP64 two at a time: short mixtures of 12 and 13 axes lose 10 %.  7
+// axes with 12 waves: short ones lose 10-15 %, 8 axes 0-3 %, more axes none.)
 template <bool STEPS>
 struct GaussMix32T {
     static constexpr bool kRng32 = true;
@@ -185,7 +186,7 @@ struct GaussMix32T {
         // FP64 in component order
         double acc = 0.0;
         int k = 0;
-        if constexpr (STEPS && FEW) {
+        if constexpr (STEPS && FEW && DIM >= 8) {
             constexpr int kStep = 4;
             for (; k + kStep <= ncomp; k += kStep) {
                 float cc[kStep][DIM], aa[kStep], bb[kStep];
@@ -300,13 +301,13 @@ struct GaussMany32 {
 // Where GaussMany32 takes GaussMix32's place (one pair against the other, 256
 // to 1000 components, FP32 samples): with 5 to 9 axes and 4.2e6 or 8e6 points
 // it is 1.00-1.11 times as fast where every term counts (sigma 0.2) and
-// 1.05-1.18 where few do (0.02).  With 10 to 12 axes GaussMix32 takes four at a
-// time itself, and is faster; with 4 axes wide mixtures lose 2-5 %, with 1.2e6
-// points (few tiles to a wave) up to 11 %; a short mixture loses its whole
-// kernel 1-2 % (two components, 8 axes, 9.8e6 points: 259 -> 261-265 us).
-// Above 12 axes it was not measured.
-inline bool many_pays(int ncomp, int dim, int64_t neval) {
-    return ncomp >= 256 && dim >= 5 && dim <= 9 && neval >= (1 << 22);
+// 1.05-1.18 where few do (0.02).  Where GaussMix32 takes four at a time itself
+// (few waves: from 10 axes on, from 8 off the integer strata) that is faster.
+// With 4 axes wide mixtures lose 2-5 %, with 1.2e6 points (few tiles to a wave)
+// up to 11 %; a short mixture loses its whole kernel 1-2 % (two components, 8
+// axes, 9.8e6 points: 259 -> 261-265 us).
+inline bool many_pays(int ncomp, int dim, int64_t neval, bool per) {
+    return ncomp >= 256 && dim >= 5 && dim <= (per ? 9 : 7) && neval >= (1 << 22);
 }
 
 // Mixture with centres t_k (1,...,1): |x - c_k|^2 = P + dim (xbar - t_k)^2,
