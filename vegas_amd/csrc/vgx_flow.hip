@@ -91,7 +91,7 @@ __device__ inline f32x4_t mfma16(bf16x4_t a, bf16x4_t b, f32x4_t c) {
 // k to those 8 slots that A and B share gives the same sum.  Here slots
 // 0..3 are k-step kt's k = 4g..4g+3 and slots 4..7 k-step kt+1's: the B
 // operand is two C-layout tiles side by side (no data movement), the A
-// operand two 8-byte pieces of a weight row.
+// operand one 16-byte read of weights in fragment order.
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 __device__ inline bf16x8_t cat8(bf16x4_t lo, bf16x4_t hi) {
     typedef short s16x8_t __attribute__((ext_vector_type(8)));
@@ -428,8 +428,8 @@ __device__ __noinline__ double exp_jac(double x) { return exp(x); }
 // axes, 6 layers, 500 components: 2450 us with row-major weights and a tile
 // at a time, 2480 -> 2175 with one-instruction relu and four ridge terms a
 // step, 1940 with the products' priority and the couplings' short quotient,
-// 1570 a call with the parameters read in place (before: three copies to the
-// host and one back, each waited for).  12 waves hold all of a layer in
+// 1570 a call, calls back to back, with the parameters read in place (before:
+// three copies to the host and one back, each waited for).  12 waves hold all of a layer in
 // registers; with 16 the kernels spill 35 and are no faster, with 8 and four
 // tiles at once 2012 where 12 took 1945.
 __global__ __launch_bounds__(kFlowThreads) void flow_sample_kernel(FlowArgs f, FlowFcn F, SampleArgs a) {
