@@ -409,3 +409,29 @@ def test_long_integrands_in_large_calls(torch, nc):
         assert torch.equal(xs, x[base:base + 1000]) and torch.equal(fs, fj[base:base + 1000])
     np.testing.assert_allclose(s1, fj.double().sum().item(), rtol=6e-8, equal_nan=False)
     np.testing.assert_allclose(s2, (fj.double() ** 2).sum().item(), rtol=1.2e-7, equal_nan=False)
+
+
+def test_eval_from_threads(torch):
+    """Threads with streams of their own evaluate different integrands through
+    one flow: each gets its own integrand's values."""
+    import threading
+    import vegas_amd as va
+    from vegas_amd.flow import CouplingFlow
+    flow, x = CouplingFlow(5, 2, seed=3), torch.rand((20000, 16), dtype=torch.float32, device='cuda')
+    fs = [va.DiagonalRidge([1.0 + k] * 100, [5.0] * 100, np.linspace(0.3, 0.7, 100), 5) for k in range(4)]
+    want = [flow.eval_fcn(f, x).clone() for f in fs]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(k):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(100):
+                if not torch.equal(flow.eval_fcn(fs[k], x), want[k]):
+                    wrong.append(k)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong

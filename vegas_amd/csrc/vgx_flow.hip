@@ -30,6 +30,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <mutex>
 #include <vector>
 
 #include "vgx_internal.h"
@@ -1163,6 +1164,7 @@ struct vgx_flow {
     Scratch saved, u0, logq, c, G, wpart, cpart, spart, misc;
     hipEvent_t held = nullptr;  // an integrand's parameters have been copied
     hipEvent_t used = nullptr;  // and the copy read
+    std::mutex hold_mu;         // from the one's record to the other's
     int step = 0;
 };
 
@@ -1290,7 +1292,8 @@ static int flow_fcn_params(const vgx_flow* fl, const vgx_integrand* fcn, FlowFcn
 // taken, so that the caller may reuse or free them.  (The kernel is then
 // already in the queue: waiting for the copy before the launch would leave
 // the GPU idle for the launch.)  A second stream's copy waits for the first's
-// reader.
+// reader; lk (of hold_mu) is held from one to the other, so that a second
+// thread's call sees that reader.
 static int flow_hold_params(vgx_flow* fl, FlowFcn* F, size_t lds, hipStream_t s) {
     const int na = F->ncomp, nc = (int)(lds / 4) - 2 * na;
     DeviceInfo info;
@@ -1306,8 +1309,9 @@ static int flow_hold_params(vgx_flow* fl, FlowFcn* F, size_t lds, hipStream_t s)
     F->c = d + 2 * na;
     return VGX_OK;
 }
-static int flow_params_held(vgx_flow* fl, hipStream_t s) {
+static int flow_params_held(vgx_flow* fl, hipStream_t s, std::unique_lock<std::mutex>& lk) {
     VGX_HIP(hipEventRecord(fl->used, s));
+    lk.unlock();
     VGX_HIP(hipEventSynchronize(fl->held));
     return VGX_OK;
 }
@@ -1321,6 +1325,8 @@ extern "C" int vgx_flow_sample(vgx_flow* fl, const vgx_integrand* fcn, int64_t n
     size_t fcn_lds;
     int rc = flow_fcn_params(fl, fcn, &F, &fcn_lds);
     if (rc) return rc;
+    std::unique_lock<std::mutex> lk(fl->hold_mu, std::defer_lock);
+    if (!sums) lk.lock();
     if (!sums && (rc = flow_hold_params(fl, &F, fcn_lds, s))) return rc;
     DeviceInfo info;
     if ((rc = device_info(&info))) return rc;
@@ -1349,7 +1355,7 @@ extern "C" int vgx_flow_sample(vgx_flow* fl, const vgx_integrand* fcn, int64_t n
     else
         hipLaunchKernelGGL(flow_sample_kernel, dim3(blocks), dim3(64 * sh.waves), lds, s, flow_args(fl), F, a);
     if ((rc = check_launch())) return rc;
-    if (!sums) return flow_params_held(fl, s);
+    if (!sums) return flow_params_held(fl, s, lk);
     std::vector<double> h((size_t)blocks * 4);
     VGX_HIP(hipMemcpyAsync(h.data(), a.part, h.size() * 8, hipMemcpyDeviceToHost, s));
     VGX_HIP(hipStreamSynchronize(s));
@@ -1483,10 +1489,11 @@ extern "C" int vgx_flow_eval(vgx_flow* fl, const vgx_integrand* fcn, const float
     if (hipFuncSetAttribute((const void*)flow_eval_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)(fcn_lds + 16)) != hipSuccess)
         return VGX_EHIP;
+    std::unique_lock<std::mutex> lk(fl->hold_mu);
     if ((rc = flow_hold_params(fl, &F, fcn_lds, s))) return rc;
     hipLaunchKernelGGL(flow_eval_kernel, dim3(blocks), dim3(256), fcn_lds + 16, s, F, fl->D, x, (uint64_t)n, f);
     if ((rc = check_launch())) return rc;
-    return flow_params_held(fl, s);
+    return flow_params_held(fl, s, lk);
 }
 
 extern "C" int vgx_flow_mfma_probe(const uint16_t* A, const uint16_t* B, float* D, void* stream) {
