@@ -326,8 +326,8 @@ int vgx_flow_get_params(const vgx_flow* fl, float* host, float* grad_host, void*
  * the stream).  sums may be NULL when xout and fout are given: nothing is
  * read back and the call returns without waiting for its kernel.  fcn:
  * GAUSSMIX or DIAGRIDGE with device FP64 parameters (evaluated in FP32; read
- * before the call returns).  xout, fout
- * (device, optional): the points and f J.  status: device int32, set to
+ * before the call returns, or, captured into a graph, when that runs).  xout,
+ * fout (device, optional): the points and f J.  status: device int32, set to
  * VGX_ENAN when f is NaN.                                                 */
 int vgx_flow_sample(vgx_flow* fl, const vgx_integrand* fcn, int64_t n, uint64_t base, uint64_t seed,
                     uint32_t iteration, double* sums, float* xout, float* fout, int32_t* status,
@@ -356,7 +356,7 @@ int vgx_flow_grad(vgx_flow* fl, const float* x, const float* f, const float* log
 /* One Adam step with the last gradient; bf16 copies refreshed.            */
 int vgx_flow_adam(vgx_flow* fl, float lr, float beta1, float beta2, float eps, float clip, void* stream);
 /* f at points x (device float[n][16]) into f (device float[n]); fcn's
- * parameters are read before the call returns.                            */
+ * parameters are read as by vgx_flow_sample.                              */
 int vgx_flow_eval(vgx_flow* fl, const vgx_integrand* fcn, const float* x, int64_t n, float* f,
                   void* stream);
 /* D = A B for 16x16 bf16 A, B (device, row-major) on one MFMA: checks the

@@ -435,3 +435,32 @@ def test_eval_from_threads(torch):
     for t in threads:
         t.join()
     assert not wrong
+
+
+def test_lazy_calls_in_a_graph(torch):
+    """A lazy sample and an evaluation captured into a graph give the eager
+    values at every replay, with eager calls and synchronisations between."""
+    import vegas_amd as va
+    from vegas_amd.flow import CouplingFlow
+    flow, n = CouplingFlow(5, 2, seed=3), 20000
+    f = va.DiagonalRidge([1.0] * 7, [20.0] * 7, np.linspace(0.3, 0.7, 7), 5)
+    other = va.DiagonalRidge([0.5], [2.0], [0.5], 5)
+    status = torch.zeros(1, dtype=torch.int32, device='cuda')
+
+    def go():
+        _, _, x, fj = flow.sample(f, n, seed=5, keep_points=True, status=status)
+        return x, fj, flow.eval_fcn(f, x)
+
+    want = [t.clone() for t in go()]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = go()
+    for _ in range(4):
+        for t in out:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(out, want))
+        flow.eval_fcn(other, out[0])
+        torch.cuda.synchronize()

@@ -1316,6 +1316,15 @@ static int flow_params_held(vgx_flow* fl, hipStream_t s, std::unique_lock<std::m
     return VGX_OK;
 }
 
+// Whether a call on s returns before its kernel has run.  (Not so a captured
+// one, whose kernel runs when the graph does and reads the arrays then.)
+static int flow_holds(hipStream_t s, bool* hold) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    VGX_HIP(hipStreamIsCapturing(s, &st));
+    *hold = st == hipStreamCaptureStatusNone;
+    return VGX_OK;
+}
+
 extern "C" int vgx_flow_sample(vgx_flow* fl, const vgx_integrand* fcn, int64_t n, uint64_t base, uint64_t seed,
                                uint32_t iteration, double* sums, float* xout, float* fout, int32_t* status,
                                void* stream) {
@@ -1325,9 +1334,11 @@ extern "C" int vgx_flow_sample(vgx_flow* fl, const vgx_integrand* fcn, int64_t n
     size_t fcn_lds;
     int rc = flow_fcn_params(fl, fcn, &F, &fcn_lds);
     if (rc) return rc;
+    bool hold = false;
+    if (!sums && (rc = flow_holds(s, &hold))) return rc;
     std::unique_lock<std::mutex> lk(fl->hold_mu, std::defer_lock);
-    if (!sums) lk.lock();
-    if (!sums && (rc = flow_hold_params(fl, &F, fcn_lds, s))) return rc;
+    if (hold) lk.lock();
+    if (hold && (rc = flow_hold_params(fl, &F, fcn_lds, s))) return rc;
     DeviceInfo info;
     if ((rc = device_info(&info))) return rc;
     const FlowShape sh = flow_shape(n, info.cus, info.cus, fcn_lds);
@@ -1355,7 +1366,7 @@ extern "C" int vgx_flow_sample(vgx_flow* fl, const vgx_integrand* fcn, int64_t n
     else
         hipLaunchKernelGGL(flow_sample_kernel, dim3(blocks), dim3(64 * sh.waves), lds, s, flow_args(fl), F, a);
     if ((rc = check_launch())) return rc;
-    if (!sums) return flow_params_held(fl, s, lk);
+    if (!sums) return hold ? flow_params_held(fl, s, lk) : VGX_OK;
     std::vector<double> h((size_t)blocks * 4);
     VGX_HIP(hipMemcpyAsync(h.data(), a.part, h.size() * 8, hipMemcpyDeviceToHost, s));
     VGX_HIP(hipStreamSynchronize(s));
@@ -1489,11 +1500,14 @@ extern "C" int vgx_flow_eval(vgx_flow* fl, const vgx_integrand* fcn, const float
     if (hipFuncSetAttribute((const void*)flow_eval_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)(fcn_lds + 16)) != hipSuccess)
         return VGX_EHIP;
-    std::unique_lock<std::mutex> lk(fl->hold_mu);
-    if ((rc = flow_hold_params(fl, &F, fcn_lds, s))) return rc;
+    bool hold = false;
+    if ((rc = flow_holds(s, &hold))) return rc;
+    std::unique_lock<std::mutex> lk(fl->hold_mu, std::defer_lock);
+    if (hold) lk.lock();
+    if (hold && (rc = flow_hold_params(fl, &F, fcn_lds, s))) return rc;
     hipLaunchKernelGGL(flow_eval_kernel, dim3(blocks), dim3(256), fcn_lds + 16, s, F, fl->D, x, (uint64_t)n, f);
     if ((rc = check_launch())) return rc;
-    return flow_params_held(fl, s, lk);
+    return hold ? flow_params_held(fl, s, lk) : VGX_OK;
 }
 
 extern "C" int vgx_flow_mfma_probe(const uint16_t* A, const uint16_t* B, float* D, void* stream) {
